@@ -88,8 +88,8 @@ int qcuCopyComplexVector(void *dst, int dst_precision, const void *src, int src_
 
 /* Launch shape of the dslash for every later call in this process (the
  * stateless qcuDslashMrhs and the solver alike): variant 0 = automatic
- * (tuning table, else MFMA for FP16/BF16 and wave-per-site VALU otherwise),
- * 1 = lane per (site, rhs), 2 = wavefront per site (VALU), 3 = wavefront per
+ * (tuning table, else by precision, Nc and m_rhs: lane per (site, rhs) or
+ * matrix cores), 1 = lane per (site, rhs), 2 = wavefront per site (VALU), 3 = wavefront per
  * site on MFMA (FP16/BF16 only), 4 = MFMA with the input rows staged in LDS
  * (FP16/BF16, Nc <= 4; spw = t steps per workgroup, 0 = 12; other shapes fall
  * back to variant 3 or 2); by, bz = traversal tile in y and z and spw =

@@ -12,7 +12,7 @@ namespace qcu {
 // Kernel variants of the one-parity hopping term.
 enum DslashVariant : int {
     kDslashAuto = 0,      // choose per precision (and from the tuning table)
-    kDslashLaneRhs = 1,   // one lane per (site, rhs), all 8 hops per lane
+    kDslashLaneRhs = 1,   // one lane per (site, rhs), all 8 hops per lane; tiled traversal for Nc <= 4
     kDslashWaveSite = 2,  // one wavefront per site: lanes = 16 rhs x 4 dimensions (VALU)
     kDslashMfma = 3,      // one wavefront per site on MFMA (FP16 / BF16 storage)
     kDslashLds = 4        // MFMA with the input rows staged in LDS: one workgroup per 4-site segment of an
@@ -61,6 +61,10 @@ void dslash_set_override(const DslashTune &t);
 hipError_t launch_dslash_wave(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 hipError_t launch_dslash_mfma(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_mfma_supported(int Nc, int prec);
+// lane-per-(site, RHS) kernels (dslash_lane.hip); by / bz that are 0 or do not divide the lattice are chosen
+hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
+bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
+void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
 hipError_t launch_dslash_lds(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_lds_supported(const Geom &g, int Nc, int prec);
 // FP32 / FP64 storage on the FP32 / FP64 matrix cores (dslash_mfma32.hip), also for batched groups

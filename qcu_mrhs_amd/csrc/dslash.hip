@@ -7,11 +7,12 @@
 // two projected rows per hop: h_r = psi_r + s_r psi_m(r), out_r += U h_r,
 // out_m(r) += c_r U h_r (include/kernel/qcu_gamma.cuh:47-324).
 //
-// This file holds the dispatcher and the lane-per-(site, rhs) VALU kernel
-// (variant kDslashLaneRhs): R lanes of one site read R consecutive complex
-// numbers for every (spin, colour); the link is a broadcast load shared by
-// those lanes.  The wave-per-site kernels live in dslash_wave.hip (VALU) and
-// dslash_mfma.hip (matrix cores).  Every variant has an optional epilogue
+// This file holds the dispatcher and the general lane-per-(site, rhs) VALU
+// kernel: R lanes of one site read R consecutive complex numbers for every
+// (spin, colour); the link is a broadcast load shared by those lanes.  It
+// serves variant kDslashLaneRhs for Nc = 8 and for vectors of 4 GiB and more;
+// the one for Nc <= 4 is in dslash_lane.hip.  The wave-per-site kernels live in
+// dslash_wave.hip (VALU) and dslash_mfma.hip (matrix cores).  Every variant has an optional epilogue
 // out = x + coef * D psi (Schur operator, full-lattice M, source preparation).
 #include <algorithm>
 #include <array>
@@ -230,8 +231,35 @@ std::vector<std::pair<std::array<int, 7>, DslashTune>> dslash_tuned_entries() {
     return v;
 }
 
+namespace {
+// Kernel chosen for a hop that names none.
+int automatic_variant(const DslashArgs &a) {
+    const bool lane = dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
+    if (a.prec == kSingle || a.prec == kDouble) {
+        // Nc = 8 fills the 16 x 16 matrix-core tile (16^4, 16 RHS: FP64 265 us against 1035 us wave per
+        // site, FP32 147 against 311 us); Nc <= 4 runs a lane per (site, RHS), faster than the
+        // wave-per-site and matrix-core kernels at every size timed (dslash_lane.hip)
+        if (a.Nc == 8) return kDslashMfma;
+        return lane ? kDslashLaneRhs : kDslashWaveSite;
+    }
+    // 16 bits: a lane per (site, RHS) where a row of right-hand sides is a whole number of 16-byte
+    // pieces (24^3 x 48, SU(3) FP16: 103 against 179 us matrix cores at 8 RHS, 188 / 207 at 12,
+    // 213 / 245 at 16, 374 / 759 at 32) or needs a second 16-wide matrix-core chunk (370 / 536 at 17);
+    // otherwise its loads straddle those pieces (190 / 175 at 6, 220 / 191 at 10), and below about
+    // 32768 lanes the matrix-core kernel's shorter chain of loads wins (8^3 x 16, 4 RHS: 8.1 / 6.7 us)
+    const bool fits16 = double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 &&
+                        double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;  // what the matrix-core kernel addresses
+    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16) && double(a.g.Vh) * a.R >= 32768.0) return kDslashLaneRhs;
+    return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
+}
+}  // namespace
+
 DslashTune dslash_fill_defaults(const DslashArgs &a, DslashTune t) {
-    if (t.variant == kDslashAuto) t.variant = dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
+    if (t.variant == kDslashAuto) t.variant = automatic_variant(a);
+    if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)) {
+        dslash_lane_tile(a.g, a.Nc, a.R, a.prec, t.by, t.bz);
+        return t;
+    }
     if (t.variant == kDslashMfma && !dslash_matrix_supported(a.Nc, a.prec)) t.variant = kDslashWaveSite;
     if (t.variant == kDslashLds && !dslash_lds_supported(a.g, a.Nc, a.prec))
         t.variant = dslash_matrix_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
@@ -272,6 +300,8 @@ hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
     const DslashTune t = dslash_resolve(a);
     if (t.variant == kDslashWaveSite) return launch_dslash_wave(a, t, stream);
     if (t.variant == kDslashLds) return launch_dslash_lds(a, t, stream);
+    if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec))
+        return launch_dslash_lane(a, t, stream);
     if (t.variant == kDslashMfma)
         return (a.prec == kSingle || a.prec == kDouble) ? launch_dslash_mfma32(a, t, stream)
                                                          : launch_dslash_mfma(a, t, stream);

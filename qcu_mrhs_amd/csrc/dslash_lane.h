@@ -1,0 +1,288 @@
+// dslash_lane.h -- device body of the lane-per-(site, RHS) hopping kernels
+// (dslash_lane.hip has the launches and the measurements).
+//
+// A workgroup takes `spb` consecutive traversal positions; lane l of it holds
+// one output site and V consecutive right-hand sides, and runs all eight hops
+// of them, so nothing is reduced across lanes and no lane idles whatever R is.
+// The walk-table rows and the 8 links of every site go through LDS (each is
+// read once by the workgroup and then broadcast to the lanes of its site); the
+// neighbour spinors are buffer loads whose (spin, colour) row offset is scalar.
+#pragma once
+
+#include <type_traits>
+
+#include "dslash_common.h"
+
+namespace qcu {
+namespace lane {
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
+}
+
+// The output of a hop is read by a later kernel only, after the caches have turned over: stored with
+// the non-temporal policy it leaves the XCD's L2 to the input spinors (24^3 x 48, 16 RHS: FP64
+// 730 -> 699 us, FP32 380 -> 363 us; 16^3 x 32, 12 RHS, FP64: 124 -> 97 us).
+constexpr int kStorePolicy = 2;  // gfx950 cache-policy bit nt
+
+// one load / store of B bytes at voffset + soffset
+template <int B> struct Raw;
+template <> struct Raw<4> {
+    using type = uint32_t;
+    __device__ __forceinline__ static type load(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+        return uint32_t(__builtin_amdgcn_raw_buffer_load_b32(r, int(v), int(s), 0));
+    }
+    __device__ __forceinline__ static void store(__amdgpu_buffer_rsrc_t r, type w, unsigned v, unsigned s) {
+        __builtin_amdgcn_raw_buffer_store_b32(int(w), r, int(v), int(s), kStorePolicy);
+    }
+};
+template <> struct Raw<8> {
+    using type = u32x2;
+    __device__ __forceinline__ static type load(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, int(v), int(s), 0));
+    }
+    __device__ __forceinline__ static void store(__amdgpu_buffer_rsrc_t r, type w, unsigned v, unsigned s) {
+        __builtin_amdgcn_raw_buffer_store_b64(w, r, int(v), int(s), kStorePolicy);
+    }
+};
+template <> struct Raw<16> {
+    using type = u32x4;
+    __device__ __forceinline__ static type load(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, int(v), int(s), 0));
+    }
+    __device__ __forceinline__ static void store(__amdgpu_buffer_rsrc_t r, type w, unsigned v, unsigned s) {
+        __builtin_amdgcn_raw_buffer_store_b128(w, r, int(v), int(s), kStorePolicy);
+    }
+};
+
+// Arithmetic of one storage type: C = stored complex, T = accumulation, Link = what LDS holds of a
+// link entry, H = one projected spinor entry.
+//   proj<K>(a, b) = a + i^K b;  madd(s, u, h): s += u h
+// FP32 / FP64 storage: everything in the storage type.
+template <typename S>
+struct Arith {
+    using T = S;
+    using C = Cx<S>;
+    using Link = Cx<S>;
+    using H = Cx<S>;
+    __device__ __forceinline__ static Link link(C u, bool fwd) { return fwd ? u : conj(u); }
+    template <int K>
+    __device__ __forceinline__ static H proj(C a, C b) { return a + ipow<K>(b); }
+    __device__ __forceinline__ static void madd(Cx<T> &s, const Link &u, H h) { cfma(s, u, h); }
+};
+// FP16 / BF16 storage: the projected entry is rounded to the storage type (as the matrix-core kernel
+// does) and a complex product is two 2-element dot products with FP32 accumulation (v_dot2_f32_{f16,
+// bf16}: half the instructions of FP32 FMAs), the link kept in LDS as the two words (Re, -Im) and
+// (Im, Re) they multiply.
+template <>
+struct Arith<__half> {
+    using T = float;
+    using C = Half2Store;
+    using Link = u32x2;
+    using H = uint32_t;
+    __device__ __forceinline__ static Link link(C u, bool fwd) {
+        const uint32_t w = __builtin_bit_cast(uint32_t, u);
+        const uint32_t sw = __builtin_amdgcn_perm(w, w, 0x01000302u);
+        return fwd ? Link{w ^ 0x80000000u, sw} : Link{w, sw ^ 0x00008000u};
+    }
+    template <int K>
+    __device__ __forceinline__ static H proj(C a, C b) {
+        const f16x2 x = __builtin_bit_cast(f16x2, a), y = __builtin_bit_cast(f16x2, b);
+        f16x2 r;
+        if constexpr ((K & 3) == 0) r = x + y;
+        else if constexpr ((K & 3) == 1) r = x + f16x2{-y[1], y[0]};
+        else if constexpr ((K & 3) == 2) r = x - y;
+        else r = x + f16x2{y[1], -y[0]};
+        return __builtin_bit_cast(uint32_t, r);
+    }
+    __device__ __forceinline__ static void madd(Cx<T> &s, const Link &u, H h) {
+        const f16x2 hh = __builtin_bit_cast(f16x2, h);
+        s.re = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, uint32_t(u[0])), hh, s.re, false);
+        s.im = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, uint32_t(u[1])), hh, s.im, false);
+    }
+};
+template <>
+struct Arith<__hip_bfloat16> {
+    using T = float;
+    using C = Bf162Store;
+    using Link = u32x2;
+    using H = uint32_t;
+    __device__ __forceinline__ static Link link(C u, bool fwd) {
+        const uint32_t w = __builtin_bit_cast(uint32_t, u);
+        const uint32_t sw = __builtin_amdgcn_perm(w, w, 0x01000302u);
+        return fwd ? Link{w ^ 0x80000000u, sw} : Link{w, sw ^ 0x00008000u};
+    }
+    template <int K>
+    __device__ __forceinline__ static H proj(C a, C b) {
+        const Cx<float> h = load_cx<float>(&a) + ipow<K>(load_cx<float>(&b));
+        C o;
+        store_cx(&o, h);
+        return __builtin_bit_cast(uint32_t, o);
+    }
+    __device__ __forceinline__ static void madd(Cx<T> &s, const Link &u, H h) {
+        const bf16x2 hh = __builtin_bit_cast(bf16x2, h);
+        s.re = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, uint32_t(u[0])), hh, s.re, false);
+        s.im = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, uint32_t(u[1])), hh, s.im, false);
+    }
+};
+
+// LDS words of one site's 8 links: one entry more than they need, so that the sites of a wavefront
+// reading the same entry start in different banks
+template <typename S, int NC>
+constexpr int kLinkRow = 8 * NC * NC + 1;
+template <typename S, int NC>
+constexpr int kSiteLds = kLinkRow<S, NC> * int(sizeof(typename Arith<S>::Link)) + 9 * int(sizeof(int));
+
+// V stored complex numbers as one register vector
+template <typename C, int V>
+struct Vec {
+    C c[V];
+};
+
+// Keeps the accumulators live here: every hop's arithmetic is done before the next hop's loads are
+// waited for.  Without it the compiler interleaves the hops until it spills (FP64, Nc = 3: 256
+// registers and 106 spilled, 1741 us at 24^3 x 48, 16 RHS, instead of 130 registers and 787 us).
+template <typename T, int NC, int V>
+__device__ __forceinline__ void pin(Cx<T> (&acc)[4][NC][V]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int v = 0; v < V; ++v) asm volatile("" : "+v"(acc[s][c][v].re), "+v"(acc[s][c][v].im));
+}
+
+template <typename S, int NC, int V, bool DAG, int MU, bool FWD>
+__device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], __amdgpu_buffer_rsrc_t r_in,
+                                    unsigned vo, unsigned row_bytes, const typename Arith<S>::Link *U) {
+    using A = Arith<S>;
+    using T = typename A::T;
+    using C = typename A::C;
+    using R = Raw<V * int(sizeof(C))>;
+    using W = Vec<C, V>;
+    constexpr int sgn = (FWD != DAG) ? 2 : 0;
+    constexpr int m0 = kMat2(MU, 0), m1 = kMat2(MU, 1);
+    constexpr int kp0 = kProjK(MU, 0) + sgn, kp1 = kProjK(MU, 1) + sgn;
+    constexpr int kr0 = kReconK(MU, 0) + sgn, kr1 = kReconK(MU, 1) + sgn;
+    asm volatile("" : "+v"(vo));  // the loads stay behind the previous hop's arithmetic (see pin)
+    W w[4][NC];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) w[s][c] = __builtin_bit_cast(W, R::load(r_in, vo, unsigned(s * NC + c) * row_bytes));
+    typename A::H h0[NC][V], h1[NC][V];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            h0[c][v] = A::template proj<kp0>(w[0][c].c[v], w[m0][c].c[v]);
+            h1[c][v] = A::template proj<kp1>(w[1][c].c[v], w[m1][c].c[v]);
+        }
+#pragma unroll
+    for (int a = 0; a < NC; ++a) {
+        Cx<T> s0[V], s1[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) s0[v] = s1[v] = {T(0), T(0)};
+#pragma unroll
+        for (int b = 0; b < NC; ++b) {
+            const typename A::Link u = U[a * NC + b];
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                A::madd(s0[v], u, h0[b][v]);
+                A::madd(s1[v], u, h1[b][v]);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            acc[0][a][v] = acc[0][a][v] + s0[v];
+            acc[m0][a][v] = acc[m0][a][v] + ipow<kr0>(s0[v]);
+            acc[1][a][v] = acc[1][a][v] + s1[v];
+            acc[m1][a][v] = acc[m1][a][v] + ipow<kr1>(s1[v]);
+        }
+    }
+    pin<T, NC, V>(acc);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// What a lane knows after the hops.
+struct Place {
+    bool active;    // holds a site of the workgroup (idle lanes repeat the last one)
+    int site;       // output site
+    int rv;         // RHS vector: right-hand sides rv V .. rv V + V - 1
+    int local;      // site within the workgroup
+    unsigned vo;    // byte offset of (site, spin 0, colour 0, rv V)
+};
+
+// acc = D in for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes per site.
+template <typename S, int NC, int V, bool DAG>
+__device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
+                                      const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
+                                      int R, int RV, int spb, int pos0, int parity, const int *walk,
+                                      unsigned vec_bytes) {
+    using A = Arith<S>;
+    using T = typename A::T;
+    using C = typename A::C;
+    constexpr int NN = NC * NC, LR = kLinkRow<S, NC>;
+    auto *sl = reinterpret_cast<typename A::Link *>(smem);
+    int *sw = reinterpret_cast<int *>(sl + spb * LR);
+    const int ns = min(spb, Vh - pos0);
+    const int *wt = walk + (long(parity) * Vh + pos0) * 9;
+    const int nt = blockDim.x;
+    for (int i = threadIdx.x; i < ns * 9; i += nt) sw[i] = wt[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < ns * 8 * NN; i += nt) {
+        const int l = i / (8 * NN), k = i / NN - l * 8, e = i - (l * 8 + k) * NN;
+        const bool fwd = (k & 1) == 0;
+        // V = U_mu(x) forward (parity of x), U_mu(x - mu)^+ backward
+        const int a = e / NC, b = e - a * NC;
+        const long li = fwd ? ((k >> 1) * 2 + parity) * long(Vh) + sw[l * 9]
+                            : ((k >> 1) * 2 + 1 - parity) * long(Vh) + sw[l * 9 + 1 + k];
+        sl[l * LR + k * NN + e] = A::link(gauge[li * NN + (fwd ? e : b * NC + a)], fwd);
+    }
+    __syncthreads();
+    Place p;
+    p.local = int(threadIdx.x) / RV;
+    p.rv = int(threadIdx.x) - p.local * RV;
+    p.active = p.local < ns;
+    const int l = min(p.local, ns - 1);
+    const unsigned rb = unsigned(R) * unsigned(sizeof(C)), sb = 4u * NC * rb;
+    const unsigned lo = unsigned(p.rv) * V * unsigned(sizeof(C));
+    const auto r_in = rsrc(in, vec_bytes);
+    const int *row = sw + l * 9;
+    const typename A::Link *U = sl + l * LR;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[s][c][v] = {T(0), T(0)};
+    // Hop order t-, z-, y-, x-, x+, y+, z+, t+: the traversal sweeps upwards, so the backward neighbours
+    // are the input sites about to leave the XCD's L2 and are read before the forward ones push them out
+    // (24^3 x 48, 16 RHS: FP64 711 -> 636 us, FP32 350 -> 323 us against x+, x-, ..., t+, t-; 786 and
+    // 393 us in the reverse order; 16^3 x 32, 12 RHS, FP64: 103 -> 79 us).
+#define QCU_BACK(MU) \
+    hop<S, NC, V, DAG, MU, false>(acc, r_in, unsigned(row[2 + 2 * MU]) * sb + lo, rb, U + (2 * MU + 1) * NN);
+#define QCU_FORW(MU) \
+    hop<S, NC, V, DAG, MU, true>(acc, r_in, unsigned(row[1 + 2 * MU]) * sb + lo, rb, U + (2 * MU) * NN);
+    QCU_BACK(3)
+    QCU_BACK(2)
+    QCU_BACK(1)
+    QCU_BACK(0)
+    QCU_FORW(0)
+    QCU_FORW(1)
+    QCU_FORW(2)
+    QCU_FORW(3)
+#undef QCU_BACK
+#undef QCU_FORW
+    p.site = row[0];
+    p.vo = unsigned(p.site) * sb + lo;
+    return p;
+}
+
+}  // namespace lane
+}  // namespace qcu

@@ -1,0 +1,195 @@
+// dslash_lane.hip -- lane-per-(site, RHS) Wilson hopping term (variant
+// kDslashLaneRhs, dslash_lane.h), every storage precision, Nc <= 4.
+//
+// What bounds it: the bytes that miss the XCD's L2 (FP64, FP32: 4.9 and 2.2 GB
+// per hop at 24^3 x 48, 16 RHS, at 6-7 TB/s, against 2.4 and 1.2 GB that the
+// operator needs) and, in 16 bits, the L2 -> L1 fill of the neighbour spinors
+// (48 lines per site; the same loads without the arithmetic take the same time).
+// Against the wave-per-site kernel, whose 16 lanes per direction idle when R is
+// no multiple of 16 and whose cross-lane sums cost 3.5 times the instructions
+// per site: FP64 24^3 x 48, 16 RHS 1012 -> 636 us, 16^3 x 32, 12 RHS 190 -> 79 us,
+// 8^4, 4 RHS 22 -> 9 us; FP32 592 -> 323 us, 109 -> 57 us, 20 -> 9 us; SU(4) 16^4,
+// 17 RHS FP32 131 -> 62 us.
+#include <algorithm>
+
+#include "dslash_lane.h"
+#include "geom.h"
+
+namespace qcu {
+namespace {
+
+using namespace lane;
+
+extern __shared__ __align__(16) unsigned char lane_smem[];
+
+// Wavefronts per SIMD the register budget is set for: accumulators, a hop's spinor rows and its projected
+// entries fit without spilling (Nc = 3: 130 registers FP64, 67 FP32, 62 FP16).
+template <typename S, int NC, int V>
+constexpr int kMinWaves = NC * V * int(sizeof(typename Arith<S>::T)) >= 32 ? 2 : NC * V * int(sizeof(typename Arith<S>::T)) >= 24 ? 3 : 4;
+
+// out = coef D in (+ xpay)
+template <typename S, int NC, int V, bool DAG>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
+    int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
+    using T = typename Arith<S>::T;
+    using C = typename Arith<S>::C;
+    using RW = Raw<V * int(sizeof(C))>;
+    using W = Vec<C, V>;
+    Cx<T> acc[4][NC][V];
+    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
+                                        xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
+    if (!p.active) return;
+    const unsigned rb = unsigned(R) * unsigned(sizeof(C));
+    const auto r_out = rsrc(out, vec_bytes);
+    if (xpay) {
+        const auto r_x = rsrc(xpay, vec_bytes);
+        W xw[4][NC];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) xw[s][c] = __builtin_bit_cast(W, RW::load(r_x, p.vo, unsigned(s * NC + c) * rb));
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                W o;
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    Cx<T> x = load_cx<T>(&xw[s][c].c[v]);
+                    x.re = fma(coef, acc[s][c][v].re, x.re);
+                    x.im = fma(coef, acc[s][c][v].im, x.im);
+                    store_cx(&o.c[v], x);
+                }
+                RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(s * NC + c) * rb);
+            }
+    } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                W o;
+#pragma unroll
+                for (int v = 0; v < V; ++v) store_cx(&o.c[v], coef * acc[s][c][v]);
+                RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(s * NC + c) * rb);
+            }
+    }
+}
+
+// Launch shape: V right-hand sides per lane, `spb` sites per workgroup of `threads` lanes.
+struct Shape {
+    int V, RV, spb, threads;
+    size_t lds;
+};
+
+template <typename S, int NC>
+Shape lane_shape(int Vh, int R, int v) {
+    Shape s;
+    s.V = v;
+    s.RV = R / s.V;
+    constexpr int per_site = kSiteLds<S, NC>;
+    // 256 lanes, fewer where the grid would leave compute units idle (a site's hops are one serial
+    // chain, so a small lattice runs at the speed of one workgroup: more, smaller ones)
+    s.threads = 256;
+    while (s.threads > 64 && s.threads / 2 >= s.RV && div_up(Vh, std::max(1, s.threads / s.RV)) < 2 * num_cus())
+        s.threads /= 2;
+    s.spb = std::max(1, s.threads / s.RV);
+    s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 ? 65536 : 40960) / per_site));  // 64 KB of LDS at most
+    s.threads = (s.spb * s.RV + 63) / 64 * 64;
+    s.lds = size_t(s.spb) * per_site;
+    return s;
+}
+
+template <typename S, int NC, int V, bool DAG>
+hipError_t launch_v(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
+    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, V);
+    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
+    hipLaunchKernelGGL((k_dslash_lane<S, NC, V, DAG>), dim3(div_up(a.g.Vh, sh.spb)), dim3(sh.threads), sh.lds, stream,
+                       static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.xpay), typename Arith<S>::T(a.coef), a.g.Vh, a.R, sh.RV, sh.spb,
+                       a.parity, tab.walk, vec_bytes);
+    return hipGetLastError();
+}
+
+template <typename S, int NC>
+hipError_t launch_nc(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    // FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
+    // the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
+    // 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache
+    // one per lane, at twice the wavefronts, is faster (16^3 x 32, 12 RHS: 57 against 61 us).
+    if constexpr (std::is_same<S, float>::value && NC <= 3) {
+        const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * sizeof(C);
+        if (a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0)
+            return a.dagger ? launch_v<S, NC, 2, true>(a, t, stream) : launch_v<S, NC, 2, false>(a, t, stream);
+    }
+    return a.dagger ? launch_v<S, NC, 1, true>(a, t, stream) : launch_v<S, NC, 1, false>(a, t, stream);
+}
+
+template <typename S>
+hipError_t launch_s(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    switch (a.Nc) {
+        case 2: return launch_nc<S, 2>(a, t, stream);
+        case 3: return launch_nc<S, 3>(a, t, stream);
+        case 4: return launch_nc<S, 4>(a, t, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+// one buffer resource spans a vector: below 4 GiB
+bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec) {
+    return Nc <= 4 && double(g.Vh) * 4.0 * Nc * R * 2.0 * double(prec_bytes(prec)) < 4294967296.0;
+}
+
+// Traversal tile: rows of x and a (by, bz) tile of them per t slice.  The input rows outside the tile
+// (2 / by + 2 / bz + the t faces of an XCD's share, per site) are read again by the neighbouring tile,
+// so the tile is as large as the XCD's 4 MB L2 lets three slices of it survive: up to 900 sites and
+// 2.75 MB per slice; a whole number of tile columns per XCD where there are 8 or more (24^3 x 48,
+// 16 RHS: (6, 12) 323 us FP32, 641 us FP64, (8, 8) -- 9 columns -- 364 and 661 us, (4, 4) 380 and
+// 708 us, untiled 398 and 839 us).
+void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz) {
+    const double site_bytes = 4.0 * Nc * R * 2.0 * double(prec_bytes(prec));
+    const int Ly = g.L[1], Lz = g.L[2], Lt = g.L[3];
+    const bool keep_y = by > 0 && Ly % by == 0, keep_z = bz > 0 && Lz % bz == 0;
+    const int want_y = by, want_z = bz;
+    double best = 1e30;
+    by = bz = 1;
+    for (int y = 1; y <= Ly; ++y) {
+        if (Ly % y || (keep_y && y != want_y)) continue;
+        for (int z = 1; z <= Lz; ++z) {
+            if (Lz % z || (keep_z && z != want_z)) continue;
+            const double sites = double(g.Lxh) * y * z;
+            const int cols = (Ly / y) * (Lz / z);
+            double cost = (y < Ly ? 1.0 / y : 0.0) + (z < Lz ? 1.0 / z : 0.0);
+            if (cols < kNumXcd) cost += double(kNumXcd) / (double(cols) * Lt);
+            else if (cols % kNumXcd) cost += 0.05;
+            if (sites > 900.0 || sites * site_bytes > 2.75e6) cost += 100.0 * sites * y * z;
+            if (cost < best) {
+                best = cost;
+                by = y;
+                bz = z;
+            }
+        }
+    }
+}
+
+hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 || a.g.L[1] % t.by ||
+        a.g.L[2] % t.bz)
+        return hipErrorInvalidValue;
+    switch (a.prec) {
+        case kDouble: return launch_s<double>(a, t, stream);
+        case kSingle: return launch_s<float>(a, t, stream);
+        case kHalf: return launch_s<__half>(a, t, stream);
+        case kBF16: return launch_s<__hip_bfloat16>(a, t, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace qcu

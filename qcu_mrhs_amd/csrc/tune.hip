@@ -92,7 +92,10 @@ hipError_t dslash_autotune(const int L[4], int Nc, int R, int prec, int reps, Ds
     std::vector<int> bys, bzs;
     divisors_upto(L[1], 12, bys);
     divisors_upto(L[2], 12, bzs);
-    const int area0 = std::max(1, def.by * def.bz);
+    DslashTune wave;  // the tile area the wave-per-site and matrix-core kernels default to
+    wave.variant = kDslashWaveSite;
+    wave = dslash_fill_defaults(base, wave);
+    const int area0 = std::max(1, wave.by * wave.bz);
     std::vector<int> variants = {kDslashWaveSite};
     if (dslash_matrix_supported(Nc, prec)) variants.push_back(kDslashMfma);
     for (int v : variants) {
@@ -113,6 +116,11 @@ hipError_t dslash_autotune(const int L[4], int Nc, int R, int prec, int reps, Ds
         }
     }
     add(kDslashLaneRhs, 0, 0, 0);
+    if (dslash_lane_supported(g, Nc, R, prec))  // its traversal tiles of 256 to 1536 sites per slice
+        for (int by : bys)
+            for (int bz : bzs)
+                if (by * bz * g.Lxh >= 256 && by * bz * g.Lxh <= 1536 && by <= 2 * bz && bz <= 2 * by)
+                    add(kDslashLaneRhs, by, bz, 0);
     // (the LDS-staged kernel, kDslashLds, is not a candidate: on the synthetic fill timed here it
     // runs up to 14 % faster than on physical fields, enough to win a pick it then loses)
     auto time_shape = [&](const DslashTune &t, double &us) -> hipError_t {
