@@ -222,13 +222,13 @@ typedef struct QcuGroupInfo_s {
 
 int qcuInvertGroups(int n_groups, const QcuRhsGroup *groups, int max_iteration, double tol, QcuGroupInfo *info);
 /* Dslash kernel the last qcuInvertGroups batch ran, as chosen by its timing
- * of the candidates: 2 = VALU wave per site, 3 = FP32 matrix cores
+ * of the candidates: 1 = lane per (site, RHS), 2 = VALU wave per site, 3 = FP32 matrix cores
  * (v_mfma_f32_16x16x4_f32, FP32 storage) per group, 5 = FP32 matrix cores
  * over the groups' right-hand sides packed into shared 16-RHS chunks; 0
  * before any batch, -1 without initGridSize. */
 int qcuGroupsDslashVariant(void);
-/* The same for the FP64 hops of the batch's defect correction: 2 = VALU wave
- * per site, 3 / 5 = FP64 matrix cores (v_mfma_f64_16x16x4_f64) per group /
+/* The same for the FP64 hops of the batch's defect correction: 1 = lane per
+ * (site, RHS), 2 = VALU wave per site, 3 / 5 = FP64 matrix cores (v_mfma_f64_16x16x4_f64) per group /
  * over packed chunks; timed once per batch shape.  No reference counterpart. */
 int qcuGroupsDslashVariant64(void);
 /* Choose the batched groups' dslash kernels for every later qcuInvertGroups

@@ -65,6 +65,13 @@ bool dslash_mfma_supported(int Nc, int prec);
 hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
 void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
+// workgroups of a launch with one RHS per lane (rows of partial sums of the fused forms below); Nc <= 4
+int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec);
+hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
+                                       const double *scale, double *partials, int &nblk, hipStream_t stream);
+hipError_t launch_dslash_lane_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
+                                    int &nblk);
+hipError_t launch_dslash_lane_groups(const DslashArgs &a, const SegTab &tab, int by, int bz, hipStream_t stream);
 hipError_t launch_dslash_lds(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_lds_supported(const Geom &g, int Nc, int prec);
 // FP32 / FP64 storage on the FP32 / FP64 matrix cores (dslash_mfma32.hip), also for batched groups
@@ -85,12 +92,12 @@ inline bool dslash_groups_matrix_supported(int Nc, int prec) {
 }
 
 // Second hop of the FP64 Schur operator fused with the reliable-update residual
-// (wave-per-site kernel, dagger 0): with v = a.xpay + a.coef D a.in on parity
+// (lane or wave-per-site kernel, dagger 0): with v = a.xpay + a.coef D a.in on parity
 // a.parity, writes lo = scale[r] (b - v) in storage lo_prec (single, half, bf16)
 // and nrm[r] = ||b - v|| (deterministic: per-workgroup partials summed in a
 // fixed order by two small launches).  v itself is not stored.  `partials` holds at least
-// dslash_residual_partials(g, R) doubles.
-long dslash_residual_partials(const Geom &g, int R);
+// dslash_residual_partials(g, Nc, R) doubles.
+long dslash_residual_partials(const Geom &g, int Nc, int R);
 hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *lo, int lo_prec, const double *scale,
                                      double *partials, long partials_cap, double *nrm, hipStream_t stream);
 
@@ -99,12 +106,11 @@ hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *l
 hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, int slices, hipStream_t stream);
 
 // Second hop of the unpreconditioned FP16 / BF16 Schur operator, t = s + coef D in with
-// a.xpay = s, with omega's inner products <t, s>, <t, t> in its epilogue (matrix-core
-// kernel, dagger 0): omega = <t, s> / <t, t> lands in st like launch_step_omega.
-// `partials` holds dslash_omega_partials(g, R) doubles.  Returns hipErrorNotSupported
-// (and launches nothing) when the tuned launch for these arguments is not the
-// matrix-core kernel; the caller then runs the separate reduction.
-long dslash_omega_partials(const Geom &g, int R);
+// a.xpay = s, with omega's inner products <t, s>, <t, t> in its epilogue (lane or
+// matrix-core kernel, dagger 0): omega = <t, s> / <t, t> lands in st like launch_step_omega.
+// `partials` holds dslash_omega_partials(g, Nc, R) doubles.  Returns hipErrorNotSupported
+// (and launches nothing) when the tuned launch for these arguments is neither; the caller then runs the separate reduction.
+long dslash_omega_partials(const Geom &g, int Nc, int R);
 hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, Cx<double> *st, hipStream_t stream);
 hipError_t launch_dslash_mfma_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
                                     int &nblk);

@@ -316,9 +316,10 @@ hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
 
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
-long dslash_omega_partials(const Geom &g, int R) {
-    // one row of R x 4 per workgroup (at most one per 4 sites, or 64 per CU for the persistent grid)
-    const long nblk = std::max<long>(div_up(g.Vh, 4), 64L * num_cus());
+long dslash_omega_partials(const Geom &g, int Nc, int R) {
+    // one row of R x 4 per workgroup (matrix cores: at most one per 4 sites, or 64 per CU for the persistent grid)
+    const long lane = Nc <= 4 ? dslash_lane_blocks(g, Nc, R, kHalf) : 0;
+    const long nblk = std::max<long>({long(div_up(g.Vh, 4)), 64L * num_cus(), lane});
     return (nblk + kDotSlices) * R * 4;
 }
 
@@ -327,10 +328,12 @@ hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, 
         !a.xpay || !partials || !st || a.R > kReduceThreads)
         return hipErrorNotSupported;
     const DslashTune t = dslash_resolve(a);
-    if (t.variant != kDslashMfma) return hipErrorNotSupported;
-    if (cap < dslash_omega_partials(a.g, a.R)) return hipErrorInvalidValue;
+    const bool lane = t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
+    if (!lane && t.variant != kDslashMfma) return hipErrorNotSupported;
+    if (cap < dslash_omega_partials(a.g, a.Nc, a.R)) return hipErrorInvalidValue;
     int nblk = 0;
-    QCU_HIP_TRY(launch_dslash_mfma_omega(a, t, partials, stream, nblk));
+    if (lane) QCU_HIP_TRY(launch_dslash_lane_omega(a, t, partials, stream, nblk));
+    else QCU_HIP_TRY(launch_dslash_mfma_omega(a, t, partials, stream, nblk));
     // [nblk][R][4] -> [kDotSlices][R][4] (after them) -> the finisher sums the slices in order
     double *p2 = partials + long(nblk) * a.R * 4;
     QCU_HIP_TRY(launch_rows_sum(p2, partials, nblk, 4 * a.R, kDotSlices, stream));

@@ -27,20 +27,15 @@ extern __shared__ __align__(16) unsigned char lane_smem[];
 template <typename S, int NC, int V>
 constexpr int kMinWaves = NC * V * int(sizeof(typename Arith<S>::T)) >= 32 ? 2 : NC * V * int(sizeof(typename Arith<S>::T)) >= 24 ? 3 : 4;
 
-// out = coef D in (+ xpay)
-template <typename S, int NC, int V, bool DAG>
-__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane(
-    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
-    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
-    int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
+// out = coef acc (+ xpay) at this lane's place
+template <typename S, int NC, int V>
+__device__ __forceinline__ void store_lane(const Cx<typename Arith<S>::T> (&acc)[4][NC][V], typename Arith<S>::C *out,
+                                           const typename Arith<S>::C *xpay, typename Arith<S>::T coef, const Place &p,
+                                           int R, unsigned vec_bytes) {
     using T = typename Arith<S>::T;
     using C = typename Arith<S>::C;
     using RW = Raw<V * int(sizeof(C))>;
     using W = Vec<C, V>;
-    Cx<T> acc[4][NC][V];
-    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
-                                        xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
-    if (!p.active) return;
     const unsigned rb = unsigned(R) * unsigned(sizeof(C));
     const auto r_out = rsrc(out, vec_bytes);
     if (xpay) {
@@ -77,6 +72,153 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane(
     }
 }
 
+// out = coef D in (+ xpay)
+template <typename S, int NC, int V, bool DAG>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
+    int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
+    Cx<typename Arith<S>::T> acc[4][NC][V];
+    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
+                                        xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
+    if (p.active) store_lane<S, NC, V>(acc, out, xpay, coef, p, R, vec_bytes);
+}
+
+// Sums `n` values per lane over the workgroup's sites, per RHS, in site order: row[rv] for the first RV lanes.
+// red: n rows of blockDim.x doubles.
+template <int N>
+__device__ __forceinline__ void sum_sites(double (&v)[N], double *red, const Place &p, int RV, int ns) {
+    __syncthreads();  // the hops' LDS is free
+    const int nt = blockDim.x;
+#pragma unroll
+    for (int k = 0; k < N; ++k) red[k * nt + threadIdx.x] = p.active ? v[k] : 0.0;
+    __syncthreads();
+    if (int(threadIdx.x) < RV) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            double t = 0.0;
+            for (int l = 0; l < ns; ++l) t += red[k * nt + l * RV + threadIdx.x];
+            v[k] = t;
+        }
+    }
+}
+
+// Reliable-update residual (FP64 hop): d = b - (xpay + coef D in) is not stored; lo = scale_r d in the inner
+// storage and part[block][r] = sum over the workgroup's sites of |d|^2.
+template <int NC, typename LO>
+__global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane_residual(
+    LO *__restrict__ lo, const Cx<double> *__restrict__ in, const Cx<double> *__restrict__ gauge,
+    const Cx<double> *__restrict__ xpay, const Cx<double> *__restrict__ b, const double *__restrict__ scale,
+    double *__restrict__ part, double coef, int Vh, int R, int spb, int parity, const int *__restrict__ walk,
+    unsigned vec_bytes) {
+    using RL = Raw<int(sizeof(LO))>;
+    using W = Vec<Cx<double>, 1>;
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    Cx<double> acc[4][NC][1];
+    const Place p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk,
+                                               vec_bytes);
+    double a2[1] = {0.0};
+    if (p.active) {
+        const unsigned rb = unsigned(R) * 16u;
+        const auto r_x = rsrc(xpay, vec_bytes), r_b = rsrc(b, vec_bytes);
+        const auto r_lo = rsrc(lo, vec_bytes / 16u * unsigned(sizeof(LO)));
+        const double sc = scale[p.rv];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            W xw[NC], bw[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                xw[c] = __builtin_bit_cast(W, Raw<16>::load(r_x, p.vo, unsigned(s * NC + c) * rb));
+                bw[c] = __builtin_bit_cast(W, Raw<16>::load(r_b, p.vo, unsigned(s * NC + c) * rb));
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                Cx<double> v = xw[c].c[0];
+                v.re = fma(coef, acc[s][c][0].re, v.re);
+                v.im = fma(coef, acc[s][c][0].im, v.im);
+                const Cx<double> d = bw[c].c[0] - v;
+                a2[0] = fma(d.re, d.re, fma(d.im, d.im, a2[0]));
+                LO o;
+                store_cx(&o, sc * d);
+                RL::store(r_lo, __builtin_bit_cast(typename RL::type, o), p.vo / 16u * unsigned(sizeof(LO)),
+                          unsigned(s * NC + c) * unsigned(R) * unsigned(sizeof(LO)));
+            }
+        }
+    }
+    sum_sites<1>(a2, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
+    if (int(threadIdx.x) < R) part[long(blockIdx.x) * R + threadIdx.x] = a2[0];
+}
+
+// Second hop of t = s + coef D in (16 bits) with omega's inner products over the stored values:
+// part[block][r][4] = Re, Im of <t, s>, <t, t>.
+template <typename S, int NC>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_omega(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay, float coef, int Vh,
+    int R, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes, double *__restrict__ part) {
+    using C = typename Arith<S>::C;
+    using RW = Raw<int(sizeof(C))>;
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    Cx<float> acc[4][NC][1];
+    const Place p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
+    float q[3] = {0.f, 0.f, 0.f};
+    if (p.active) {
+        const unsigned rb = unsigned(R) * unsigned(sizeof(C));
+        const auto r_out = rsrc(out, vec_bytes), r_x = rsrc(xpay, vec_bytes);
+        C xw[4][NC];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) xw[s][c] = __builtin_bit_cast(C, RW::load(r_x, p.vo, unsigned(s * NC + c) * rb));
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const Cx<float> x = load_cx<float>(&xw[s][c]);
+                const Cx<float> v = {fmaf(coef, acc[s][c][0].re, x.re), fmaf(coef, acc[s][c][0].im, x.im)};
+                C o;
+                store_cx(&o, v);
+                RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(s * NC + c) * rb);
+                const Cx<float> t = load_cx<float>(&o);  // as a separate reduction would read it
+                q[0] = fmaf(x.re, t.re, fmaf(x.im, t.im, q[0]));
+                q[1] = fmaf(t.re, x.im, fmaf(-t.im, x.re, q[1]));
+                q[2] = fmaf(t.re, t.re, fmaf(t.im, t.im, q[2]));
+            }
+    }
+    double w[3] = {double(q[0]), double(q[1]), double(q[2])};
+    sum_sites<3>(w, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
+    if (int(threadIdx.x) < R) {
+        double *row = part + (long(blockIdx.x) * R + threadIdx.x) * 4;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) row[k] = w[k];
+        row[3] = 0.0;
+    }
+}
+
+// Every group of a batch in one launch (blockIdx.y = group, SegTab layout); spb[g] sites per workgroup.
+struct GroupSites {
+    int spb[kMaxGroups];
+};
+template <typename S, int NC, bool DAG>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_groups(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
+    typename Arith<S>::T coef, int Vh, int parity, const int *__restrict__ walk, SegTab tab, GroupSites gs) {
+    using T = typename Arith<S>::T;
+    using C = typename Arith<S>::C;
+    const int grp = blockIdx.y;
+    if (tab.done && tab.done[grp]) return;
+    const int spb = gs.spb[grp], R = tab.R[grp];
+    const int nblk = (Vh + spb - 1) / spb;
+    if (int(blockIdx.x) >= nblk) return;
+    const long off = tab.n * tab.base[grp];
+    const unsigned vec_bytes = unsigned(tab.n * R * long(sizeof(C)));
+    Cx<T> acc[4][NC][1];
+    const Place p = hops<S, NC, 1, DAG>(acc, lane_smem, in + off, gauge, Vh, R, R, spb,
+                                        xcd_remap(blockIdx.x, nblk) * spb, parity, walk, vec_bytes);
+    if (p.active) store_lane<S, NC, 1>(acc, out + off, xpay ? xpay + off : nullptr, coef, p, R, vec_bytes);
+}
+
 // Launch shape: V right-hand sides per lane, `spb` sites per workgroup of `threads` lanes.
 struct Shape {
     int V, RV, spb, threads;
@@ -97,8 +239,86 @@ Shape lane_shape(int Vh, int R, int v) {
     s.spb = std::max(1, s.threads / s.RV);
     s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 ? 65536 : 40960) / per_site));  // 64 KB of LDS at most
     s.threads = (s.spb * s.RV + 63) / 64 * 64;
-    s.lds = size_t(s.spb) * per_site;
+    s.lds = std::max(size_t(s.spb) * per_site, size_t(s.threads) * 3 * sizeof(double));  // hops, then sums over sites
     return s;
+}
+
+template <typename S>
+Shape lane_shape_nc(int Nc, int Vh, int R) {
+    return Nc == 2 ? lane_shape<S, 2>(Vh, R, 1) : Nc == 3 ? lane_shape<S, 3>(Vh, R, 1) : lane_shape<S, 4>(Vh, R, 1);
+}
+
+template <int NC, typename LO>
+hipError_t launch_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, const double *scale,
+                           double *partials, int &nblk, hipStream_t stream) {
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
+    const Shape sh = lane_shape<double, NC>(a.g.Vh, a.R, 1);
+    nblk = div_up(a.g.Vh, sh.spb);
+    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * 16);
+    hipLaunchKernelGGL((k_dslash_lane_residual<NC, LO>), dim3(nblk), dim3(sh.threads), sh.lds, stream,
+                       static_cast<LO *>(lo), static_cast<const Cx<double> *>(a.in),
+                       static_cast<const Cx<double> *>(a.gauge), static_cast<const Cx<double> *>(a.xpay),
+                       static_cast<const Cx<double> *>(b), scale, partials, a.coef, a.g.Vh, a.R, sh.spb, a.parity,
+                       tab.walk, vec_bytes);
+    return hipGetLastError();
+}
+
+template <int NC>
+hipError_t launch_residual_lo(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
+                              const double *scale, double *partials, int &nblk, hipStream_t stream) {
+    switch (lo_prec) {
+        case kSingle: return launch_residual<NC, Cx<float>>(a, t, b, lo, scale, partials, nblk, stream);
+        case kHalf: return launch_residual<NC, Half2Store>(a, t, b, lo, scale, partials, nblk, stream);
+        case kBF16: return launch_residual<NC, Bf162Store>(a, t, b, lo, scale, partials, nblk, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <typename S, int NC>
+hipError_t launch_omega(const DslashArgs &a, const DslashTune &t, double *partials, int &nblk, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
+    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, 1);
+    nblk = div_up(a.g.Vh, sh.spb);
+    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
+    hipLaunchKernelGGL((k_dslash_lane_omega<S, NC>), dim3(nblk), dim3(sh.threads), sh.lds, stream,
+                       static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.xpay), float(a.coef), a.g.Vh, a.R, sh.spb, a.parity, tab.walk,
+                       vec_bytes, partials);
+    return hipGetLastError();
+}
+
+template <typename S, int NC>
+hipError_t launch_groups(const DslashArgs &a, const SegTab &seg, int by, int bz, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, by, bz, tab, stream));
+    GroupSites gs{};
+    int nmax = 1, smax = 1;
+    for (int k = 0; k < seg.G; ++k) {
+        gs.spb[k] = std::min(std::max(1, 256 / seg.R[k]), std::max(1, 40960 / kSiteLds<S, NC>));
+        nmax = std::max(nmax, div_up(a.g.Vh, gs.spb[k]));
+        smax = std::max(smax, gs.spb[k]);
+    }
+    auto k = a.dagger ? k_dslash_lane_groups<S, NC, true> : k_dslash_lane_groups<S, NC, false>;
+    constexpr int per_site = kSiteLds<S, NC>;
+    hipLaunchKernelGGL(k, dim3(nmax, seg.G), dim3(256), size_t(smax) * per_site, stream,
+                       static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.xpay), typename Arith<S>::T(a.coef), a.g.Vh, a.parity, tab.walk, seg,
+                       gs);
+    return hipGetLastError();
+}
+
+template <typename S>
+hipError_t launch_groups_s(const DslashArgs &a, const SegTab &seg, int by, int bz, hipStream_t stream) {
+    switch (a.Nc) {
+        case 2: return launch_groups<S, 2>(a, seg, by, bz, stream);
+        case 3: return launch_groups<S, 3>(a, seg, by, bz, stream);
+        case 4: return launch_groups<S, 4>(a, seg, by, bz, stream);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 template <typename S, int NC, int V, bool DAG>
@@ -188,6 +408,55 @@ hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStrea
         case kSingle: return launch_s<float>(a, t, stream);
         case kHalf: return launch_s<__half>(a, t, stream);
         case kBF16: return launch_s<__hip_bfloat16>(a, t, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec) {
+    const Shape sh = prec == kDouble ? lane_shape_nc<double>(Nc, g.Vh, R)
+                     : prec == kSingle ? lane_shape_nc<float>(Nc, g.Vh, R)
+                                       : lane_shape_nc<__half>(Nc, g.Vh, R);
+    return div_up(g.Vh, sh.spb);
+}
+
+hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
+                                       const double *scale, double *partials, int &nblk, hipStream_t stream) {
+    if (a.prec != kDouble || !dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 ||
+        a.g.L[1] % t.by || a.g.L[2] % t.bz)
+        return hipErrorInvalidValue;
+    switch (a.Nc) {
+        case 2: return launch_residual_lo<2>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
+        case 3: return launch_residual_lo<3>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
+        case 4: return launch_residual_lo<4>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_dslash_lane_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
+                                    int &nblk) {
+    if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 || a.g.L[1] % t.by || a.g.L[2] % t.bz)
+        return hipErrorInvalidValue;
+    const bool h = a.prec == kHalf;
+    if (!h && a.prec != kBF16) return hipErrorInvalidValue;
+    switch (a.Nc) {
+        case 2: return h ? launch_omega<__half, 2>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 2>(a, t, partials, nblk, stream);
+        case 3: return h ? launch_omega<__half, 3>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 3>(a, t, partials, nblk, stream);
+        case 4: return h ? launch_omega<__half, 4>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 4>(a, t, partials, nblk, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_dslash_lane_groups(const DslashArgs &a, const SegTab &tab, int by, int bz, hipStream_t stream) {
+    if (tab.G < 1 || tab.G > kMaxGroups || by <= 0 || bz <= 0 || a.g.L[1] % by || a.g.L[2] % bz)
+        return hipErrorInvalidValue;
+    for (int k = 0; k < tab.G; ++k)
+        if (tab.R[k] < 1 || !dslash_supported(a.Nc, tab.R[k]) || !dslash_lane_supported(a.g, a.Nc, tab.R[k], a.prec))
+            return hipErrorInvalidValue;
+    switch (a.prec) {
+        case kDouble: return launch_groups_s<double>(a, tab, by, bz, stream);
+        case kSingle: return launch_groups_s<float>(a, tab, by, bz, stream);
+        case kHalf: return launch_groups_s<__half>(a, tab, by, bz, stream);
+        case kBF16: return launch_groups_s<__hip_bfloat16>(a, tab, by, bz, stream);
         default: return hipErrorInvalidValue;
     }
 }

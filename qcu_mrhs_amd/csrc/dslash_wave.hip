@@ -280,33 +280,24 @@ constexpr int kResidualSlices = 64;  // first-level slices of the per-workgroup 
 
 template <int NC, typename LO>
 hipError_t launch_residual_nc(const DslashArgs &a, const DslashTune &t, const void *b, void *lo,
-                              const double *scale, double *partials, double *nrm, hipStream_t stream) {
-    const int nblk = div_up(a.g.Vh, 4 * t.spw);
+                              const double *scale, double *partials, int &nblk, hipStream_t stream) {
+    nblk = div_up(a.g.Vh, 4 * t.spw);
     hipLaunchKernelGGL((k_dslash_wave_residual<NC, LO>), dim3(nblk), dim3(256), size_t(4) * a.R * sizeof(double),
                        stream, static_cast<LO *>(lo), static_cast<const Cx<double> *>(a.in),
                        static_cast<const Cx<double> *>(a.gauge), static_cast<const Cx<double> *>(a.xpay),
                        static_cast<const Cx<double> *>(b), scale, partials, a.coef, a.g, a.R, a.parity, t.by, t.bz,
                        t.spw);
-    QCU_HIP_TRY(hipGetLastError());
-    // partials [nblk][R] -> [kResidualSlices][R] (stored after them) -> nrm
-    double *p2 = partials + long(nblk) * a.R;
-    const int cols = a.R < 256 ? a.R : 256;
-    hipLaunchKernelGGL(k_rows_sum, dim3(kResidualSlices, div_up(a.R, cols)), dim3(256), 0, stream, p2,
-                       static_cast<const double *>(partials), nblk, a.R, div_up(nblk, kResidualSlices), false);
-    QCU_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_rows_sum, dim3(1, div_up(a.R, cols)), dim3(256), 0, stream, nrm,
-                       static_cast<const double *>(p2), kResidualSlices, a.R, kResidualSlices, true);
     return hipGetLastError();
 }
 
 template <typename LO>
 hipError_t launch_residual_lo_t(const DslashArgs &a, const DslashTune &t, const void *b, void *lo,
-                                const double *scale, double *partials, double *nrm, hipStream_t stream) {
+                                const double *scale, double *partials, int &nblk, hipStream_t stream) {
     switch (a.Nc) {
-        case 2: return launch_residual_nc<2, LO>(a, t, b, lo, scale, partials, nrm, stream);
-        case 3: return launch_residual_nc<3, LO>(a, t, b, lo, scale, partials, nrm, stream);
-        case 4: return launch_residual_nc<4, LO>(a, t, b, lo, scale, partials, nrm, stream);
-        case 8: return launch_residual_nc<8, LO>(a, t, b, lo, scale, partials, nrm, stream);
+        case 2: return launch_residual_nc<2, LO>(a, t, b, lo, scale, partials, nblk, stream);
+        case 3: return launch_residual_nc<3, LO>(a, t, b, lo, scale, partials, nblk, stream);
+        case 4: return launch_residual_nc<4, LO>(a, t, b, lo, scale, partials, nblk, stream);
+        case 8: return launch_residual_nc<8, LO>(a, t, b, lo, scale, partials, nblk, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -398,7 +389,10 @@ hipError_t launch_dslash_wave(const DslashArgs &a, const DslashTune &t, hipStrea
     }
 }
 
-long dslash_residual_partials(const Geom &g, int R) { return (long(div_up(g.Vh, 4)) + kResidualSlices) * R; }
+long dslash_residual_partials(const Geom &g, int Nc, int R) {
+    const int lane = Nc <= 4 ? dslash_lane_blocks(g, Nc, R, kDouble) : 0;
+    return (long(std::max(div_up(g.Vh, 4), lane)) + kResidualSlices) * R;
+}
 
 hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, int slices, hipStream_t stream) {
     if (nrows < 1 || cols < 1 || slices < 1) return hipErrorInvalidValue;
@@ -414,22 +408,34 @@ hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *l
         a.R < 1 || 32L * a.R > 65536L || !dslash_supported(a.Nc, a.R))
         return hipErrorInvalidValue;
     if (a.g.Vh <= 0) return hipSuccess;
-    // the wave kernel's launch shape for this operator (forced when the tuned variant is another)
+    // the lane kernel where the hop itself runs it, else the wave kernel
+    if (partials_cap < dslash_residual_partials(a.g, a.Nc, a.R)) return hipErrorInvalidValue;
     DslashTune t = dslash_resolve(a);
-    if (t.variant != kDslashWaveSite) {
-        DslashArgs w = a;
-        w.tune = DslashTune{};
-        w.tune.variant = kDslashWaveSite;
-        t = dslash_resolve(w);
+    int nblk = 0;
+    if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)) {
+        QCU_HIP_TRY(launch_dslash_lane_residual(a, t, b, lo, lo_prec, scale, partials, nblk, stream));
+    } else {
+        if (t.variant != kDslashWaveSite) {
+            DslashArgs w = a;
+            w.tune = DslashTune{};
+            w.tune.variant = kDslashWaveSite;
+            t = dslash_resolve(w);
+        }
+        if (t.by <= 0 || t.bz <= 0 || t.spw <= 0 || a.g.L[1] % t.by || a.g.L[2] % t.bz) return hipErrorInvalidValue;
+        switch (lo_prec) {
+            case kSingle: QCU_HIP_TRY(launch_residual_lo_t<Cx<float>>(a, t, b, lo, scale, partials, nblk, stream)); break;
+            case kHalf: QCU_HIP_TRY(launch_residual_lo_t<Half2Store>(a, t, b, lo, scale, partials, nblk, stream)); break;
+            case kBF16: QCU_HIP_TRY(launch_residual_lo_t<Bf162Store>(a, t, b, lo, scale, partials, nblk, stream)); break;
+            default: return hipErrorInvalidValue;
+        }
     }
-    if (t.by <= 0 || t.bz <= 0 || t.spw <= 0 || a.g.L[1] % t.by || a.g.L[2] % t.bz) return hipErrorInvalidValue;
-    if ((long(div_up(a.g.Vh, 4 * t.spw)) + kResidualSlices) * a.R > partials_cap) return hipErrorInvalidValue;
-    switch (lo_prec) {
-        case kSingle: return launch_residual_lo_t<Cx<float>>(a, t, b, lo, scale, partials, nrm, stream);
-        case kHalf: return launch_residual_lo_t<Half2Store>(a, t, b, lo, scale, partials, nrm, stream);
-        case kBF16: return launch_residual_lo_t<Bf162Store>(a, t, b, lo, scale, partials, nrm, stream);
-        default: return hipErrorInvalidValue;
-    }
+    // partials [nblk][R] -> [kResidualSlices][R] (stored after them) -> nrm
+    double *p2 = partials + long(nblk) * a.R;
+    const int cols = a.R < 256 ? a.R : 256;
+    QCU_HIP_TRY(launch_rows_sum(p2, partials, nblk, a.R, kResidualSlices, stream));
+    hipLaunchKernelGGL(k_rows_sum, dim3(1, div_up(a.R, cols)), dim3(256), 0, stream, nrm,
+                       static_cast<const double *>(p2), kResidualSlices, a.R, kResidualSlices, true);
+    return hipGetLastError();
 }
 
 hipError_t launch_dslash_wave_groups(const DslashArgs &a, const SegTab &tab, int by, int bz, hipStream_t stream) {

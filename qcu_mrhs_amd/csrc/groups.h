@@ -57,10 +57,10 @@ public:
     // Allocates the batch buffers and picks each group's dslash shape (sites
     // per wavefront) by timing it on the inner precision; cached per precision.
     hipError_t autotune(const void *glo, int prec, hipStream_t s);
-    // dslash kernel the autotuner chose for the batch (2 = VALU wave-per-site, 3 = FP32 matrix cores per
-    // group, 5 = FP32 matrix cores over the groups' RHS packed into shared chunks)
+    // dslash kernel the autotuner chose for the batch (1 = lane per (site, RHS), 2 = VALU wave-per-site,
+    // 3 = FP32 matrix cores per group, 5 = FP32 matrix cores over the groups' RHS packed into shared chunks)
     int dslash_variant() const { return variant_; }
-    // and for the FP64 hops of the defect correction (2 = VALU, 3 / 5 = FP64 matrix cores; timed in solve)
+    // and for the FP64 hops of the defect correction (1 = lane, 2 = wave, 3 / 5 = FP64 matrix cores; timed in solve)
     int dslash_variant64() const { return variant64_; }
 
     // Solve M x = b for the batch held in b_full(); result in x_full().
@@ -74,6 +74,7 @@ private:
     hipError_t iteration(const void *glo, int P, double kappa, hipStream_t s);
     hipError_t tune64(const void *g64, hipStream_t s);
     SegTab tab_with(const int *done) const;
+    bool lane_supported(int prec) const;
 
     Geom g_;
     int Nc_;
@@ -81,7 +82,8 @@ private:
     long n_;
     SegTab tab_;
     int by_ = 0, bz_ = 0;
-    // group dslash kernel (autotuned): 2 = wave-per-site VALU, 3 = matrix cores per group, 5 = matrix cores
+    int lane_by_[2] = {0, 0}, lane_bz_[2] = {0, 0};  // traversal tiles of the lane kernel: inner precision, FP64
+    // group dslash kernel (autotuned): 1 = lane per (site, RHS), 2 = wave-per-site VALU, 3 = matrix cores per group, 5 = matrix cores
     // with the groups' RHS packed into shared 16-RHS chunks (sites per wavefront spw_packed_)
     int variant_ = 2;
     int spw_packed_ = 1;

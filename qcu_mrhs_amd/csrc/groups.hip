@@ -89,6 +89,9 @@ hipError_t GroupSolver::ensure(int prec) {
         const DslashTune t = dslash_resolve(a);
         by_ = t.by;
         bz_ = t.bz;
+        lane_by_[0] = lane_bz_[0] = lane_by_[1] = lane_bz_[1] = 0;
+        dslash_lane_tile(g_, Nc_, tab_.Rmax, prec, lane_by_[0], lane_bz_[0]);
+        dslash_lane_tile(g_, Nc_, tab_.Rmax, kDouble, lane_by_[1], lane_bz_[1]);
     }
     return hipSuccess;
 }
@@ -106,6 +109,8 @@ hipError_t GroupSolver::dslash(void *out, const void *in, const void *gauge, int
                                const void *xpay, double coef, const SegTab &tab, hipStream_t s) {
     DslashArgs a{out, in, gauge, xpay, coef, g_, Nc_, 0, parity, 0, prec};
     const int v = prec == kDouble ? variant64_ : variant_;
+    const int hi = prec == kDouble ? 1 : 0;
+    if (v == kDslashLaneRhs) return launch_dslash_lane_groups(a, tab, lane_by_[hi], lane_bz_[hi], s);
     if (v == kGroupsPacked && dslash_groups_matrix_supported(Nc_, prec))
         return launch_dslash_mfma32_packed(a, tab, by_, bz_, prec == kDouble ? spw_packed64_ : spw_packed_, s);
     if (v == kDslashMfma && dslash_groups_matrix_supported(Nc_, prec))
@@ -113,8 +118,10 @@ hipError_t GroupSolver::dslash(void *out, const void *in, const void *gauge, int
     return launch_dslash_wave_groups(a, tab, by_, bz_, s);
 }
 
-// FP64 hops of the defect correction: the whole batch's hop timed on the VALU wave kernel and on
-// the FP64 matrix cores (each group with its inner-precision shape), the faster one kept
+bool GroupSolver::lane_supported(int prec) const { return dslash_lane_supported(g_, Nc_, tab_.Rmax, prec); }
+
+// FP64 hops of the defect correction: the whole batch's hop timed on the wave kernel, on the FP64
+// matrix cores (each group with its inner-precision shape) and on the lane kernel, the fastest kept
 hipError_t GroupSolver::tune64(const void *g64, hipStream_t s) {
     if (tuned64_) return hipSuccess;
     variant64_ = kDslashWaveSite;
@@ -132,8 +139,9 @@ hipError_t GroupSolver::tune64(const void *g64, hipStream_t s) {
     float best = 1e30f;
     int best_v = kDslashWaveSite;
     int best_spw = 1;
-    const std::pair<int, int> cands[] = {{kDslashWaveSite, 0}, {kDslashMfma, 0}, {kGroupsPacked, 1},
-                                         {kGroupsPacked, 2}, {kGroupsPacked, 4}};
+    std::vector<std::pair<int, int>> cands{{kDslashWaveSite, 0}, {kDslashMfma, 0}, {kGroupsPacked, 1},
+                                           {kGroupsPacked, 2}, {kGroupsPacked, 4}};
+    if (lane_supported(kDouble)) cands.push_back({kDslashLaneRhs, 0});
     for (const auto &c : cands) {
         variant64_ = c.first;
         if (c.second > 0) spw_packed64_ = c.second;
@@ -253,6 +261,25 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
                 best_variant = kGroupsPacked;
                 best_packed = spw;
             }
+        }
+    }
+    // a lane per (site, RHS): its launch shape follows from the group sizes
+    if (err == hipSuccess && lane_supported(prec)) {
+        for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = 0;
+        err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
+        const SegTab t = tab_with(done_);
+        variant_ = kDslashLaneRhs;
+        if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);  // warm-up
+        if (err == hipSuccess) err = hipEventRecord(e0, s);
+        for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
+            err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
+        if (err == hipSuccess) err = hipEventRecord(e1, s);
+        if (err == hipSuccess) err = hipEventSynchronize(e1);
+        float ms = 0.f;
+        if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
+        if (err == hipSuccess && ms < best_total) {
+            best_total = ms;
+            best_variant = kDslashLaneRhs;
         }
     }
     variant_ = best_variant;

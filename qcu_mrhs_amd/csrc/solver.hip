@@ -172,7 +172,7 @@ hipError_t BiCGStab::ensure(int prec) {
         alloc_prec_ = prec;
     }
     if ((prec == kHalf || prec == kBF16) && !dotp_) {
-        dotp_cap_ = dslash_omega_partials(g_, R_);
+        dotp_cap_ = dslash_omega_partials(g_, Nc_, R_);
         dotp_ = static_cast<double *>(dmalloc(sizeof(double) * size_t(dotp_cap_), err));
         if (err != hipSuccess) return err;
     }
@@ -181,7 +181,7 @@ hipError_t BiCGStab::ensure(int prec) {
         if (err != hipSuccess) return err;
     }
     if (prec >= 0 && prec != kDouble && !part_) {
-        part_cap_ = dslash_residual_partials(g_, R_);
+        part_cap_ = dslash_residual_partials(g_, Nc_, R_);
         part_ = static_cast<double *>(dmalloc(sizeof(double) * size_t(part_cap_), err));
         if (err != hipSuccess) return err;
     }

@@ -57,3 +57,31 @@ def test_lane_kernel_edges(prec, L, Nc, R):
 @pytest.mark.parametrize("Nc,R,dagger", [(3, 28, 0), (2, 46, 1)])
 def test_two_rhs_per_lane(Nc, R, dagger):
     _check((16, 16, 16, 32), Nc, R, S, 1, dagger, True, 950 + Nc)
+
+
+@pytest.mark.parametrize("inner", [H, B, S])
+@pytest.mark.parametrize("L,Nc,R", [((8, 8, 8, 8), 3, 16), ((12, 6, 10, 4), 2, 24), ((8, 6, 4, 20), 4, 20)])
+def test_mixed_solve_on_lane_kernels(inner, L, Nc, R):
+    """A reliable-update solve whose hops, fused omega (16 bits) and fused FP64
+    residual run on the lane kernel, with sites that do not fill the last
+    workgroup: the FP64 true residual through the oracle operator."""
+    kappa, tol = 0.12, 1e-10
+    gauge = fields.gauge_field(L, Nc, 970 + Nc, kind="smooth", eps=0.8)
+    b = fields.gaussian_sources(L, Nc, R, 980 + R)
+    api.initGridSize(L, Nc, R, D, inner)
+    d_g = api.DeviceArray.from_complex(gauge.reshape(-1))
+    api.loadQcuGauge(d_g, D)
+    api.getDslash(0, 1.0 / (2 * kappa) - 4.0)
+    bs = [api.DeviceArray.from_complex(b[r]) for r in range(R)]
+    xs = [api.DeviceArray(b[r].nbytes) for r in range(R)]
+    for r in range(R):
+        api.pushBackFermions(xs[r], bs[r])
+    info = api.qcuInvertEx(500, tol)
+    x = np.stack([xs[r].complex(b[r].size) for r in range(R)])
+    api.finalizeQcu()
+    bm = fields.to_mrhs(b, Nc)
+    res = bm - oracle.mat(fields.to_mrhs(x, Nc), gauge, L, Nc, R, kappa)
+    rel = (oracle.norm(res, R) / oracle.norm(bm, R)).max()
+    print("case lane solve", L, Nc, R, inner, info["iterations"], rel, flush=True)
+    assert info["converged"] and info["reliable_updates"] >= 1
+    assert rel <= 1.01 * tol and abs(info["true_rel_residual"] - rel) <= 0.01 * tol
