@@ -608,6 +608,10 @@ int reduce_blocks(long n, int R, int max_blocks) {
     const int per_block = (kReduceThreads / R) * R;
     const long N = n * R;
     long nb = (N + per_block * 8L - 1) / (per_block * 8L);  // >= 8 entries per lane
+    // fewer workgroups than compute units: down to one entry per lane, which costs the finishing kernel
+    // less than the serial trips cost here (the x / r update at 8^4, 4 RHS, FP64: 16.3 us with 48
+    // workgroups, 5 us with 256)
+    if (nb < 256) nb = std::min<long>(256, (N + per_block - 1) / per_block);
     if (nb > max_blocks) nb = max_blocks;
     if (nb < 1) nb = 1;
     return int(nb);

@@ -39,6 +39,9 @@ struct DslashArgs {
     int dagger;
     int prec;           // storage precision of out/in/gauge/xpay (Prec)
     DslashTune tune{};
+    // Sum the hops in the order of the wave-per-site kernel (16 bits: of the matrix-core kernel), bit for
+    // bit: for callers that see the rounding of this storage type in vectors of a wider one
+    bool keep_order = false;
 };
 
 bool dslash_supported(int Nc, int R);

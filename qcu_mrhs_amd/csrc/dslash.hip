@@ -235,6 +235,8 @@ namespace {
 // Kernel chosen for a hop that names none.
 int automatic_variant(const DslashArgs &a) {
     const bool lane = dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
+    if (a.keep_order && a.prec != kSingle) return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
+    if (a.keep_order && a.Nc == 8) return kDslashWaveSite;
     if (a.prec == kSingle || a.prec == kDouble) {
         // Nc = 8 fills the 16 x 16 matrix-core tile (16^4, 16 RHS: FP64 265 us against 1035 us wave per
         // site, FP32 147 against 311 us); Nc <= 4 runs a lane per (site, RHS), faster than the
@@ -245,11 +247,10 @@ int automatic_variant(const DslashArgs &a) {
     // 16 bits: a lane per (site, RHS) where a row of right-hand sides is a whole number of 16-byte
     // pieces (24^3 x 48, SU(3) FP16: 103 against 179 us matrix cores at 8 RHS, 188 / 207 at 12,
     // 213 / 245 at 16, 374 / 759 at 32) or needs a second 16-wide matrix-core chunk (370 / 536 at 17);
-    // otherwise its loads straddle those pieces (190 / 175 at 6, 220 / 191 at 10), and below about
-    // 32768 lanes the matrix-core kernel's shorter chain of loads wins (8^3 x 16, 4 RHS: 8.1 / 6.7 us)
+    // otherwise its loads straddle those pieces (190 / 175 at 6, 220 / 191 at 10)
     const bool fits16 = double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 &&
                         double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;  // what the matrix-core kernel addresses
-    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16) && double(a.g.Vh) * a.R >= 32768.0) return kDslashLaneRhs;
+    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16)) return kDslashLaneRhs;
     return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
 }
 }  // namespace
@@ -327,7 +328,14 @@ hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, 
     if (!dslash_supported(a.Nc, a.R) || a.g.Vh <= 0 || (a.prec != kHalf && a.prec != kBF16) || a.dagger ||
         !a.xpay || !partials || !st || a.R > kReduceThreads)
         return hipErrorNotSupported;
-    const DslashTune t = dslash_resolve(a);
+    DslashTune t = dslash_resolve(a);
+    // below 32768 lanes the lane kernel's chain of eight hops is longer than the matrix-core kernel's
+    // one round of loads (8^3 x 16, 4 RHS: 8.1 against 6.7 us)
+    if (t.variant == kDslashLaneRhs && double(a.g.Vh) * a.R < 32768.0 && dslash_mfma_supported(a.Nc, a.prec)) {
+        t = DslashTune{};
+        t.variant = kDslashMfma;
+        t = dslash_fill_defaults(a, t);
+    }
     const bool lane = t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
     if (!lane && t.variant != kDslashMfma) return hipErrorNotSupported;
     if (cap < dslash_omega_partials(a.g, a.Nc, a.R)) return hipErrorInvalidValue;

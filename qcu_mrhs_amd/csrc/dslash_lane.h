@@ -157,24 +157,29 @@ __device__ __forceinline__ void pin(Cx<T> (&acc)[4][NC][V]) {
             for (int v = 0; v < V; ++v) asm volatile("" : "+v"(acc[s][c][v].re), "+v"(acc[s][c][v].im));
 }
 
+// the 4 NC entries of one neighbour spinor
+template <typename C, int NC, int V>
+__device__ __forceinline__ void load_spinor(Vec<C, V> (&w)[4][NC], __amdgpu_buffer_rsrc_t r_in, unsigned vo,
+                                            unsigned row_bytes) {
+    using R = Raw<V * int(sizeof(C))>;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            w[s][c] = __builtin_bit_cast(Vec<C, V>, R::load(r_in, vo, unsigned(s * NC + c) * row_bytes));
+}
+
+// acc += (1 -+ gamma) V w for one hop
 template <typename S, int NC, int V, bool DAG, int MU, bool FWD>
-__device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], __amdgpu_buffer_rsrc_t r_in,
-                                    unsigned vo, unsigned row_bytes, const typename Arith<S>::Link *U) {
+__device__ __forceinline__ void hop_arith(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
+                                          const Vec<typename Arith<S>::C, V> (&w)[4][NC],
+                                          const typename Arith<S>::Link *U) {
     using A = Arith<S>;
     using T = typename A::T;
-    using C = typename A::C;
-    using R = Raw<V * int(sizeof(C))>;
-    using W = Vec<C, V>;
     constexpr int sgn = (FWD != DAG) ? 2 : 0;
     constexpr int m0 = kMat2(MU, 0), m1 = kMat2(MU, 1);
     constexpr int kp0 = kProjK(MU, 0) + sgn, kp1 = kProjK(MU, 1) + sgn;
     constexpr int kr0 = kReconK(MU, 0) + sgn, kr1 = kReconK(MU, 1) + sgn;
-    asm volatile("" : "+v"(vo));  // the loads stay behind the previous hop's arithmetic (see pin)
-    W w[4][NC];
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) w[s][c] = __builtin_bit_cast(W, R::load(r_in, vo, unsigned(s * NC + c) * row_bytes));
     typename A::H h0[NC][V], h1[NC][V];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -205,7 +210,16 @@ __device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], _
             acc[m1][a][v] = acc[m1][a][v] + ipow<kr1>(s1[v]);
         }
     }
-    pin<T, NC, V>(acc);
+}
+
+template <typename S, int NC, int V, bool DAG, int MU, bool FWD>
+__device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], __amdgpu_buffer_rsrc_t r_in,
+                                    unsigned vo, unsigned row_bytes, const typename Arith<S>::Link *U) {
+    asm volatile("" : "+v"(vo));  // the loads stay behind the previous hop's arithmetic (see pin)
+    Vec<typename Arith<S>::C, V> w[4][NC];
+    load_spinor<typename Arith<S>::C, NC, V>(w, r_in, vo, row_bytes);
+    hop_arith<S, NC, V, DAG, MU, FWD>(acc, w, U);
+    pin<typename Arith<S>::T, NC, V>(acc);
     __builtin_amdgcn_sched_barrier(0);
 }
 
@@ -219,7 +233,9 @@ struct Place {
 };
 
 // acc = D in for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes per site.
-template <typename S, int NC, int V, bool DAG>
+// ORD: the hops of each direction are summed apart and then as ((x + z) + (y + t)), the wave-per-site
+// kernel's order (four sets of accumulators), instead of one after the other.
+template <typename S, int NC, int V, bool DAG, bool ORD = false>
 __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
                                       const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
                                       int R, int RV, int spb, int pos0, int parity, const int *walk,
@@ -255,20 +271,24 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     const auto r_in = rsrc(in, vec_bytes);
     const int *row = sw + l * 9;
     const typename A::Link *U = sl + l * LR;
+    constexpr int NA = ORD ? 4 : 1;
+    Cx<T> sums[NA][4][NC][V];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int m = 0; m < NA; ++m)
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
-            for (int v = 0; v < V; ++v) acc[s][c][v] = {T(0), T(0)};
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int v = 0; v < V; ++v) sums[m][s][c][v] = {T(0), T(0)};
     // Hop order t-, z-, y-, x-, x+, y+, z+, t+: the traversal sweeps upwards, so the backward neighbours
     // are the input sites about to leave the XCD's L2 and are read before the forward ones push them out
     // (24^3 x 48, 16 RHS: FP64 711 -> 636 us, FP32 350 -> 323 us against x+, x-, ..., t+, t-; 786 and
     // 393 us in the reverse order; 16^3 x 32, 12 RHS, FP64: 103 -> 79 us).
 #define QCU_BACK(MU) \
-    hop<S, NC, V, DAG, MU, false>(acc, r_in, unsigned(row[2 + 2 * MU]) * sb + lo, rb, U + (2 * MU + 1) * NN);
+    hop<S, NC, V, DAG, MU, false>(sums[ORD ? MU : 0], r_in, unsigned(row[2 + 2 * MU]) * sb + lo, rb, U + (2 * MU + 1) * NN);
 #define QCU_FORW(MU) \
-    hop<S, NC, V, DAG, MU, true>(acc, r_in, unsigned(row[1 + 2 * MU]) * sb + lo, rb, U + (2 * MU) * NN);
+    hop<S, NC, V, DAG, MU, true>(sums[ORD ? MU : 0], r_in, unsigned(row[1 + 2 * MU]) * sb + lo, rb, U + (2 * MU) * NN);
     QCU_BACK(3)
     QCU_BACK(2)
     QCU_BACK(1)
@@ -279,6 +299,17 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     QCU_FORW(3)
 #undef QCU_BACK
 #undef QCU_FORW
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                if constexpr (ORD)
+                    acc[s][c][v] = (sums[0][s][c][v] + sums[2][s][c][v]) + (sums[1][s][c][v] + sums[3][s][c][v]);
+                else
+                    acc[s][c][v] = sums[0][s][c][v];
+            }
     p.site = row[0];
     p.vo = unsigned(p.site) * sb + lo;
     return p;

@@ -73,15 +73,103 @@ __device__ __forceinline__ void store_lane(const Cx<typename Arith<S>::T> (&acc)
 }
 
 // out = coef D in (+ xpay)
-template <typename S, int NC, int V, bool DAG>
-__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane(
+template <typename S, int NC, int V, bool DAG, bool ORD = false>
+__global__ __launch_bounds__(256, ORD ? 2 : (kMinWaves<S, NC, V>)) void k_dslash_lane(
     typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
     const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
     int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
     Cx<typename Arith<S>::T> acc[4][NC][V];
-    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
-                                        xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
+    const Place p = hops<S, NC, V, DAG, ORD>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
+                                             xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
     if (p.active) store_lane<S, NC, V>(acc, out, xpay, coef, p, R, vec_bytes);
+}
+
+// Small lattices: the two hops of each direction in a wavefront of their own, the four wavefronts' sums
+// combined through LDS (wavefront mu finishes spin mu).  A lane then waits for two dependent loads (its
+// walk row, then links and both spinors together) instead of ten, and a lattice that would leave most
+// SIMDs without a wavefront has four times as many.
+template <typename S, int NC, bool DAG, int MU>
+__device__ __forceinline__ void direction(Cx<typename Arith<S>::T> (&acc)[4][NC][1], const typename Arith<S>::C *in,
+                                          const typename Arith<S>::C *gauge, int Vh, unsigned rb, unsigned lo,
+                                          int parity, const int *row, unsigned vec_bytes) {
+    using A = Arith<S>;
+    using C = typename A::C;
+    constexpr int NN = NC * NC;
+    const int site = row[0], nf = row[1 + 2 * MU], nb = row[2 + 2 * MU];
+    const unsigned sb = 4u * NC * rb;
+    const auto r_in = rsrc(in, vec_bytes);
+    Vec<C, 1> wf[4][NC], wb[4][NC];
+    load_spinor<C, NC, 1>(wb, r_in, unsigned(nb) * sb + lo, rb);
+    load_spinor<C, NC, 1>(wf, r_in, unsigned(nf) * sb + lo, rb);
+    const C *gf = gauge + ((MU * 2 + parity) * long(Vh) + site) * NN, *gb = gauge + ((MU * 2 + 1 - parity) * long(Vh) + nb) * NN;
+    typename A::Link uf[NN], ub[NN];
+#pragma unroll
+    for (int a = 0; a < NC; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b) {
+            ub[a * NC + b] = A::link(gb[b * NC + a], false);
+            uf[a * NC + b] = A::link(gf[a * NC + b], true);
+        }
+    hop_arith<S, NC, 1, DAG, MU, false>(acc, wb, ub);
+    hop_arith<S, NC, 1, DAG, MU, true>(acc, wf, uf);
+}
+
+template <typename S, int NC, bool DAG>
+__global__ __launch_bounds__(256) void k_dslash_lane_split(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
+    int R, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
+    using T = typename Arith<S>::T;
+    using C = typename Arith<S>::C;
+    using RW = Raw<int(sizeof(C))>;
+    auto *part = reinterpret_cast<Cx<T> *>(lane_smem);  // [spin][wavefront][colour][lane]
+    const int lane = threadIdx.x & 63;
+    const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pos0 = xcd_remap(blockIdx.x, gridDim.x) * spb;
+    const int ns = min(spb, Vh - pos0);
+    const int local = lane / R, r = lane - local * R;
+    const int *row = walk + (long(parity) * Vh + pos0 + min(local, ns - 1)) * 9;
+    const unsigned rb = unsigned(R) * unsigned(sizeof(C)), lo = unsigned(r) * unsigned(sizeof(C));
+    Cx<T> acc[4][NC][1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[s][c][0] = {T(0), T(0)};
+    if (mu == 0) direction<S, NC, DAG, 0>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
+    else if (mu == 1) direction<S, NC, DAG, 1>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
+    else if (mu == 2) direction<S, NC, DAG, 2>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
+    else direction<S, NC, DAG, 3>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) part[((s * 4 + mu) * NC + c) * 64 + lane] = acc[s][c][0];
+    const bool active = local < ns;
+    const unsigned vo = unsigned(row[0]) * 4u * NC * rb + unsigned(mu) * NC * rb + lo;
+    C xw[NC];
+    if (xpay) {
+        const auto r_x = rsrc(xpay, vec_bytes);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) xw[c] = __builtin_bit_cast(C, RW::load(r_x, vo, unsigned(c) * rb));
+    }
+    __syncthreads();
+    if (!active) return;
+    const auto r_out = rsrc(out, vec_bytes);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const Cx<T> *q = part + (mu * 4 * NC + c) * 64 + lane;
+        Cx<T> v = (q[0] + q[2 * NC * 64]) + (q[NC * 64] + q[3 * NC * 64]);  // the wave-per-site kernel's order
+        if (xpay) {
+            Cx<T> x = load_cx<T>(&xw[c]);
+            x.re = fma(coef, v.re, x.re);
+            x.im = fma(coef, v.im, x.im);
+            v = x;
+        } else {
+            v = coef * v;
+        }
+        C o;
+        store_cx(&o, v);
+        RW::store(r_out, __builtin_bit_cast(typename RW::type, o), vo, unsigned(c) * rb);
+    }
 }
 
 // Sums `n` values per lane over the workgroup's sites, per RHS, in site order: row[rv] for the first RV lanes.
@@ -321,23 +409,52 @@ hipError_t launch_groups_s(const DslashArgs &a, const SegTab &seg, int by, int b
     }
 }
 
-template <typename S, int NC, int V, bool DAG>
+template <typename S, int NC, int V, bool DAG, bool ORD = false>
 hipError_t launch_v(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
     using C = typename Arith<S>::C;
     GeomTables tab;
     QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
     const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, V);
     const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
-    hipLaunchKernelGGL((k_dslash_lane<S, NC, V, DAG>), dim3(div_up(a.g.Vh, sh.spb)), dim3(sh.threads), sh.lds, stream,
+    hipLaunchKernelGGL((k_dslash_lane<S, NC, V, DAG, ORD>), dim3(div_up(a.g.Vh, sh.spb)), dim3(sh.threads), sh.lds, stream,
                        static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
                        static_cast<const C *>(a.xpay), typename Arith<S>::T(a.coef), a.g.Vh, a.R, sh.RV, sh.spb,
                        a.parity, tab.walk, vec_bytes);
     return hipGetLastError();
 }
 
+// Four wavefronts per (site, RHS) pay while the lattice holds fewer lanes than four wavefronts per SIMD
+// (65536; 8^4, 4 RHS, FP64: 9.0 -> 5.6 us, 8^3 x 16, 16 RHS, FP16: 7.0 -> 5.5 us; at 98304 lanes 14.8 ->
+// 15.9 us), twice that for up to 4 RHS, whose links few lanes share (16^4, 4 RHS, FP32: 19.4 -> 15.6 us),
+// and with no more than a quarter of a wavefront's lanes idle.
+bool split_over_directions(const Geom &g, int R) {
+    if (R > 64 || (64 / R) * R < 48) return false;
+    return double(g.Vh) * R <= (R <= 4 ? 131072.0 : 65536.0);
+}
+
+template <typename S, int NC>
+hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
+    const int spb = 64 / a.R;
+    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
+    auto k = a.dagger ? k_dslash_lane_split<S, NC, true> : k_dslash_lane_split<S, NC, false>;
+    hipLaunchKernelGGL(k, dim3(div_up(a.g.Vh, spb)), dim3(256), size_t(16) * NC * 64 * sizeof(Cx<typename Arith<S>::T>),
+                       stream, static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.xpay), typename Arith<S>::T(a.coef), a.g.Vh, a.R, spb, a.parity,
+                       tab.walk, vec_bytes);
+    return hipGetLastError();
+}
+
 template <typename S, int NC>
 hipError_t launch_nc(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
     using C = typename Arith<S>::C;
+    if (split_over_directions(a.g, a.R)) return launch_split<S, NC>(a, t, stream);
+    if constexpr (std::is_same<S, float>::value)
+        if (a.keep_order)
+            return a.dagger ? launch_v<S, NC, 1, true, true>(a, t, stream)
+                            : launch_v<S, NC, 1, false, true>(a, t, stream);
     // FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
     // the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
     // 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache

@@ -327,6 +327,7 @@ void start_dslash(int parity, int daggerFlag) {
     bool ok = hip_ok(launch_gather(c->bufA, P, table(c->q_in, 0, c->user_prec), c->user_prec, n, c->R,
                                    c->stream), "gather");
     DslashArgs a{c->bufB, c->bufA, c->gauge(P), nullptr, 1.0, c->g, c->Nc, c->R, parity, daggerFlag ? 1 : 0, P};
+    a.keep_order = prec_bytes(P) < prec_bytes(c->user_prec);
     ok = ok && a.gauge && hip_ok(launch_dslash(a, c->stream), "dslash");
     ok = ok && hip_ok(launch_scatter(table(c->q_out, 0, c->user_prec), c->user_prec, c->bufB, P, n, c->R,
                                      c->stream), "scatter");
@@ -347,12 +348,14 @@ void mat_Qcu(int daggerFlag) {
     bool ok = hip_ok(launch_gather(A, P, table(c->q_in, 0, c->user_prec), c->user_prec, 2 * n, c->R,
                                    c->stream), "gather");
     ok = ok && ensure_clover(c);
+    const bool keep = prec_bytes(P) < prec_bytes(c->user_prec);
     for (int p = 0; p < 2 && ok; ++p) {
         char *in_p = A + p * n * c->R * eb, *out_p = B + p * n * c->R * eb;
         if (c->clover) {
             // out_p = A_pp in_p - kappa D_p in_{1-p}  (A Hermitian: the dagger reaches D only)
             DslashArgs a{out_p, A + (1 - p) * n * c->R * eb, c->gauge(P), nullptr, 1.0, c->g, c->Nc, c->R, p,
                          daggerFlag ? 1 : 0, P};
+            a.keep_order = keep;
             ok = a.gauge && hip_ok(launch_dslash(a, c->stream), "dslash");
             ok = ok && hip_ok(launch_clover_apply(out_p, in_p, c->clover_set.term(P, p), out_p, -c->kappa, c->g.Vh,
                                                   c->Nc, c->R, P, CloverSet::storage(P), c->stream),
@@ -362,6 +365,7 @@ void mat_Qcu(int daggerFlag) {
         // out_p = in_p - kappa D_p in_{1-p}   (src/qcu_interface.cu:174-255)
         DslashArgs a{out_p, A + (1 - p) * n * c->R * eb, c->gauge(P), in_p,
                      -c->kappa, c->g, c->Nc, c->R, p, daggerFlag ? 1 : 0, P};
+        a.keep_order = keep;
         ok = a.gauge && hip_ok(launch_dslash(a, c->stream), "dslash");
     }
     ok = ok && hip_ok(launch_scatter(table(c->q_out, 0, c->user_prec), c->user_prec, B, P, 2 * n, c->R,

@@ -1,5 +1,6 @@
 """GPU parity of the lane-per-(site, RHS) hopping kernel at the edges of its
-launch shape: right-hand sides that fill no wavefront, one lane per site and
+launch shapes (eight hops per lane, and the directions split over four
+wavefronts on small lattices): right-hand sides that fill no wavefront, one lane per site and
 more lanes than a wavefront per site, sites that do not fill the last
 workgroup, lattices of a single workgroup, and the form with two right-hand
 sides per lane (fields beyond 256 MiB in FP32); xpay and the dagger on the
@@ -48,7 +49,8 @@ def _check(L, Nc, R, prec, parity, dagger, xpay, seed):
 @pytest.mark.parametrize("prec", [D, S, H, B])
 @pytest.mark.parametrize("L,Nc,R", [((2, 2, 2, 2), 3, 1), ((4, 2, 6, 4), 3, 5), ((6, 4, 2, 10), 2, 17),
                                     ((4, 6, 4, 6), 4, 33), ((6, 6, 4, 4), 3, 70), ((4, 4, 4, 2), 4, 130),
-                                    ((14, 6, 10, 6), 3, 3), ((8, 12, 8, 16), 3, 12), ((12, 6, 6, 8), 4, 1)])
+                                    ((14, 6, 10, 6), 3, 3), ((8, 12, 8, 16), 3, 12), ((12, 6, 6, 8), 4, 1),
+                                    ((4, 4, 4, 8), 2, 64), ((18, 16, 12, 22), 3, 5), ((24, 14, 18, 24), 2, 1)])
 def test_lane_kernel_edges(prec, L, Nc, R):
     for k, (parity, dagger, xpay) in enumerate([(0, 0, False), (1, 1, True)]):
         _check(L, Nc, R, prec, parity, dagger, xpay, 900 + 7 * R + k)
@@ -85,3 +87,31 @@ def test_mixed_solve_on_lane_kernels(inner, L, Nc, R):
     print("case lane solve", L, Nc, R, inner, info["iterations"], rel, flush=True)
     assert info["converged"] and info["reliable_updates"] >= 1
     assert rel <= 1.01 * tol and abs(info["true_rel_residual"] - rel) <= 0.01 * tol
+
+
+@pytest.mark.parametrize("L,Nc,R,inner", [((8, 8, 8, 8), 3, 4, S), ((16, 12, 16, 20), 2, 24, S), ((12, 10, 14, 6), 4, 7, S),
+                                          ((8, 6, 4, 4), 3, 16, H), ((8, 6, 4, 4), 3, 16, B)])
+def test_operator_on_wider_vectors_keeps_its_rounding(L, Nc, R, inner):
+    """start_dslash on double-precision vectors in a lower precision sums the
+    hops in the order of the wave-per-site (16 bits: matrix-core) kernel: the
+    same bits as that kernel chosen explicitly."""
+    gauge = fields.gauge_field(L, Nc, 990 + Nc, kind="smooth", eps=0.8)
+    half = fields.half_volume(L) * 4 * Nc
+    g = fields.rng(991)
+    b = g.standard_normal((R, half)) + 1j * g.standard_normal((R, half))
+    api.initGridSize(L, Nc, R, D, inner)
+    d_g = api.DeviceArray.from_complex(gauge.reshape(-1))
+    api.loadQcuGauge(d_g, D)
+    api.getDslash(0, 0.1)
+    bs = [api.DeviceArray.from_complex(v) for v in b]
+    got = []
+    for variant in ("auto", "wave" if inner == S else "mfma"):
+        xs = [api.DeviceArray(16 * half) for _ in range(R)]
+        api.dslash_tune(variant)
+        for r in range(R):
+            api.pushBackFermions(xs[r], bs[r])
+        api.start_dslash(1, 0)
+        got.append(np.stack([x.complex(half) for x in xs]))
+    api.finalizeQcu()
+    print("case lane order", L, Nc, R, inner, flush=True)
+    np.testing.assert_array_equal(got[0], got[1])
