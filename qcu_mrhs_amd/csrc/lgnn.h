@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "blas.h"
+#include "geom.h"
 #include "solver.h"
 
 namespace qcu {
@@ -40,6 +41,15 @@ constexpr size_t kLgnnFragBytes = 8 * 64 * 16;  // MFMA fragments of M stored af
 hipError_t launch_lgnn_mfma(void *out, const void *in, const void *gauge, void *q, const Cx<float> *mcol,
                             const int *walk, const Geom &g, int Nc, int R, int prec, bool projected,
                             hipStream_t s);
+
+// FP32 kernels on matrix cores (lgnn_stencil.hip); `walk`: the even sites' walk table, gauge and stencil
+// (mcol) FP32.  mix32: q_k(y) = sum_k' M[k][k'] (T_k' in)(y) on the even sites, q 8 FP32 half vectors back
+// to back.  gram: partial sums of dL/dM* = sum (T_{k^1} dphi) conj(T_k' w)^T, `blocks` <= max_blocks rows
+// of 1040 FP64 entries (the first 1024 written).
+hipError_t launch_lgnn_mix32(void *q, const void *in, int prec, const void *gauge, const Cx<float> *mcol,
+                             const int *walk, const Geom &g, int Nc, int R, hipStream_t s);
+hipError_t launch_lgnn_gram(Cx<double> *part, int max_blocks, int &blocks, const void *dphi, const void *w,
+                            const void *gauge, const int *walk, const Geom &g, int Nc, int R, hipStream_t s);
 
 class LgnnPreconditioner : public Preconditioner {
 public:
@@ -95,13 +105,12 @@ private:
     hipError_t apply_mfma(void *out, const void *in, int prec, hipStream_t s);
     hipError_t collapse(hipStream_t s);
     hipError_t project_w2(hipStream_t s);  // W2[o][h] = P_h W2[o][h], h = 1..8
-    // stencil: collapsed stencil to apply (default the network's); hops: where the 8 hop
-    // fields of the input go (default the work field u_)
+    // stencil: collapsed stencil to apply (default the network's)
     hipError_t forward(const void *in, int prec, void *out, int out_prec, hipStream_t s,
-                       const Cx<float> *stencil = nullptr, void *hops = nullptr);
-    // gradient of a loss whose derivative with respect to the network output N w is dphi
-    // (FP32 odd field w; hops = the 8 hop fields forward(w) produced, default u_)
-    hipError_t accumulate_grad(const void *w, const void *dphi, hipStream_t s, const void *hops = nullptr);
+                       const Cx<float> *stencil = nullptr);
+    // gradient of a loss whose derivative with respect to the network output N w is dphi (FP32 odd fields)
+    hipError_t accumulate_grad(const void *w, const void *dphi, hipStream_t s);
+    hipError_t tables(GeomTables &tab, hipStream_t s) const;  // walk table in the FP32 hop's traversal order
     // FP32 odd Schur operator with the FP32 gauge copy: out = A in (dagger: A^+)
     hipError_t schur32(void *out, const void *in, double kappa, int dagger, hipStream_t s);
     hipError_t ensure_power(int K, hipStream_t s);
@@ -124,11 +133,11 @@ private:
     Cx<float> *madj_ = nullptr;                  // the stencil of N^+ (same layout)
     // residual-power objective work fields (FP32 odd half vectors): w_0..w_K, g, A^+ g, N^+ A^+ g,
     // the dslash intermediate on the even sites, and per-RHS scale factors
-    std::vector<void *> pw_, phops_;
+    std::vector<void *> pw_;
     void *pg_ = nullptr, *pu_ = nullptr, *pn_ = nullptr, *ptmp_ = nullptr;
     double *pscale_ = nullptr;
-    // work fields (FP32): u[8] hop fields on even sites, q[8], odd scratch
-    void *u_ = nullptr, *q_ = nullptr, *inf_ = nullptr, *phi_ = nullptr, *dlt_ = nullptr;
+    // work fields (FP32): q[8] on the even sites, odd scratch
+    void *q_ = nullptr, *inf_ = nullptr, *phi_ = nullptr, *dlt_ = nullptr;
     C64 *gm_ = nullptr;                          // dL/dM* partials [nblk][32*32 + 16]
     int gram_blocks_ = 0;
     double *dnorm_ = nullptr, *dloss_ = nullptr, *hbuf_ = nullptr;

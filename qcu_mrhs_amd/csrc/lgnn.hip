@@ -17,74 +17,6 @@ namespace {
 
 using C32 = Cx<float>;
 
-// out_k(y) = V_k(y) in(nb_k(y)) for every site y of parity `pout` and hop k;
-// V = U_mu(y) forward, U_mu(y - mu)^+ backward (link on the neighbour parity).
-template <typename CS, int NC>
-__global__ __launch_bounds__(256) void k_transport8(C32 *__restrict__ out, const CS *__restrict__ in,
-                                                   const C32 *__restrict__ gauge, const int *__restrict__ nbr,
-                                                   int Vh, int R, int pout) {
-    const int site = blockIdx.x * blockDim.y + threadIdx.y;
-    if (site >= Vh) return;
-    const int r = threadIdx.x;
-    const long sl = 4L * NC * R;
-    const long fsize = long(Vh) * sl;
-    const int *nrow = nbr + (long(pout) * Vh + site) * 8;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int mu = k >> 1;
-        const bool fwd = (k & 1) == 0;
-        const int nb = nrow[k];
-        const C32 *U = fwd ? gauge + ((long(mu) * 2 + pout) * Vh + site) * NC * NC
-                           : gauge + ((long(mu) * 2 + 1 - pout) * Vh + nb) * NC * NC;
-        const CS *src = in + nb * sl + r;
-        C32 *dst = out + k * fsize + site * sl + r;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            C32 v[NC];
-#pragma unroll
-            for (int b = 0; b < NC; ++b) v[b] = load_cx<float>(src + (s * NC + b) * R);
-#pragma unroll
-            for (int a = 0; a < NC; ++a) {
-                C32 acc = {0.f, 0.f};
-#pragma unroll
-                for (int b = 0; b < NC; ++b) {
-                    if (fwd) cfma(acc, U[a * NC + b], v[b]);
-                    else cfma_conj(acc, U[b * NC + a], v[b]);
-                }
-                dst[(s * NC + a) * R] = acc;
-            }
-        }
-    }
-}
-
-// q[(k,s)] = sum_{(k',s')} M[(k,s)][(k',s')] u[(k',s')] per (even site, colour, rhs)
-__global__ __launch_bounds__(256) void k_mix(C32 *__restrict__ q, const C32 *__restrict__ u,
-                                            const C32 *__restrict__ mcol, long ncol, int Nc, int R, long fsize) {
-    __shared__ C32 M[32 * 32];
-    for (int i = threadIdx.x; i < 1024; i += blockDim.x) M[i] = mcol[i];
-    __syncthreads();
-    const long stride = long(gridDim.x) * blockDim.x;
-    for (long j = long(blockIdx.x) * blockDim.x + threadIdx.x; j < ncol; j += stride) {
-        // j enumerates (site, colour, rhs) with rhs fastest
-        const long r = j % R;
-        const long rest = j / R;
-        const long c = rest % Nc;
-        const long site = rest / Nc;
-        C32 x[32];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) x[k * 4 + s] = u[k * fsize + ((site * 4 + s) * Nc + c) * R + r];
-#pragma unroll 4
-        for (int i = 0; i < 32; ++i) {
-            C32 acc = {0.f, 0.f};
-#pragma unroll
-            for (int jj = 0; jj < 32; ++jj) cfma(acc, M[i * 32 + jj], x[jj]);
-            q[(i >> 2) * fsize + ((site * 4 + (i & 3)) * Nc + c) * R + r] = acc;
-        }
-    }
-}
-
 // out(x) = M0 in(x) + sum_k V_k(x) q_k(nb_k(x)) on the odd sites
 template <typename CS, typename CO, int NC>
 __global__ __launch_bounds__(256) void k_gather8(CO *__restrict__ out, const CS *__restrict__ in,
@@ -145,58 +77,6 @@ __global__ __launch_bounds__(256) void k_gather8(CO *__restrict__ out, const CS 
         for (int c = 0; c < NC; ++c) store_cx(o + (s * NC + c) * R, acc[s][c]);
 }
 
-// Partial sums of G[(k,s)][(k',s')] = sum_j a_{k^1}[s](j) conj(b_k'[s'](j)) over
-// columns j = (even site, colour, rhs); a = transported dL/dphi*, b = u.
-// Block partials in FP64; thread t owns entries 4t .. 4t+3.  Each block walks
-// a contiguous range of sites; per site the (colour, rhs) columns are one
-// contiguous run of Nc*R entries in every (field, spin) row.
-constexpr int kGramTile = 32;
-__global__ __launch_bounds__(256) void k_gram(C64 *__restrict__ part, const C32 *__restrict__ a,
-                                             const C32 *__restrict__ b, int Vh, int ncr, long fsize) {
-    __shared__ C32 sa[32][kGramTile];
-    __shared__ C32 sb[32][kGramTile];
-    const int t = threadIdx.x;
-    const int i = t >> 3;            // row (k, s)
-    const int j0 = (t & 7) * 4;      // first of 4 columns (k', s')
-    C64 acc[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-    const int per_block = (Vh + int(gridDim.x) - 1) / int(gridDim.x);
-    const int lo = per_block * int(blockIdx.x);
-    const int hi = lo + per_block < Vh ? lo + per_block : Vh;
-    for (int site = lo; site < hi; ++site) {
-        const long sbase = long(site) * 4 * ncr;
-        for (int cr0 = 0; cr0 < ncr; cr0 += kGramTile) {
-            // stage kGramTile columns of both 32-vectors
-            for (int e = t; e < 32 * kGramTile; e += blockDim.x) {
-                const int row = e / kGramTile, col = e % kGramTile;
-                const int cr = cr0 + col;
-                C32 va = {0.f, 0.f}, vb = {0.f, 0.f};
-                if (cr < ncr) {
-                    const int k = row >> 2, sp = row & 3;
-                    const long off = sbase + long(sp) * ncr + cr;
-                    va = a[(k ^ 1) * fsize + off];
-                    vb = b[k * fsize + off];
-                }
-                sa[row][col] = va;
-                sb[row][col] = vb;
-            }
-            __syncthreads();
-#pragma unroll 4
-            for (int col = 0; col < kGramTile; ++col) {
-                const C32 x = sa[i][col];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const C32 y = sb[j0 + q][col];
-                    acc[q].re += double(x.re) * y.re + double(x.im) * y.im;
-                    acc[q].im += double(x.im) * y.re - double(x.re) * y.im;
-                }
-            }
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) part[long(blockIdx.x) * 1040 + i * 32 + j0 + q] = acc[q];
-}
-
 // Partial sums of G0[s][t] = sum_j d[s](j) conj(p[t](j)) over odd-site columns.
 __global__ __launch_bounds__(256) void k_gram0(C64 *__restrict__ part, const C32 *__restrict__ d,
                                               const C32 *__restrict__ p, long ncol, int Nc, int R) {
@@ -242,10 +122,13 @@ __global__ __launch_bounds__(256) void k_gram0(C64 *__restrict__ part, const C32
 //   dL/dM* = G, dL/dW2[o][h]* = sum_h' G[h][h'] W1[o][h']^+, dL/dW1[o][h']* = sum_h W2[o][h]^+ G[h][h']
 // (h = 0 pairs with M0).  The stored gradient is 2 dL/dW* = dL/dRe W + i dL/dIm W,
 // accumulated over batches.
-// G[e] = sum over the block partials of entry e (fixed order: strided lanes, then a tree)
-__global__ __launch_bounds__(256) void k_sum_partials(C64 *__restrict__ G, const C64 *__restrict__ part, int nblk) {
+// G[e] = sum over the block partials of entry e (fixed order: strided lanes, then a tree); nblk_g
+// rows hold the 1024 entries of G, nblk_0 those of G0
+__global__ __launch_bounds__(256) void k_sum_partials(C64 *__restrict__ G, const C64 *__restrict__ part, int nblk_g,
+                                                     int nblk_0) {
     __shared__ double sr[256], si[256];
     const int e = blockIdx.x;
+    const int nblk = e < 1024 ? nblk_g : nblk_0;
     double ar = 0.0, ai = 0.0;
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
         ar += part[long(b) * 1040 + e].re;
@@ -264,13 +147,13 @@ __global__ __launch_bounds__(256) void k_sum_partials(C64 *__restrict__ G, const
     if (threadIdx.x == 0) G[e] = {sr[0], si[0]};
 }
 
-__global__ void k_chain(C64 *g1, C64 *g2, const C64 *w1, const C64 *w2, const C64 *Gsum, int C) {
-    __shared__ C64 G[1040];
-    for (int e = threadIdx.x; e < 1040; e += blockDim.x) G[e] = Gsum[e];
-    __syncthreads();
+// one wavefront per workgroup: the entries are independent and each is a chain of 64 products (one
+// workgroup for all 1152 entries of 8 channels took 67 us)
+__global__ __launch_bounds__(64) void k_chain(C64 *__restrict__ g1, C64 *__restrict__ g2, const C64 *__restrict__ w1,
+                                             const C64 *__restrict__ w2, const C64 *__restrict__ G, int C) {
     // entry (o, h, s, t) of W: flattened ((o * 9 + h) * 4 + s) * 4 + t
     const int total = C * 9 * 16;
-    for (int e = threadIdx.x; e < total; e += blockDim.x) {
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
         const int t = e & 3, s = (e >> 2) & 3, h = (e >> 4) % 9, o = e / 144;
         C64 a2 = {0.0, 0.0}, a1 = {0.0, 0.0};
         if (h == 0) {
@@ -449,13 +332,11 @@ LgnnPreconditioner::LgnnPreconditioner(const Geom &g, int Nc, int R, int channel
 
 LgnnPreconditioner::~LgnnPreconditioner() {
     for (void *p : {(void *)w1_, (void *)w2_, (void *)g1_, (void *)g2_, (void *)m1_, (void *)m2_, (void *)v1_,
-                    (void *)v2_, (void *)mcol_, (void *)madj_, u_, q_, inf_, phi_, dlt_, (void *)gm_, (void *)dnorm_,
+                    (void *)v2_, (void *)mcol_, (void *)madj_, q_, inf_, phi_, dlt_, (void *)gm_, (void *)dnorm_,
                     pg_, pu_, pn_, ptmp_, (void *)pscale_,
                     (void *)dloss_, gauge32_, q16_, glo_[0], glo_[1]})
         if (p) (void)hipFree(p);
     for (void *p : pw_)
-        if (p) (void)hipFree(p);
-    for (void *p : phops_)
         if (p) (void)hipFree(p);
     if (hbuf_) (void)hipHostFree(hbuf_);
     reduce_work_free(red_);
@@ -466,15 +347,14 @@ bool LgnnPreconditioner::supports(int prec) const {
 }
 
 hipError_t LgnnPreconditioner::ensure_work32(hipStream_t) {
-    if (u_) return hipSuccess;
+    if (q_) return hipSuccess;
     hipError_t err = hipSuccess;
     const size_t half32 = size_t(n_) * R_ * sizeof(C32);
-    u_ = dmal(8 * half32, err);
     q_ = dmal(8 * half32, err);
     inf_ = dmal(half32, err);
     phi_ = dmal(half32, err);
     dlt_ = dmal(half32, err);
-    gram_blocks_ = 512;
+    gram_blocks_ = 768;  // 3 workgroups per compute unit
     gm_ = static_cast<C64 *>(dmal(sizeof(C64) * 1040 * size_t(gram_blocks_ + 1), err));
     if (err != hipSuccess) set_error(5, "learned preconditioner: allocation failed (%s)", hipGetErrorString(err));
     return err;
@@ -559,34 +439,24 @@ hipError_t LgnnPreconditioner::collapse(hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t LgnnPreconditioner::tables(GeomTables &tab, hipStream_t s) const {
+    int by = 0, bz = 0;
+    dslash_lane_tile(g_, Nc_, R_, kSingle, by, bz);
+    return geom_tables(g_, by, bz, tab, s);
+}
+
 hipError_t LgnnPreconditioner::forward(const void *in, int prec, void *out, int out_prec, hipStream_t s,
-                                       const Cx<float> *stencil, void *hops) {
+                                       const Cx<float> *stencil) {
     const Cx<float> *mc = stencil ? stencil : mcol_;
     QCU_HIP_TRY(ensure_work32(s));
-    if (!in || !out || !u_ || !q_) return hipErrorInvalidValue;
+    if (!in || !out || !q_) return hipErrorInvalidValue;
     GeomTables tab;
-    QCU_HIP_TRY(geom_tables(g_, g_.L[1], g_.L[2], tab, s));
+    QCU_HIP_TRY(tables(tab, s));
     const int spb = R_ >= 256 ? 1 : 256 / R_;
     const dim3 block(R_, spb), grid(div_up(g_.Vh, spb));
-    const long fsize = n_ * R_;
-    C32 *u = static_cast<C32 *>(hops ? hops : u_), *q = static_cast<C32 *>(q_);
+    C32 *q = static_cast<C32 *>(q_);
     const C32 *g32 = static_cast<const C32 *>(gauge32_);
-    hipError_t e = dispatch_nc(Nc_, [&](auto ncv) -> hipError_t {
-        constexpr int NC = decltype(ncv)::value;
-        switch (prec) {
-            case kDouble: hipLaunchKernelGGL((k_transport8<Cx<double>, NC>), grid, block, 0, s, u, static_cast<const Cx<double> *>(in), g32, tab.nbr, g_.Vh, R_, 0); break;
-            case kSingle: hipLaunchKernelGGL((k_transport8<Cx<float>, NC>), grid, block, 0, s, u, static_cast<const Cx<float> *>(in), g32, tab.nbr, g_.Vh, R_, 0); break;
-            case kHalf: hipLaunchKernelGGL((k_transport8<Half2Store, NC>), grid, block, 0, s, u, static_cast<const Half2Store *>(in), g32, tab.nbr, g_.Vh, R_, 0); break;
-            case kBF16: hipLaunchKernelGGL((k_transport8<Bf162Store, NC>), grid, block, 0, s, u, static_cast<const Bf162Store *>(in), g32, tab.nbr, g_.Vh, R_, 0); break;
-            default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    });
-    if (e != hipSuccess) return e;
-    const long ncol = long(g_.Vh) * Nc_ * R_;
-    hipLaunchKernelGGL(k_mix, dim3(int(std::min<long>((ncol + 255) / 256, 8192))), dim3(256), 0, s, q, u, mc, ncol,
-                       Nc_, R_, fsize);
-    QCU_HIP_TRY(hipGetLastError());
+    QCU_HIP_TRY(launch_lgnn_mix32(q, in, prec, g32, mc, tab.walk, g_, Nc_, R_, s));
     const C32 *m0 = mc + 1024;
     return dispatch_nc(Nc_, [&](auto ncv) -> hipError_t {
         constexpr int NC = decltype(ncv)::value;
@@ -649,10 +519,10 @@ hipError_t LgnnPreconditioner::zero_grad(hipStream_t s) {
 hipError_t LgnnPreconditioner::loss_grad(const void *in, const void *target, double *loss_host, hipStream_t s) {
     if (!ready()) return hipErrorInvalidValue;
     QCU_HIP_TRY(ensure_fields(s));
-    // the FP32 work fields (phi_, dlt_, u_, q_, gm_) must exist before their pointers are passed on
+    // the FP32 work fields (phi_, dlt_, q_, gm_) must exist before their pointers are passed on
     QCU_HIP_TRY(ensure_work32(s));
     const long N = n_ * R_;
-    // forward in FP32 (keeps u for the gradient)
+    // forward in FP32
     QCU_HIP_TRY(forward(in, kSingle, phi_, kSingle, s));
     // per-RHS ||e||^2, then d = (phi - e) / ||e||^2 and loss = sum ||phi - e||^2 / ||e||^2
     QCU_HIP_TRY(launch_norm(dnorm_, target, n_, R_, kSingle, false, red_, 0, s));
@@ -675,23 +545,12 @@ hipError_t LgnnPreconditioner::loss_grad(const void *in, const void *target, dou
     return accumulate_grad(in, dlt_, s);
 }
 
-hipError_t LgnnPreconditioner::accumulate_grad(const void *w, const void *dphi, hipStream_t s, const void *hops) {
-    // a_k = T_k dphi on the even sites (the adjoint of hop k is hop k ^ 1), into q
+hipError_t LgnnPreconditioner::accumulate_grad(const void *w, const void *dphi, hipStream_t s) {
     GeomTables tab;
-    QCU_HIP_TRY(geom_tables(g_, g_.L[1], g_.L[2], tab, s));
-    const int spb = R_ >= 256 ? 1 : 256 / R_;
-    const dim3 block(R_, spb), grid(div_up(g_.Vh, spb));
-    QCU_HIP_TRY(dispatch_nc(Nc_, [&](auto ncv) -> hipError_t {
-        constexpr int NC = decltype(ncv)::value;
-        hipLaunchKernelGGL((k_transport8<Cx<float>, NC>), grid, block, 0, s, static_cast<C32 *>(q_),
-                           static_cast<const C32 *>(dphi), static_cast<const C32 *>(gauge32_), tab.nbr, g_.Vh, R_, 0);
-        return hipGetLastError();
-    }));
+    QCU_HIP_TRY(tables(tab, s));
     const long ncol = long(g_.Vh) * Nc_ * R_;
-    const long fsize = n_ * R_;
-    hipLaunchKernelGGL(k_gram, dim3(gram_blocks_), dim3(256), 0, s, gm_, static_cast<const C32 *>(q_),
-                       static_cast<const C32 *>(hops ? hops : u_), g_.Vh, Nc_ * R_, fsize);
-    QCU_HIP_TRY(hipGetLastError());
+    int gram_rows = 0;
+    QCU_HIP_TRY(launch_lgnn_gram(gm_, gram_blocks_, gram_rows, dphi, w, gauge32_, tab.walk, g_, Nc_, R_, s));
     // the input itself is needed in FP32 for the M0 gradient
     const C32 *inf = static_cast<const C32 *>(w);
     hipLaunchKernelGGL(k_gram0, dim3(gram_blocks_), dim3(256), 0, s, gm_, static_cast<const C32 *>(dphi), inf, ncol,
@@ -699,9 +558,9 @@ hipError_t LgnnPreconditioner::accumulate_grad(const void *w, const void *dphi, 
     QCU_HIP_TRY(hipGetLastError());
     // partial sums land after the per-block partials
     C64 *gsum = gm_ + 1040 * size_t(gram_blocks_);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1040), dim3(256), 0, s, gsum, gm_, gram_blocks_);
+    hipLaunchKernelGGL(k_sum_partials, dim3(1040), dim3(256), 0, s, gsum, gm_, gram_rows, gram_blocks_);
     QCU_HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_chain, dim3(1), dim3(256), 0, s, g1_, g2_, w1_, w2_, gsum, C_);
+    hipLaunchKernelGGL(k_chain, dim3(div_up(C_ * 144, 64)), dim3(64), 0, s, g1_, g2_, w1_, w2_, gsum, C_);
     return hipGetLastError();
 }
 
@@ -732,10 +591,6 @@ hipError_t LgnnPreconditioner::ensure_power(int K, hipStream_t s) {
     const size_t half32 = size_t(n_) * R_ * sizeof(C32);
     while (int(pw_.size()) < K + 1) {
         pw_.push_back(dmal(half32, err));
-        if (err != hipSuccess) return err;
-    }
-    while (int(phops_.size()) < K) {  // the 8 hop fields of each factor's input, kept for the gradient
-        phops_.push_back(dmal(8 * half32, err));
         if (err != hipSuccess) return err;
     }
     if (pg_) return hipSuccess;
@@ -773,7 +628,7 @@ hipError_t LgnnPreconditioner::power_loss_grad(const void *v, int K, double kapp
     QCU_HIP_TRY(launch_convert(pw_[0], kSingle, v, kSingle, N, pscale_, R_, s));
     // w_{j+1} = w_j - A N w_j
     for (int j = 0; j < K; ++j) {
-        QCU_HIP_TRY(forward(pw_[j], kSingle, phi_, kSingle, s, nullptr, phops_[j]));
+        QCU_HIP_TRY(forward(pw_[j], kSingle, phi_, kSingle, s));
         QCU_HIP_TRY(schur32(pu_, phi_, kappa, 0, s));
         AxpyArgs ax{kXsay, pw_[j + 1], pw_[j], pu_, nullptr, ones, nullptr, nullptr, n_, R_, kSingle};
         QCU_HIP_TRY(launch_axpy(ax, s));
@@ -792,7 +647,7 @@ hipError_t LgnnPreconditioner::power_loss_grad(const void *v, int K, double kapp
         QCU_HIP_TRY(schur32(pu_, pg_, kappa, 1, s));
         if (j > 0) QCU_HIP_TRY(forward(pu_, kSingle, pn_, kSingle, s, madj_));
         QCU_HIP_TRY(launch_convert(dlt_, kSingle, pu_, kSingle, N, pscale_ + R_, R_, s));
-        QCU_HIP_TRY(accumulate_grad(pw_[j], dlt_, s, phops_[j]));
+        QCU_HIP_TRY(accumulate_grad(pw_[j], dlt_, s));
         if (j > 0) {
             AxpyArgs ax{kXsay, pg_, pg_, pn_, nullptr, ones, nullptr, nullptr, n_, R_, kSingle};
             QCU_HIP_TRY(launch_axpy(ax, s));
