@@ -42,10 +42,17 @@ struct DslashArgs {
     // Sum the hops in the order of the wave-per-site kernel (16 bits: of the matrix-core kernel), bit for
     // bit: for callers that see the rounding of this storage type in vectors of a wider one
     bool keep_order = false;
+    // Clover blocks of the output parity (launch_dslash_clover, launch_dslash_omega and
+    // launch_dslash_residual_lo), FP64 for FP64 storage, else FP32
+    const void *clover = nullptr;
+    const void *clover_in = nullptr;  // what they are applied to (null: the result of the hop)
 };
 
 bool dslash_supported(int Nc, int R);
 hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream);
+// a.clover_in given: out = A clover_in + coef D in (xpay not read); else out = A (coef D in + xpay).
+// out may not alias in or clover_in
+hipError_t launch_dslash_clover(const DslashArgs &a, hipStream_t stream);
 
 // resolved launch shape (after defaults / tuning table)
 DslashTune dslash_resolve(const DslashArgs &a);
@@ -69,6 +76,8 @@ hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStrea
 bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
 void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
 // workgroups of a launch with one RHS per lane (rows of partial sums of the fused forms below); Nc <= 4
+// the clover forms of the lane kernel replace the separate clover pass for these arguments and shape
+bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t);
 int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec);
 hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
                                        const double *scale, double *partials, int &nblk, hipStream_t stream);

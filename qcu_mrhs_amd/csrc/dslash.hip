@@ -21,6 +21,7 @@
 #include <tuple>
 
 #include "blas.h"
+#include "clover.h"
 #include "dslash_common.h"
 
 namespace qcu {
@@ -315,6 +316,23 @@ hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
     }
 }
 
+hipError_t launch_dslash_clover(const DslashArgs &a, hipStream_t stream) {
+    if (!a.clover || !dslash_supported(a.Nc, a.R)) return hipErrorInvalidValue;
+    if (a.g.Vh <= 0) return hipSuccess;
+    const DslashTune t = dslash_resolve(a);
+    if (dslash_lane_clover_fused(a, t)) return launch_dslash_lane(a, t, stream);
+    DslashArgs h = a;
+    h.clover = h.clover_in = nullptr;
+    if (a.clover_in) {
+        h.xpay = nullptr;
+        h.coef = 1.0;
+    }
+    QCU_HIP_TRY(launch_dslash(h, stream));
+    return launch_clover_apply(a.out, a.clover_in ? a.clover_in : a.out, a.clover, a.clover_in ? a.out : nullptr,
+                               a.clover_in ? a.coef : 0.0, a.g.Vh, a.Nc, a.R, a.prec,
+                               a.prec == kDouble ? kDouble : kSingle, stream);
+}
+
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
 long dslash_omega_partials(const Geom &g, int Nc, int R) {
@@ -326,12 +344,13 @@ long dslash_omega_partials(const Geom &g, int Nc, int R) {
 
 hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, Cx<double> *st, hipStream_t stream) {
     if (!dslash_supported(a.Nc, a.R) || a.g.Vh <= 0 || (a.prec != kHalf && a.prec != kBF16) || a.dagger ||
-        !a.xpay || !partials || !st || a.R > kReduceThreads)
+        !(a.clover ? a.clover_in : a.xpay) || !partials || !st || a.R > kReduceThreads)
         return hipErrorNotSupported;
     DslashTune t = dslash_resolve(a);
+    if (a.clover && !dslash_lane_clover_fused(a, t)) return hipErrorNotSupported;
     // below 32768 lanes the lane kernel's chain of eight hops is longer than the matrix-core kernel's
     // one round of loads (8^3 x 16, 4 RHS: 8.1 against 6.7 us)
-    if (t.variant == kDslashLaneRhs && double(a.g.Vh) * a.R < 32768.0 && dslash_mfma_supported(a.Nc, a.prec)) {
+    if (t.variant == kDslashLaneRhs && !a.clover && double(a.g.Vh) * a.R < 32768.0 && dslash_mfma_supported(a.Nc, a.prec)) {
         t = DslashTune{};
         t.variant = kDslashMfma;
         t = dslash_fill_defaults(a, t);

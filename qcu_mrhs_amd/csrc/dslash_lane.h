@@ -223,6 +223,12 @@ __device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], _
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// What a workgroup loads into LDS besides its links, in the same wait: nothing, or (Clover, below) the
+// clover blocks of its sites.
+struct NoExtra {
+    __device__ __forceinline__ void load(const int *, int) const {}
+};
+
 // What a lane knows after the hops.
 struct Place {
     bool active;    // holds a site of the workgroup (idle lanes repeat the last one)
@@ -235,11 +241,11 @@ struct Place {
 // acc = D in for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes per site.
 // ORD: the hops of each direction are summed apart and then as ((x + z) + (y + t)), the wave-per-site
 // kernel's order (four sets of accumulators), instead of one after the other.
-template <typename S, int NC, int V, bool DAG, bool ORD = false>
+template <typename S, int NC, int V, bool DAG, bool ORD = false, typename X = NoExtra>
 __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
                                       const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
                                       int R, int RV, int spb, int pos0, int parity, const int *walk,
-                                      unsigned vec_bytes) {
+                                      unsigned vec_bytes, const X &extra = X{}) {
     using A = Arith<S>;
     using T = typename A::T;
     using C = typename A::C;
@@ -260,6 +266,7 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
                             : ((k >> 1) * 2 + 1 - parity) * long(Vh) + sw[l * 9 + 1 + k];
         sl[l * LR + k * NN + e] = A::link(gauge[li * NN + (fwd ? e : b * NC + a)], fwd);
     }
+    extra.load(sw, ns);
     __syncthreads();
     Place p;
     p.local = int(threadIdx.x) / RV;
@@ -314,6 +321,83 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     p.vo = unsigned(p.site) * sb + lo;
     return p;
 }
+
+// Clover blocks of a workgroup's sites: [site][chirality][2 NC][2 NC], complex in the accumulation type.
+// In LDS a row of kCloverRow entries per site (one more than it needs: banks, as the links).
+template <int NC>
+constexpr int kCloverRow = 8 * NC * NC + 1;
+
+template <typename S, int NC>
+struct Clover {
+    using T = typename Arith<S>::T;
+    const Cx<T> *blocks;  // of the output parity
+    Cx<T> *lds;
+
+    __device__ __forceinline__ void load(const int *sw, int ns) const {
+        constexpr int per = 8 * NC * NC;
+        for (int i = threadIdx.x; i < ns * per; i += blockDim.x) {
+            const int l = i / per, e = i - l * per;
+            lds[l * kCloverRow<NC> + e] = blocks[long(sw[l * 9]) * per + e];
+        }
+    }
+
+    // x given: rows of A x + coef acc (xpay not read); else rows of A (coef acc + xpay).
+    // emit(s, c, value[V], x_entry[V]) for every (spin, colour); x_entry is what the block was applied to
+    template <int V, typename F>
+    __device__ __forceinline__ void rows(const Cx<T> (&acc)[4][NC][V], const typename Arith<S>::C *x,
+                                         const typename Arith<S>::C *xpay, T coef, const Place &p, int ns,
+                                         unsigned row_bytes, unsigned vec_bytes, F &&emit) const {
+        using C = typename Arith<S>::C;
+        using RW = Raw<V * int(sizeof(C))>;
+        using W = Vec<C, V>;
+        constexpr int n = 2 * NC;
+        const auto r_x = rsrc(x ? x : xpay, vec_bytes);
+        const Cx<T> *own = lds + min(p.local, ns - 1) * kCloverRow<NC>;
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+            Cx<T> v[n][V];
+            if (x || xpay) {
+                W w[n];
+#pragma unroll
+                for (int k = 0; k < n; ++k) w[k] = __builtin_bit_cast(W, RW::load(r_x, p.vo, unsigned(ch * n + k) * row_bytes));
+#pragma unroll
+                for (int k = 0; k < n; ++k)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) v[k][i] = load_cx<T>(&w[k].c[i]);
+            }
+            if (!x) {
+#pragma unroll
+                for (int k = 0; k < n; ++k)
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        const Cx<T> h = acc[2 * ch + k / NC][k % NC][i];
+                        v[k][i] = xpay ? Cx<T>{fma(coef, h.re, v[k][i].re), fma(coef, h.im, v[k][i].im)} : coef * h;
+                    }
+            }
+#pragma unroll
+            for (int row = 0; row < n; ++row) {
+                Cx<T> o[V];
+#pragma unroll
+                for (int i = 0; i < V; ++i) o[i] = {T(0), T(0)};
+#pragma unroll
+                for (int k = 0; k < n; ++k) {
+                    const Cx<T> b = own[(ch * n + row) * n + k];
+#pragma unroll
+                    for (int i = 0; i < V; ++i) cfma(o[i], b, v[k][i]);
+                }
+                if (x) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        const Cx<T> h = acc[2 * ch + row / NC][row % NC][i];
+                        o[i].re = fma(coef, h.re, o[i].re);
+                        o[i].im = fma(coef, h.im, o[i].im);
+                    }
+                }
+                emit(ch * n + row, o, v[row]);
+            }
+        }
+    }
+};
 
 }  // namespace lane
 }  // namespace qcu

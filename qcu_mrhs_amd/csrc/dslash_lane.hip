@@ -84,6 +84,45 @@ __global__ __launch_bounds__(256, ORD ? 2 : (kMinWaves<S, NC, V>)) void k_dslash
     if (p.active) store_lane<S, NC, V>(acc, out, xpay, coef, p, R, vec_bytes);
 }
 
+// LDS of a workgroup with clover blocks: the hops', then the blocks.
+template <typename S, int NC>
+__host__ __device__ constexpr int clover_offset(int spb) {
+    return (spb * kSiteLds<S, NC> + 15) / 16 * 16;
+}
+template <typename S, int NC>
+__device__ __forceinline__ Clover<S, NC> clover_lds(const Cx<typename Arith<S>::T> *blocks, int spb) {
+    return {blocks, reinterpret_cast<Cx<typename Arith<S>::T> *>(lane_smem + clover_offset<S, NC>(spb))};
+}
+
+// With the clover blocks of the output sites: out = A x + coef D in, or (x null) out = A (coef D in + xpay).
+// The hop's sums never leave the registers in between; a separate pass over the vector reads and writes it
+// once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 57 us, FP64 185 -> 143 us against hop and pass; 5 RHS FP32 at
+// 98304 sites 34 -> 29 us).  Half of what is left over the bare hop is the blocks' 72 LDS reads per lane.
+template <typename S, int NC, int V, bool DAG>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clover(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ x,
+    const typename Arith<S>::C *xpay, const Cx<typename Arith<S>::T> *__restrict__ blocks, typename Arith<S>::T coef,
+    int Vh, int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
+    using T = typename Arith<S>::T;
+    using C = typename Arith<S>::C;
+    using RW = Raw<V * int(sizeof(C))>;
+    const int pos0 = xcd_remap(blockIdx.x, gridDim.x) * spb;
+    const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
+    Cx<T> acc[4][NC][V];
+    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb, pos0, parity, walk, vec_bytes, cl);
+    if (!p.active) return;
+    const unsigned rb = unsigned(R) * unsigned(sizeof(C));
+    const auto r_out = rsrc(out, vec_bytes);
+    cl.template rows<V>(acc, x, xpay, coef, p, min(spb, Vh - pos0), rb, vec_bytes,
+                        [&](int row, const Cx<T>(&o)[V], const Cx<T>(&)[V]) {
+                            Vec<C, V> w;
+#pragma unroll
+                            for (int i = 0; i < V; ++i) store_cx(&w.c[i], o[i]);
+                            RW::store(r_out, __builtin_bit_cast(typename RW::type, w), p.vo, unsigned(row) * rb);
+                        });
+}
+
 // Small lattices: the two hops of each direction in a wavefront of their own, the four wavefronts' sums
 // combined through LDS (wavefront mu finishes spin mu).  A lane then waits for two dependent loads (its
 // walk row, then links and both spinors together) instead of ten, and a lattice that would leave most
@@ -192,44 +231,59 @@ __device__ __forceinline__ void sum_sites(double (&v)[N], double *red, const Pla
 }
 
 // Reliable-update residual (FP64 hop): d = b - (xpay + coef D in) is not stored; lo = scale_r d in the inner
-// storage and part[block][r] = sum over the workgroup's sites of |d|^2.
-template <int NC, typename LO>
+// storage and part[block][r] = sum over the workgroup's sites of |d|^2.  CLOV: A xpay (clover blocks) in
+// place of xpay.
+template <int NC, typename LO, bool CLOV>
 __global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane_residual(
     LO *__restrict__ lo, const Cx<double> *__restrict__ in, const Cx<double> *__restrict__ gauge,
-    const Cx<double> *__restrict__ xpay, const Cx<double> *__restrict__ b, const double *__restrict__ scale,
-    double *__restrict__ part, double coef, int Vh, int R, int spb, int parity, const int *__restrict__ walk,
+    const Cx<double> *__restrict__ xpay, const Cx<double> *__restrict__ blocks, const Cx<double> *__restrict__ b,
+    const double *__restrict__ scale, double *__restrict__ part, double coef, int Vh, int R, int spb, int parity, const int *__restrict__ walk,
     unsigned vec_bytes) {
     using RL = Raw<int(sizeof(LO))>;
     using W = Vec<Cx<double>, 1>;
     const int blk = xcd_remap(blockIdx.x, gridDim.x);
     Cx<double> acc[4][NC][1];
-    const Place p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk,
-                                               vec_bytes);
+    const Clover<double, NC> cl = clover_lds<double, NC>(blocks, spb);
+    Place p;
+    if constexpr (CLOV)
+        p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes, cl);
+    else
+        p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
     double a2[1] = {0.0};
     if (p.active) {
         const unsigned rb = unsigned(R) * 16u;
         const auto r_x = rsrc(xpay, vec_bytes), r_b = rsrc(b, vec_bytes);
         const auto r_lo = rsrc(lo, vec_bytes / 16u * unsigned(sizeof(LO)));
         const double sc = scale[p.rv];
+        const auto finish = [&](int row, Cx<double> v, Cx<double> bv) {
+            const Cx<double> d = bv - v;
+            a2[0] = fma(d.re, d.re, fma(d.im, d.im, a2[0]));
+            LO o;
+            store_cx(&o, sc * d);
+            RL::store(r_lo, __builtin_bit_cast(typename RL::type, o), p.vo / 16u * unsigned(sizeof(LO)),
+                      unsigned(row) * unsigned(R) * unsigned(sizeof(LO)));
+        };
+        if constexpr (CLOV) {
+            cl.template rows<1>(acc, xpay, nullptr, coef, p, min(spb, Vh - blk * spb), rb, vec_bytes,
+                                [&](int row, const Cx<double>(&v)[1], const Cx<double>(&)[1]) {
+                                    finish(row, v[0], __builtin_bit_cast(W, Raw<16>::load(r_b, p.vo, unsigned(row) * rb)).c[0]);
+                                });
+        } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            W xw[NC], bw[NC];
+            for (int s = 0; s < 4; ++s) {
+                W xw[NC], bw[NC];
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                xw[c] = __builtin_bit_cast(W, Raw<16>::load(r_x, p.vo, unsigned(s * NC + c) * rb));
-                bw[c] = __builtin_bit_cast(W, Raw<16>::load(r_b, p.vo, unsigned(s * NC + c) * rb));
-            }
+                for (int c = 0; c < NC; ++c) {
+                    xw[c] = __builtin_bit_cast(W, Raw<16>::load(r_x, p.vo, unsigned(s * NC + c) * rb));
+                    bw[c] = __builtin_bit_cast(W, Raw<16>::load(r_b, p.vo, unsigned(s * NC + c) * rb));
+                }
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                Cx<double> v = xw[c].c[0];
-                v.re = fma(coef, acc[s][c][0].re, v.re);
-                v.im = fma(coef, acc[s][c][0].im, v.im);
-                const Cx<double> d = bw[c].c[0] - v;
-                a2[0] = fma(d.re, d.re, fma(d.im, d.im, a2[0]));
-                LO o;
-                store_cx(&o, sc * d);
-                RL::store(r_lo, __builtin_bit_cast(typename RL::type, o), p.vo / 16u * unsigned(sizeof(LO)),
-                          unsigned(s * NC + c) * unsigned(R) * unsigned(sizeof(LO)));
+                for (int c = 0; c < NC; ++c) {
+                    Cx<double> v = xw[c].c[0];
+                    v.re = fma(coef, acc[s][c][0].re, v.re);
+                    v.im = fma(coef, acc[s][c][0].im, v.im);
+                    finish(s * NC + c, v, bw[c].c[0]);
+                }
             }
         }
     }
@@ -238,40 +292,53 @@ __global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane
 }
 
 // Second hop of t = s + coef D in (16 bits) with omega's inner products over the stored values:
-// part[block][r][4] = Re, Im of <t, s>, <t, t>.
-template <typename S, int NC>
+// part[block][r][4] = Re, Im of <t, s>, <t, t>.  CLOV: t = A s + coef D in (clover blocks).
+template <typename S, int NC, bool CLOV>
 __global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_omega(
     typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
-    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay, float coef, int Vh,
-    int R, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes, double *__restrict__ part) {
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
+    const Cx<float> *__restrict__ blocks, float coef, int Vh, int R, int spb, int parity,
+    const int *__restrict__ walk, unsigned vec_bytes, double *__restrict__ part) {
     using C = typename Arith<S>::C;
     using RW = Raw<int(sizeof(C))>;
     const int blk = xcd_remap(blockIdx.x, gridDim.x);
     Cx<float> acc[4][NC][1];
-    const Place p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
+    const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
+    Place p;
+    if constexpr (CLOV)
+        p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes, cl);
+    else
+        p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
     float q[3] = {0.f, 0.f, 0.f};
     if (p.active) {
         const unsigned rb = unsigned(R) * unsigned(sizeof(C));
         const auto r_out = rsrc(out, vec_bytes), r_x = rsrc(xpay, vec_bytes);
-        C xw[4][NC];
+        const auto finish = [&](int row, Cx<float> v, Cx<float> x) {
+            C o;
+            store_cx(&o, v);
+            RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(row) * rb);
+            const Cx<float> t = load_cx<float>(&o);  // as a separate reduction would read it
+            q[0] = fmaf(x.re, t.re, fmaf(x.im, t.im, q[0]));
+            q[1] = fmaf(t.re, x.im, fmaf(-t.im, x.re, q[1]));
+            q[2] = fmaf(t.re, t.re, fmaf(t.im, t.im, q[2]));
+        };
+        if constexpr (CLOV) {
+            cl.template rows<1>(acc, xpay, nullptr, coef, p, min(spb, Vh - blk * spb), rb, vec_bytes,
+                                [&](int row, const Cx<float>(&v)[1], const Cx<float>(&x)[1]) { finish(row, v[0], x[0]); });
+        } else {
+            C xw[4][NC];
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 4; ++s)
 #pragma unroll
-            for (int c = 0; c < NC; ++c) xw[s][c] = __builtin_bit_cast(C, RW::load(r_x, p.vo, unsigned(s * NC + c) * rb));
+                for (int c = 0; c < NC; ++c) xw[s][c] = __builtin_bit_cast(C, RW::load(r_x, p.vo, unsigned(s * NC + c) * rb));
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 4; ++s)
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const Cx<float> x = load_cx<float>(&xw[s][c]);
-                const Cx<float> v = {fmaf(coef, acc[s][c][0].re, x.re), fmaf(coef, acc[s][c][0].im, x.im)};
-                C o;
-                store_cx(&o, v);
-                RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(s * NC + c) * rb);
-                const Cx<float> t = load_cx<float>(&o);  // as a separate reduction would read it
-                q[0] = fmaf(x.re, t.re, fmaf(x.im, t.im, q[0]));
-                q[1] = fmaf(t.re, x.im, fmaf(-t.im, x.re, q[1]));
-                q[2] = fmaf(t.re, t.re, fmaf(t.im, t.im, q[2]));
-            }
+                for (int c = 0; c < NC; ++c) {
+                    const Cx<float> x = load_cx<float>(&xw[s][c]);
+                    finish(s * NC + c, {fmaf(coef, acc[s][c][0].re, x.re), fmaf(coef, acc[s][c][0].im, x.im)}, x);
+                }
+        }
     }
     double w[3] = {double(q[0]), double(q[1]), double(q[2])};
     sum_sites<3>(w, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
@@ -314,26 +381,34 @@ struct Shape {
 };
 
 template <typename S, int NC>
-Shape lane_shape(int Vh, int R, int v) {
+Shape lane_shape(int Vh, int R, int v, bool clover = false) {
     Shape s;
     s.V = v;
     s.RV = R / s.V;
-    constexpr int per_site = kSiteLds<S, NC>;
+    const int blocks = clover ? kCloverRow<NC> * int(sizeof(Cx<typename Arith<S>::T>)) : 0;
+    const int per_site = kSiteLds<S, NC> + blocks;
     // 256 lanes, fewer where the grid would leave compute units idle (a site's hops are one serial
     // chain, so a small lattice runs at the speed of one workgroup: more, smaller ones)
     s.threads = 256;
     while (s.threads > 64 && s.threads / 2 >= s.RV && div_up(Vh, std::max(1, s.threads / s.RV)) < 2 * num_cus())
         s.threads /= 2;
     s.spb = std::max(1, s.threads / s.RV);
-    s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 ? 65536 : 40960) / per_site));  // 64 KB of LDS at most
+    s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 || clover ? 65520 : 40960) / per_site));  // 64 KB of LDS at most
     s.threads = (s.spb * s.RV + 63) / 64 * 64;
-    s.lds = std::max(size_t(s.spb) * per_site, size_t(s.threads) * 3 * sizeof(double));  // hops, then sums over sites
+    const size_t lds = clover ? clover_offset<S, NC>(s.spb) + size_t(s.spb) * blocks : size_t(s.spb) * per_site;
+    s.lds = std::max(lds, size_t(s.threads) * 3 * sizeof(double));  // hops, then sums over sites
     return s;
 }
 
+// fewest sites per workgroup of the forms that leave a partial sum per workgroup
 template <typename S>
-Shape lane_shape_nc(int Nc, int Vh, int R) {
-    return Nc == 2 ? lane_shape<S, 2>(Vh, R, 1) : Nc == 3 ? lane_shape<S, 3>(Vh, R, 1) : lane_shape<S, 4>(Vh, R, 1);
+int min_sites(int Nc, int Vh, int R) {
+    const auto least = [&](auto nc) {
+        return std::min(lane_shape<S, decltype(nc)::value>(Vh, R, 1).spb, lane_shape<S, decltype(nc)::value>(Vh, R, 1, true).spb);
+    };
+    return Nc == 2   ? least(std::integral_constant<int, 2>{})
+           : Nc == 3 ? least(std::integral_constant<int, 3>{})
+                     : least(std::integral_constant<int, 4>{});
 }
 
 template <int NC, typename LO>
@@ -341,12 +416,15 @@ hipError_t launch_residual(const DslashArgs &a, const DslashTune &t, const void 
                            double *partials, int &nblk, hipStream_t stream) {
     GeomTables tab;
     QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
-    const Shape sh = lane_shape<double, NC>(a.g.Vh, a.R, 1);
+    const Shape sh = lane_shape<double, NC>(a.g.Vh, a.R, 1, a.clover != nullptr);
     nblk = div_up(a.g.Vh, sh.spb);
     const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * 16);
-    hipLaunchKernelGGL((k_dslash_lane_residual<NC, LO>), dim3(nblk), dim3(sh.threads), sh.lds, stream,
+    auto k = a.clover ? k_dslash_lane_residual<NC, LO, true> : k_dslash_lane_residual<NC, LO, false>;
+    hipLaunchKernelGGL(k, dim3(nblk), dim3(sh.threads), sh.lds, stream,
                        static_cast<LO *>(lo), static_cast<const Cx<double> *>(a.in),
-                       static_cast<const Cx<double> *>(a.gauge), static_cast<const Cx<double> *>(a.xpay),
+                       static_cast<const Cx<double> *>(a.gauge),
+                       static_cast<const Cx<double> *>(a.clover ? a.clover_in : a.xpay),
+                       static_cast<const Cx<double> *>(a.clover),
                        static_cast<const Cx<double> *>(b), scale, partials, a.coef, a.g.Vh, a.R, sh.spb, a.parity,
                        tab.walk, vec_bytes);
     return hipGetLastError();
@@ -368,12 +446,14 @@ hipError_t launch_omega(const DslashArgs &a, const DslashTune &t, double *partia
     using C = typename Arith<S>::C;
     GeomTables tab;
     QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
-    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, 1);
+    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, 1, a.clover != nullptr);
     nblk = div_up(a.g.Vh, sh.spb);
     const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
-    hipLaunchKernelGGL((k_dslash_lane_omega<S, NC>), dim3(nblk), dim3(sh.threads), sh.lds, stream,
+    auto k = a.clover ? k_dslash_lane_omega<S, NC, true> : k_dslash_lane_omega<S, NC, false>;
+    hipLaunchKernelGGL(k, dim3(nblk), dim3(sh.threads), sh.lds, stream,
                        static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
-                       static_cast<const C *>(a.xpay), float(a.coef), a.g.Vh, a.R, sh.spb, a.parity, tab.walk,
+                       static_cast<const C *>(a.clover ? a.clover_in : a.xpay),
+                       static_cast<const Cx<float> *>(a.clover), float(a.coef), a.g.Vh, a.R, sh.spb, a.parity, tab.walk,
                        vec_bytes, partials);
     return hipGetLastError();
 }
@@ -423,6 +503,21 @@ hipError_t launch_v(const DslashArgs &a, const DslashTune &t, hipStream_t stream
     return hipGetLastError();
 }
 
+template <typename S, int NC, int V, bool DAG>
+hipError_t launch_clover_v(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    GeomTables tab;
+    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
+    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, V, true);
+    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
+    hipLaunchKernelGGL((k_dslash_lane_clover<S, NC, V, DAG>), dim3(div_up(a.g.Vh, sh.spb)), dim3(sh.threads), sh.lds,
+                       stream, static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.clover_in), static_cast<const C *>(a.xpay),
+                       static_cast<const Cx<typename Arith<S>::T> *>(a.clover), typename Arith<S>::T(a.coef), a.g.Vh,
+                       a.R, sh.RV, sh.spb, a.parity, tab.walk, vec_bytes);
+    return hipGetLastError();
+}
+
 // Four wavefronts per (site, RHS) pay while the lattice holds fewer lanes than four wavefronts per SIMD
 // (65536; 8^4, 4 RHS, FP64: 9.0 -> 5.6 us, 8^3 x 16, 16 RHS, FP16: 7.0 -> 5.5 us; at 98304 lanes 14.8 ->
 // 15.9 us), twice that for up to 4 RHS, whose links few lanes share (16^4, 4 RHS, FP32: 19.4 -> 15.6 us),
@@ -447,24 +542,34 @@ hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t st
     return hipGetLastError();
 }
 
+// FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
+// the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
+// 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache
+// one per lane, at twice the wavefronts, is faster (16^3 x 32, 12 RHS: 57 against 61 us).
+template <typename S, int NC>
+bool two_per_lane(const DslashArgs &a) {
+    const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * 8.0;
+    return std::is_same<S, float>::value && NC <= 3 && a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0;
+}
+
+template <typename S, int NC, int V>
+hipError_t launch_dag(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
+    if constexpr (V == 1 || (std::is_same<S, float>::value && NC <= 3)) {
+        if (a.clover)
+            return a.dagger ? launch_clover_v<S, NC, V, true>(a, t, stream) : launch_clover_v<S, NC, V, false>(a, t, stream);
+        return a.dagger ? launch_v<S, NC, V, true>(a, t, stream) : launch_v<S, NC, V, false>(a, t, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
 template <typename S, int NC>
 hipError_t launch_nc(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
-    using C = typename Arith<S>::C;
-    if (split_over_directions(a.g, a.R)) return launch_split<S, NC>(a, t, stream);
+    if (!a.clover && split_over_directions(a.g, a.R)) return launch_split<S, NC>(a, t, stream);
     if constexpr (std::is_same<S, float>::value)
         if (a.keep_order)
             return a.dagger ? launch_v<S, NC, 1, true, true>(a, t, stream)
                             : launch_v<S, NC, 1, false, true>(a, t, stream);
-    // FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
-    // the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
-    // 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache
-    // one per lane, at twice the wavefronts, is faster (16^3 x 32, 12 RHS: 57 against 61 us).
-    if constexpr (std::is_same<S, float>::value && NC <= 3) {
-        const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * sizeof(C);
-        if (a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0)
-            return a.dagger ? launch_v<S, NC, 2, true>(a, t, stream) : launch_v<S, NC, 2, false>(a, t, stream);
-    }
-    return a.dagger ? launch_v<S, NC, 1, true>(a, t, stream) : launch_v<S, NC, 1, false>(a, t, stream);
+    return two_per_lane<S, NC>(a) ? launch_dag<S, NC, 2>(a, t, stream) : launch_dag<S, NC, 1>(a, t, stream);
 }
 
 template <typename S>
@@ -516,6 +621,11 @@ void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz) 
     }
 }
 
+bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t) {
+    return t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec) && !a.keep_order &&
+           !split_over_directions(a.g, a.R);
+}
+
 hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
     if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 || a.g.L[1] % t.by ||
         a.g.L[2] % t.bz)
@@ -530,10 +640,9 @@ hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStrea
 }
 
 int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec) {
-    const Shape sh = prec == kDouble ? lane_shape_nc<double>(Nc, g.Vh, R)
-                     : prec == kSingle ? lane_shape_nc<float>(Nc, g.Vh, R)
-                                       : lane_shape_nc<__half>(Nc, g.Vh, R);
-    return div_up(g.Vh, sh.spb);
+    return div_up(g.Vh, prec == kDouble   ? min_sites<double>(Nc, g.Vh, R)
+                        : prec == kSingle ? min_sites<float>(Nc, g.Vh, R)
+                                          : min_sites<__half>(Nc, g.Vh, R));
 }
 
 hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,

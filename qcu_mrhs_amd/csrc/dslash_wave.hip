@@ -404,7 +404,7 @@ hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, i
 
 hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *lo, int lo_prec, const double *scale,
                                      double *partials, long partials_cap, double *nrm, hipStream_t stream) {
-    if (a.prec != kDouble || a.dagger || !a.in || !a.gauge || !a.xpay || !b || !lo || !scale || !partials || !nrm ||
+    if (a.prec != kDouble || a.dagger || !a.in || !a.gauge || !(a.clover ? a.clover_in : a.xpay) || !b || !lo || !scale || !partials || !nrm ||
         a.R < 1 || 32L * a.R > 65536L || !dslash_supported(a.Nc, a.R))
         return hipErrorInvalidValue;
     if (a.g.Vh <= 0) return hipSuccess;
@@ -415,6 +415,7 @@ hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *l
     if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)) {
         QCU_HIP_TRY(launch_dslash_lane_residual(a, t, b, lo, lo_prec, scale, partials, nblk, stream));
     } else {
+        if (a.clover) return hipErrorNotSupported;
         if (t.variant != kDslashWaveSite) {
             DslashArgs w = a;
             w.tune = DslashTune{};

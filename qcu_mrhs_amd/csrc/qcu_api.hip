@@ -353,13 +353,12 @@ void mat_Qcu(int daggerFlag) {
         char *in_p = A + p * n * c->R * eb, *out_p = B + p * n * c->R * eb;
         if (c->clover) {
             // out_p = A_pp in_p - kappa D_p in_{1-p}  (A Hermitian: the dagger reaches D only)
-            DslashArgs a{out_p, A + (1 - p) * n * c->R * eb, c->gauge(P), nullptr, 1.0, c->g, c->Nc, c->R, p,
+            DslashArgs a{out_p, A + (1 - p) * n * c->R * eb, c->gauge(P), nullptr, -c->kappa, c->g, c->Nc, c->R, p,
                          daggerFlag ? 1 : 0, P};
             a.keep_order = keep;
-            ok = a.gauge && hip_ok(launch_dslash(a, c->stream), "dslash");
-            ok = ok && hip_ok(launch_clover_apply(out_p, in_p, c->clover_set.term(P, p), out_p, -c->kappa, c->g.Vh,
-                                                  c->Nc, c->R, P, CloverSet::storage(P), c->stream),
-                              "clover");
+            a.clover = c->clover_set.term(P, p);
+            a.clover_in = in_p;
+            ok = a.gauge && hip_ok(launch_dslash_clover(a, c->stream), "dslash with clover term");
             continue;
         }
         // out_p = in_p - kappa D_p in_{1-p}   (src/qcu_interface.cu:174-255)

@@ -91,6 +91,9 @@ private:
     // was computed and the caller runs the separate reduction
     hipError_t schur_omega(void *out, const void *in, void *tmp, const void *gauge, int prec, double kappa,
                            bool &fused, hipStream_t s);
+    // out = blocks clover_in + coef D in, or (clover_in null) blocks (coef D in + xpay)
+    hipError_t dslash_clover(void *out, const void *in, const void *gauge, int prec, int parity, const void *blocks,
+                             const void *clover_in, const void *xpay, double coef, int dagger, hipStream_t s);
     // out = A_pp in + coef y (clover term or its inverse of parity p, storage `prec`)
     hipError_t clover_apply(void *out, const void *in, const void *blocks, const void *y, double coef, int prec,
                             hipStream_t s);

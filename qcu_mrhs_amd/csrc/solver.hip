@@ -33,8 +33,9 @@
 // Wilson-clover operator M = A - kappa D (set_clover): the same recurrences on
 // the Schur system A_oo - kappa^2 D_oe A_ee^{-1} D_eo with
 // b' = b_o + kappa D_oe A_ee^{-1} b_e and x_e = A_ee^{-1} (b_e + kappa D_eo x_o);
-// the clover blocks and their inverse are applied by two extra passes per
-// Schur operator (FP64 for FP64 vectors, an FP32 copy for the inner ones).
+// the clover blocks and their inverse are applied in the hops' epilogues, where
+// the lane kernel runs them, else by two extra passes per Schur operator (FP64
+// for FP64 vectors, an FP32 copy for the inner ones).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -210,14 +211,21 @@ hipError_t BiCGStab::clover_apply(void *out, const void *in, const void *blocks,
     return launch_clover_apply(out, in, blocks, y, coef, g_.Vh, Nc_, R_, prec, CloverSet::storage(prec), s);
 }
 
+hipError_t BiCGStab::dslash_clover(void *out, const void *in, const void *gauge, int prec, int parity,
+                                   const void *blocks, const void *clover_in, const void *xpay, double coef,
+                                   int dagger, hipStream_t s) {
+    DslashArgs a{out, in, gauge, xpay, coef, g_, Nc_, R_, parity, dagger, prec};
+    a.clover = blocks;
+    a.clover_in = clover_in;
+    return launch_dslash_clover(a, s);
+}
+
 hipError_t BiCGStab::apply_schur(void *out, const void *in, void *tmp, const void *gauge, int prec,
                                  double kappa, int dagger, hipStream_t s) {
     if (clover_) {
         // A is Hermitian, so the dagger only reaches the hops
-        QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, dagger, s));
-        QCU_HIP_TRY(clover_apply(tmp, tmp, clover_->inverse(prec, 0), nullptr, 0.0, prec, s));
-        QCU_HIP_TRY(dslash(out, tmp, gauge, prec, 1, nullptr, 1.0, dagger, s));
-        return clover_apply(out, in, clover_->term(prec, 1), out, -kappa * kappa, prec, s);
+        QCU_HIP_TRY(dslash_clover(tmp, in, gauge, prec, 0, clover_->inverse(prec, 0), nullptr, nullptr, 1.0, dagger, s));
+        return dslash_clover(out, tmp, gauge, prec, 1, clover_->term(prec, 1), in, nullptr, -kappa * kappa, dagger, s);
     }
     QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, dagger, s));
     QCU_HIP_TRY(dslash(out, tmp, gauge, prec, 1, in, -kappa * kappa, dagger, s));
@@ -227,13 +235,20 @@ hipError_t BiCGStab::apply_schur(void *out, const void *in, void *tmp, const voi
 hipError_t BiCGStab::schur_omega(void *out, const void *in, void *tmp, const void *gauge, int prec, double kappa,
                                  bool &fused, hipStream_t s) {
     fused = false;
-    if (clover_ || !dotp_ || (prec != kHalf && prec != kBF16)) return apply_schur(out, in, tmp, gauge, prec, kappa, 0, s);
-    QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, 0, s));
+    if (!dotp_ || (prec != kHalf && prec != kBF16)) return apply_schur(out, in, tmp, gauge, prec, kappa, 0, s);
+    if (clover_)
+        QCU_HIP_TRY(dslash_clover(tmp, in, gauge, prec, 0, clover_->inverse(prec, 0), nullptr, nullptr, 1.0, 0, s));
+    else
+        QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, 0, s));
     DslashArgs a;
     a.out = out;
     a.in = tmp;
     a.gauge = gauge;
     a.xpay = in;
+    if (clover_) {
+        a.clover = clover_->term(prec, 1);
+        a.clover_in = in;
+    }
     a.coef = -kappa * kappa;
     a.g = g_;
     a.Nc = Nc_;
@@ -247,6 +262,7 @@ hipError_t BiCGStab::schur_omega(void *out, const void *in, void *tmp, const voi
         return hipSuccess;
     }
     if (e != hipErrorNotSupported) return e;
+    if (clover_) return launch_dslash_clover(a, s);
     return dslash(out, tmp, gauge, prec, 1, in, -kappa * kappa, 0, s);
 }
 
@@ -255,7 +271,11 @@ hipError_t BiCGStab::residual_lo(const void *x_o, const void *g64, double kappa,
     a.out = nullptr;
     a.in = tmp64_;
     a.gauge = g64;
-    a.xpay = clover_ ? ax64_ : x_o;
+    a.xpay = x_o;
+    if (clover_) {
+        a.clover = clover_->term(kDouble, 1);
+        a.clover_in = x_o;
+    }
     a.coef = -kappa * kappa;
     a.g = g_;
     a.Nc = Nc_;
@@ -263,9 +283,17 @@ hipError_t BiCGStab::residual_lo(const void *x_o, const void *g64, double kappa,
     a.parity = 1;
     a.dagger = 0;
     a.prec = kDouble;
-    if (32L * R_ <= 65536L)  // 4 R doubles of LDS per workgroup
+    if (32L * R_ <= 65536L) {  // 4 R doubles of LDS per workgroup
+        hipError_t e = launch_dslash_residual_lo(a, bp_, r_, prec, dscale_ + R_, part_, part_cap_, dn_, s);
+        if (!clover_ || e != hipErrorNotSupported) return e;
+        // a kernel without the clover form: A_oo x_o apart
+        QCU_HIP_TRY(clover_apply(ax64_, x_o, a.clover, nullptr, 0.0, kDouble, s));
+        a.xpay = ax64_;
+        a.clover = a.clover_in = nullptr;
         return launch_dslash_residual_lo(a, bp_, r_, prec, dscale_ + R_, part_, part_cap_, dn_, s);
-    QCU_HIP_TRY(dslash(v64_, tmp64_, g64, kDouble, 1, a.xpay, -kappa * kappa, 0, s));
+    }
+    a.out = v64_;
+    QCU_HIP_TRY(clover_ ? launch_dslash_clover(a, s) : dslash(v64_, tmp64_, g64, kDouble, 1, x_o, -kappa * kappa, 0, s));
     return launch_residual_lo(dn_, r_, prec, bp_, v64_, dscale_ + R_, n_, R_, red_, 7, s);
 }
 
@@ -278,12 +306,11 @@ hipError_t BiCGStab::true_residual(const void *b_full, const void *x_full, const
     std::vector<double> rr(R_, 0.0), bb(R_, 0.0);
     for (int p = 0; p < 2; ++p) {
         // tmp = A_pp x_p - kappa D_p x_{1-p} = (M x)_p ; v = b_p - tmp
-        const void *ax = x + p * nR;
-        if (clover_) {
-            QCU_HIP_TRY(clover_apply(v64_, x + p * nR, clover_->term(kDouble, p), nullptr, 0.0, kDouble, s));
-            ax = v64_;
-        }
-        QCU_HIP_TRY(dslash(tmp64_, x + (1 - p) * nR, g64, kDouble, p, ax, -kappa, 0, s));
+        if (clover_)
+            QCU_HIP_TRY(dslash_clover(tmp64_, x + (1 - p) * nR, g64, kDouble, p, clover_->term(kDouble, p), x + p * nR,
+                                      nullptr, -kappa, 0, s));
+        else
+            QCU_HIP_TRY(dslash(tmp64_, x + (1 - p) * nR, g64, kDouble, p, x + p * nR, -kappa, 0, s));
         QCU_HIP_TRY(launch_xsay_norm(dn_, v64_, b + p * nR, tmp64_, n_, R_, kDouble, false, red_, 4, s));
         QCU_HIP_TRY(launch_norm(dn_ + R_, b + p * nR, n_, R_, kDouble, false, red_, 5, s));
         QCU_HIP_TRY(hipMemcpyAsync(h_, dn_, sizeof(double) * 2 * R_, hipMemcpyDeviceToHost, s));
@@ -456,12 +483,12 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
                 QCU_HIP_TRY(hipGetLastError());
             }
             // FP64 Schur operator on x_o: first hop into tmp64_, second hop fused with b' - A x_o
-            // (clover: tmp64_ = A_ee^{-1} D_eo x_o and the fused hop's xpay A_oo x_o)
-            QCU_HIP_TRY(dslash(tmp64_, x_o, gauge.g64, kDouble, 0, nullptr, 1.0, 0, s));
-            if (clover_) {
-                QCU_HIP_TRY(clover_apply(tmp64_, tmp64_, clover_->inverse(kDouble, 0), nullptr, 0.0, kDouble, s));
-                QCU_HIP_TRY(clover_apply(ax64_, x_o, clover_->term(kDouble, 1), nullptr, 0.0, kDouble, s));
-            }
+            // (clover: tmp64_ = A_ee^{-1} D_eo x_o)
+            if (clover_)
+                QCU_HIP_TRY(dslash_clover(tmp64_, x_o, gauge.g64, kDouble, 0, clover_->inverse(kDouble, 0), nullptr,
+                                          nullptr, 1.0, 0, s));
+            else
+                QCU_HIP_TRY(dslash(tmp64_, x_o, gauge.g64, kDouble, 0, nullptr, 1.0, 0, s));
             QCU_HIP_TRY(residual_lo(x_o, gauge.g64, kappa, P, s));
             QCU_HIP_TRY(hipMemcpyAsync(h_, dn_, sizeof(double) * R_, hipMemcpyDeviceToHost, s));
             QCU_HIP_TRY(hipStreamSynchronize(s));
@@ -535,8 +562,7 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
     // Schur operator): an axpy replaces the dslash.
     if (clover_) {
         // x_e = A_ee^{-1} (b_e + kappa D_eo x_o)
-        QCU_HIP_TRY(dslash(x_e, x_o, gauge.g64, kDouble, 0, b_e, kappa, 0, s));
-        QCU_HIP_TRY(clover_apply(x_e, x_e, clover_->inverse(kDouble, 0), nullptr, 0.0, kDouble, s));
+        QCU_HIP_TRY(dslash_clover(x_e, x_o, gauge.g64, kDouble, 0, clover_->inverse(kDouble, 0), nullptr, b_e, kappa, 0, s));
     } else if (!last_rt.empty()) {
         QCU_HIP_TRY(launch_scalar_fill(kap_, C64{kappa, 0.0}, R_, s));
         AxpyArgs ax{kXpay, x_e, b_e, tmp64_, nullptr, kap_, nullptr, nullptr, n_, R_, kDouble};
