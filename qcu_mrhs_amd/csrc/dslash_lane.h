@@ -212,12 +212,18 @@ __device__ __forceinline__ void hop_arith(Cx<typename Arith<S>::T> (&acc)[4][NC]
     }
 }
 
+// the neighbour spinor of a hop; the loads stay behind the arithmetic before them (see pin)
+template <typename C, int NC, int V>
+__device__ __forceinline__ void fetch(Vec<C, V> (&w)[4][NC], __amdgpu_buffer_rsrc_t r_in, unsigned vo,
+                                      unsigned row_bytes) {
+    asm volatile("" : "+v"(vo));
+    load_spinor<C, NC, V>(w, r_in, vo, row_bytes);
+}
+
 template <typename S, int NC, int V, bool DAG, int MU, bool FWD>
-__device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V], __amdgpu_buffer_rsrc_t r_in,
-                                    unsigned vo, unsigned row_bytes, const typename Arith<S>::Link *U) {
-    asm volatile("" : "+v"(vo));  // the loads stay behind the previous hop's arithmetic (see pin)
-    Vec<typename Arith<S>::C, V> w[4][NC];
-    load_spinor<typename Arith<S>::C, NC, V>(w, r_in, vo, row_bytes);
+__device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
+                                    const Vec<typename Arith<S>::C, V> (&w)[4][NC],
+                                    const typename Arith<S>::Link *U) {
     hop_arith<S, NC, V, DAG, MU, FWD>(acc, w, U);
     pin<typename Arith<S>::T, NC, V>(acc);
     __builtin_amdgcn_sched_barrier(0);
@@ -241,7 +247,8 @@ struct Place {
 // acc = D in for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes per site.
 // ORD: the hops of each direction are summed apart and then as ((x + z) + (y + t)), the wave-per-site
 // kernel's order (four sets of accumulators), instead of one after the other.
-template <typename S, int NC, int V, bool DAG, bool ORD = false, typename X = NoExtra>
+// AHEAD: the next hop's spinor is loaded before the arithmetic of this one.
+template <typename S, int NC, int V, bool DAG, bool ORD = false, bool AHEAD = false, typename X = NoExtra>
 __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
                                       const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
                                       int R, int RV, int spb, int pos0, int parity, const int *walk,
@@ -292,20 +299,34 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     // are the input sites about to leave the XCD's L2 and are read before the forward ones push them out
     // (24^3 x 48, 16 RHS: FP64 711 -> 636 us, FP32 350 -> 323 us against x+, x-, ..., t+, t-; 786 and
     // 393 us in the reverse order; 16^3 x 32, 12 RHS, FP64: 103 -> 79 us).
-#define QCU_BACK(MU) \
-    hop<S, NC, V, DAG, MU, false>(sums[ORD ? MU : 0], r_in, unsigned(row[2 + 2 * MU]) * sb + lo, rb, U + (2 * MU + 1) * NN);
-#define QCU_FORW(MU) \
-    hop<S, NC, V, DAG, MU, true>(sums[ORD ? MU : 0], r_in, unsigned(row[1 + 2 * MU]) * sb + lo, rb, U + (2 * MU) * NN);
-    QCU_BACK(3)
-    QCU_BACK(2)
-    QCU_BACK(1)
-    QCU_BACK(0)
-    QCU_FORW(0)
-    QCU_FORW(1)
-    QCU_FORW(2)
-    QCU_FORW(3)
-#undef QCU_BACK
-#undef QCU_FORW
+#define QCU_FETCH(W, MU, FWD) \
+    fetch<C, NC, V>(W, r_in, unsigned(row[2 + 2 * MU - FWD]) * sb + lo, rb);
+#define QCU_HOP(W, MU, FWD) hop<S, NC, V, DAG, MU, FWD>(sums[ORD ? MU : 0], W, U + (2 * MU + 1 - FWD) * NN);
+#define QCU_STEP(MU, FWD) { Vec<C, V> w[4][NC]; QCU_FETCH(w, MU, FWD) QCU_HOP(w, MU, FWD) }
+    if constexpr (AHEAD) {
+        Vec<C, V> w0[4][NC], w1[4][NC];
+        QCU_FETCH(w0, 3, false)
+        QCU_FETCH(w1, 2, false) QCU_HOP(w0, 3, false)
+        QCU_FETCH(w0, 1, false) QCU_HOP(w1, 2, false)
+        QCU_FETCH(w1, 0, false) QCU_HOP(w0, 1, false)
+        QCU_FETCH(w0, 0, true) QCU_HOP(w1, 0, false)
+        QCU_FETCH(w1, 1, true) QCU_HOP(w0, 0, true)
+        QCU_FETCH(w0, 2, true) QCU_HOP(w1, 1, true)
+        QCU_FETCH(w1, 3, true) QCU_HOP(w0, 2, true)
+        QCU_HOP(w1, 3, true)
+    } else {
+        QCU_STEP(3, false)
+        QCU_STEP(2, false)
+        QCU_STEP(1, false)
+        QCU_STEP(0, false)
+        QCU_STEP(0, true)
+        QCU_STEP(1, true)
+        QCU_STEP(2, true)
+        QCU_STEP(3, true)
+    }
+#undef QCU_STEP
+#undef QCU_HOP
+#undef QCU_FETCH
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll

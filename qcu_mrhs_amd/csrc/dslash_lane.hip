@@ -27,6 +27,13 @@ extern __shared__ __align__(16) unsigned char lane_smem[];
 template <typename S, int NC, int V>
 constexpr int kMinWaves = NC * V * int(sizeof(typename Arith<S>::T)) >= 32 ? 2 : NC * V * int(sizeof(typename Arith<S>::T)) >= 24 ? 3 : 4;
 
+// 16 bits, Nc <= 3: the next hop's spinor is loaded ahead, at 12 registers and no loss of occupancy (24^3 x 48:
+// 104 -> 97 us at 4 RHS, 333 -> 328 at 24, equal at 32; Nc = 4: 84 -> 87 us at 16^3 x 32, 32 RHS).  Not in
+// FP32 and FP64, whose lines then come into the L2 a hop too early (16^3 x 32, 12 RHS, FP64: 107 -> 111 us;
+// 24^3 x 48, 16 RHS: 645 -> 683 us, FP32 325 -> 339 us).
+template <typename S, int NC>
+constexpr bool kAhead = sizeof(typename Arith<S>::C) == 4 && NC <= 3;
+
 // out = coef acc (+ xpay) at this lane's place
 template <typename S, int NC, int V>
 __device__ __forceinline__ void store_lane(const Cx<typename Arith<S>::T> (&acc)[4][NC][V], typename Arith<S>::C *out,
@@ -79,7 +86,7 @@ __global__ __launch_bounds__(256, ORD ? 2 : (kMinWaves<S, NC, V>)) void k_dslash
     const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *xpay, typename Arith<S>::T coef, int Vh,
     int R, int RV, int spb, int parity, const int *__restrict__ walk, unsigned vec_bytes) {
     Cx<typename Arith<S>::T> acc[4][NC][V];
-    const Place p = hops<S, NC, V, DAG, ORD>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
+    const Place p = hops<S, NC, V, DAG, ORD, !ORD && kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, RV, spb,
                                              xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes);
     if (p.active) store_lane<S, NC, V>(acc, out, xpay, coef, p, R, vec_bytes);
 }
@@ -96,8 +103,8 @@ __device__ __forceinline__ Clover<S, NC> clover_lds(const Cx<typename Arith<S>::
 
 // With the clover blocks of the output sites: out = A x + coef D in, or (x null) out = A (coef D in + xpay).
 // The hop's sums never leave the registers in between; a separate pass over the vector reads and writes it
-// once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 57 us, FP64 185 -> 143 us against hop and pass; 5 RHS FP32 at
-// 98304 sites 34 -> 29 us).  Half of what is left over the bare hop is the blocks' 72 LDS reads per lane.
+// once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 57 us, FP64 185 -> 143 us against hop and pass; FP32, 5 RHS, at
+// 20 x 14 x 10 x 18 34 -> 29 us).  Half of what is left over the bare hop is the blocks' 72 LDS reads per lane.
 template <typename S, int NC, int V, bool DAG>
 __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clover(
     typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
@@ -110,7 +117,8 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clov
     const int pos0 = xcd_remap(blockIdx.x, gridDim.x) * spb;
     const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
     Cx<T> acc[4][NC][V];
-    const Place p = hops<S, NC, V, DAG>(acc, lane_smem, in, gauge, Vh, R, RV, spb, pos0, parity, walk, vec_bytes, cl);
+    const Place p =
+        hops<S, NC, V, DAG, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, RV, spb, pos0, parity, walk, vec_bytes, cl);
     if (!p.active) return;
     const unsigned rb = unsigned(R) * unsigned(sizeof(C));
     const auto r_out = rsrc(out, vec_bytes);
@@ -306,9 +314,10 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_omeg
     const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
     Place p;
     if constexpr (CLOV)
-        p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes, cl);
+        p = hops<S, NC, 1, false, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity,
+                                                        walk, vec_bytes, cl);
     else
-        p = hops<S, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
+        p = hops<S, NC, 1, false, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
     float q[3] = {0.f, 0.f, 0.f};
     if (p.active) {
         const unsigned rb = unsigned(R) * unsigned(sizeof(C));
@@ -369,7 +378,7 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_grou
     const long off = tab.n * tab.base[grp];
     const unsigned vec_bytes = unsigned(tab.n * R * long(sizeof(C)));
     Cx<T> acc[4][NC][1];
-    const Place p = hops<S, NC, 1, DAG>(acc, lane_smem, in + off, gauge, Vh, R, R, spb,
+    const Place p = hops<S, NC, 1, DAG, false, kAhead<S, NC>>(acc, lane_smem, in + off, gauge, Vh, R, R, spb,
                                         xcd_remap(blockIdx.x, nblk) * spb, parity, walk, vec_bytes);
     if (p.active) store_lane<S, NC, 1>(acc, out + off, xpay ? xpay + off : nullptr, coef, p, R, vec_bytes);
 }
@@ -549,17 +558,14 @@ hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t st
 template <typename S, int NC>
 bool two_per_lane(const DslashArgs &a) {
     const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * 8.0;
-    return std::is_same<S, float>::value && NC <= 3 && a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0;
+    return a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0;
 }
 
 template <typename S, int NC, int V>
 hipError_t launch_dag(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
-    if constexpr (V == 1 || (std::is_same<S, float>::value && NC <= 3)) {
-        if (a.clover)
-            return a.dagger ? launch_clover_v<S, NC, V, true>(a, t, stream) : launch_clover_v<S, NC, V, false>(a, t, stream);
-        return a.dagger ? launch_v<S, NC, V, true>(a, t, stream) : launch_v<S, NC, V, false>(a, t, stream);
-    }
-    return hipErrorInvalidValue;
+    if (a.clover)
+        return a.dagger ? launch_clover_v<S, NC, V, true>(a, t, stream) : launch_clover_v<S, NC, V, false>(a, t, stream);
+    return a.dagger ? launch_v<S, NC, V, true>(a, t, stream) : launch_v<S, NC, V, false>(a, t, stream);
 }
 
 template <typename S, int NC>
@@ -569,7 +575,9 @@ hipError_t launch_nc(const DslashArgs &a, const DslashTune &t, hipStream_t strea
         if (a.keep_order)
             return a.dagger ? launch_v<S, NC, 1, true, true>(a, t, stream)
                             : launch_v<S, NC, 1, false, true>(a, t, stream);
-    return two_per_lane<S, NC>(a) ? launch_dag<S, NC, 2>(a, t, stream) : launch_dag<S, NC, 1>(a, t, stream);
+    if constexpr (std::is_same<S, float>::value && NC <= 3)
+        if (two_per_lane<S, NC>(a)) return launch_dag<S, NC, 2>(a, t, stream);
+    return launch_dag<S, NC, 1>(a, t, stream);
 }
 
 template <typename S>
