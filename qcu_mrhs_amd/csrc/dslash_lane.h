@@ -212,13 +212,19 @@ __device__ __forceinline__ void hop_arith(Cx<typename Arith<S>::T> (&acc)[4][NC]
     }
 }
 
-// the neighbour spinor of a hop; the loads stay behind the arithmetic before them (see pin)
+// Where the spinors come from: an RHS-innermost half vector (C [site][spin][colour][rhs]).  The loads of a
+// fetch stay behind the arithmetic before them (see pin).
 template <typename C, int NC, int V>
-__device__ __forceinline__ void fetch(Vec<C, V> (&w)[4][NC], __amdgpu_buffer_rsrc_t r_in, unsigned vo,
-                                      unsigned row_bytes) {
-    asm volatile("" : "+v"(vo));
-    load_spinor<C, NC, V>(w, r_in, vo, row_bytes);
-}
+struct MrhsRows {
+    static constexpr bool kSiteFast = false;  // consecutive lanes: consecutive right-hand sides
+    __amdgpu_buffer_rsrc_t r;
+    unsigned row_bytes, lo;  // lo: byte offset of the lane's right-hand sides in a row
+    __device__ __forceinline__ void fetch(Vec<C, V> (&w)[4][NC], int site) const {
+        unsigned vo = unsigned(site) * (4u * NC * row_bytes) + lo;
+        asm volatile("" : "+v"(vo));
+        load_spinor<C, NC, V>(w, r, vo, row_bytes);
+    }
+};
 
 template <typename S, int NC, int V, bool DAG, int MU, bool FWD>
 __device__ __forceinline__ void hop(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
@@ -244,15 +250,15 @@ struct Place {
     unsigned vo;    // byte offset of (site, spin 0, colour 0, rv V)
 };
 
-// acc = D in for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes per site.
+// acc = D (spinors of src) for the workgroup's sites, from traversal position pos0 on.  smem: kSiteLds bytes
+// per site.
 // ORD: the hops of each direction are summed apart and then as ((x + z) + (y + t)), the wave-per-site
 // kernel's order (four sets of accumulators), instead of one after the other.
 // AHEAD: the next hop's spinor is loaded before the arithmetic of this one.
-template <typename S, int NC, int V, bool DAG, bool ORD = false, bool AHEAD = false, typename X = NoExtra>
-__device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
-                                      const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
-                                      int R, int RV, int spb, int pos0, int parity, const int *walk,
-                                      unsigned vec_bytes, const X &extra = X{}) {
+template <typename S, int NC, int V, bool DAG, bool ORD, bool AHEAD, typename SRC, typename X>
+__device__ __forceinline__ Place hops_from(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
+                                           const SRC &src, const typename Arith<S>::C *gauge, int Vh, int RV, int spb,
+                                           int pos0, int parity, const int *walk, const X &extra) {
     using A = Arith<S>;
     using T = typename A::T;
     using C = typename A::C;
@@ -276,13 +282,15 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     extra.load(sw, ns);
     __syncthreads();
     Place p;
-    p.local = int(threadIdx.x) / RV;
-    p.rv = int(threadIdx.x) - p.local * RV;
-    p.active = p.local < ns;
+    if constexpr (SRC::kSiteFast) {
+        p.rv = int(threadIdx.x) / spb;
+        p.local = int(threadIdx.x) - p.rv * spb;
+    } else {
+        p.local = int(threadIdx.x) / RV;
+        p.rv = int(threadIdx.x) - p.local * RV;
+    }
+    p.active = p.local < ns && p.rv < RV;
     const int l = min(p.local, ns - 1);
-    const unsigned rb = unsigned(R) * unsigned(sizeof(C)), sb = 4u * NC * rb;
-    const unsigned lo = unsigned(p.rv) * V * unsigned(sizeof(C));
-    const auto r_in = rsrc(in, vec_bytes);
     const int *row = sw + l * 9;
     const typename A::Link *U = sl + l * LR;
     constexpr int NA = ORD ? 4 : 1;
@@ -299,8 +307,7 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
     // are the input sites about to leave the XCD's L2 and are read before the forward ones push them out
     // (24^3 x 48, 16 RHS: FP64 711 -> 636 us, FP32 350 -> 323 us against x+, x-, ..., t+, t-; 786 and
     // 393 us in the reverse order; 16^3 x 32, 12 RHS, FP64: 103 -> 79 us).
-#define QCU_FETCH(W, MU, FWD) \
-    fetch<C, NC, V>(W, r_in, unsigned(row[2 + 2 * MU - FWD]) * sb + lo, rb);
+#define QCU_FETCH(W, MU, FWD) src.fetch(W, row[2 + 2 * MU - FWD]);
 #define QCU_HOP(W, MU, FWD) hop<S, NC, V, DAG, MU, FWD>(sums[ORD ? MU : 0], W, U + (2 * MU + 1 - FWD) * NN);
 #define QCU_STEP(MU, FWD) { Vec<C, V> w[4][NC]; QCU_FETCH(w, MU, FWD) QCU_HOP(w, MU, FWD) }
     if constexpr (AHEAD) {
@@ -339,8 +346,85 @@ __device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V],
                     acc[s][c][v] = sums[0][s][c][v];
             }
     p.site = row[0];
-    p.vo = unsigned(p.site) * sb + lo;
     return p;
+}
+
+// acc = D in, `in` an RHS-innermost half vector of vec_bytes
+template <typename S, int NC, int V, bool DAG, bool ORD = false, bool AHEAD = false, typename X = NoExtra>
+__device__ __forceinline__ Place hops(Cx<typename Arith<S>::T> (&acc)[4][NC][V], unsigned char *smem,
+                                      const typename Arith<S>::C *in, const typename Arith<S>::C *gauge, int Vh,
+                                      int R, int RV, int spb, int pos0, int parity, const int *walk,
+                                      unsigned vec_bytes, const X &extra = X{}) {
+    using C = typename Arith<S>::C;
+    const unsigned rb = unsigned(R) * unsigned(sizeof(C));
+    const MrhsRows<C, NC, V> src{rsrc(in, vec_bytes), rb, unsigned(int(threadIdx.x) % RV) * V * unsigned(sizeof(C))};
+    Place p = hops_from<S, NC, V, DAG, ORD, AHEAD>(acc, smem, src, gauge, Vh, RV, spb, pos0, parity, walk, extra);
+    p.vo = unsigned(p.site) * (4u * NC * rb) + src.lo;
+    return p;
+}
+
+// Small lattices: the two hops of each direction in a wavefront of their own, the four wavefronts' sums
+// combined through LDS (wavefront mu finishes spin mu).  A lane then waits for two dependent loads (its
+// walk row, then links and both spinors together) instead of ten, and a lattice that would leave most
+// SIMDs without a wavefront has four times as many.
+template <typename S, int NC, bool DAG, int MU, typename SRC>
+__device__ __forceinline__ void direction(Cx<typename Arith<S>::T> (&acc)[4][NC][1], const SRC &src,
+                                          const typename Arith<S>::C *gauge, int Vh, int parity, const int *row) {
+    using A = Arith<S>;
+    using C = typename A::C;
+    constexpr int NN = NC * NC;
+    const int site = row[0], nf = row[1 + 2 * MU], nb = row[2 + 2 * MU];
+    Vec<C, 1> wf[4][NC], wb[4][NC];
+    src.fetch(wb, nb);
+    src.fetch(wf, nf);
+    const C *gf = gauge + ((MU * 2 + parity) * long(Vh) + site) * NN, *gb = gauge + ((MU * 2 + 1 - parity) * long(Vh) + nb) * NN;
+    typename A::Link uf[NN], ub[NN];
+#pragma unroll
+    for (int a = 0; a < NC; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b) {
+            ub[a * NC + b] = A::link(gb[b * NC + a], false);
+            uf[a * NC + b] = A::link(gf[a * NC + b], true);
+        }
+    hop_arith<S, NC, 1, DAG, MU, false>(acc, wb, ub);
+    hop_arith<S, NC, 1, DAG, MU, true>(acc, wf, uf);
+}
+
+template <typename S, int NC, bool DAG, typename SRC>
+__device__ __forceinline__ void direction_of(int mu, Cx<typename Arith<S>::T> (&acc)[4][NC][1], const SRC &src,
+                                             const typename Arith<S>::C *gauge, int Vh, int parity, const int *row) {
+    using T = typename Arith<S>::T;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[s][c][0] = {T(0), T(0)};
+    if (mu == 0) direction<S, NC, DAG, 0>(acc, src, gauge, Vh, parity, row);
+    else if (mu == 1) direction<S, NC, DAG, 1>(acc, src, gauge, Vh, parity, row);
+    else if (mu == 2) direction<S, NC, DAG, 2>(acc, src, gauge, Vh, parity, row);
+    else direction<S, NC, DAG, 3>(acc, src, gauge, Vh, parity, row);
+}
+
+// part: [spin][wavefront][colour][lane] complex, the sums of wavefront mu's two hops; combined for spin mu
+template <typename T, int NC>
+__device__ __forceinline__ void put_parts(Cx<T> *part, int mu, int lane, const Cx<T> (&acc)[4][NC][1]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) part[((s * 4 + mu) * NC + c) * 64 + lane] = acc[s][c][0];
+}
+template <typename T, int NC>
+__device__ __forceinline__ Cx<T> sum_parts(const Cx<T> *part, int mu, int lane, int c) {
+    const Cx<T> *q = part + (mu * 4 * NC + c) * 64 + lane;
+    return (q[0] + q[2 * NC * 64]) + (q[NC * 64] + q[3 * NC * 64]);  // the wave-per-site kernel's order
+}
+
+// Four wavefronts per (site, RHS) pay while a launch holds fewer lanes than four wavefronts per SIMD
+// (65536; 8^4, 4 RHS, FP64: 9.0 -> 5.6 us, 8^3 x 16, 16 RHS, FP16: 7.0 -> 5.5 us; at 98304 lanes 14.8 ->
+// 15.9 us), twice that for up to 4 RHS, whose links few lanes share (16^4, 4 RHS, FP32: 19.4 -> 15.6 us),
+// and with no more than a quarter of a wavefront's lanes idle.
+inline bool split_over_directions(double sites, int R) {
+    if (R > 64 || (64 / R) * R < 48) return false;
+    return sites * R <= (R <= 4 ? 131072.0 : 65536.0);
 }
 
 // Clover blocks of a workgroup's sites: [site][chirality][2 NC][2 NC], complex in the accumulation type.
@@ -362,37 +446,34 @@ struct Clover {
         }
     }
 
-    // x given: rows of A x + coef acc (xpay not read); else rows of A (coef acc + xpay).
-    // emit(s, c, value[V], x_entry[V]) for every (spin, colour); x_entry is what the block was applied to
-    template <int V, typename F>
-    __device__ __forceinline__ void rows(const Cx<T> (&acc)[4][NC][V], const typename Arith<S>::C *x,
-                                         const typename Arith<S>::C *xpay, T coef, const Place &p, int ns,
-                                         unsigned row_bytes, unsigned vec_bytes, F &&emit) const {
-        using C = typename Arith<S>::C;
-        using RW = Raw<V * int(sizeof(C))>;
-        using W = Vec<C, V>;
+    // TERM: rows of A x + coef acc, x = read(entry); else rows of A (coef acc [+ read(entry) if have]).
+    // read(spin * NC + colour) returns the stored entry; emit(entry, value[V], x_entry[V]) is called for
+    // each, x_entry being what the block was applied to
+    template <int V, typename G, typename F>
+    __device__ __forceinline__ void rows_of(const Cx<T> (&acc)[4][NC][V], bool term, bool have, T coef, int site,
+                                            G &&read, F &&emit) const {
+        using W = Vec<typename Arith<S>::C, V>;
         constexpr int n = 2 * NC;
-        const auto r_x = rsrc(x ? x : xpay, vec_bytes);
-        const Cx<T> *own = lds + min(p.local, ns - 1) * kCloverRow<NC>;
+        const Cx<T> *own = lds + site * kCloverRow<NC>;
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch) {
             Cx<T> v[n][V];
-            if (x || xpay) {
+            if (term || have) {
                 W w[n];
 #pragma unroll
-                for (int k = 0; k < n; ++k) w[k] = __builtin_bit_cast(W, RW::load(r_x, p.vo, unsigned(ch * n + k) * row_bytes));
+                for (int k = 0; k < n; ++k) w[k] = read(ch * n + k);
 #pragma unroll
                 for (int k = 0; k < n; ++k)
 #pragma unroll
                     for (int i = 0; i < V; ++i) v[k][i] = load_cx<T>(&w[k].c[i]);
             }
-            if (!x) {
+            if (!term) {
 #pragma unroll
                 for (int k = 0; k < n; ++k)
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
                         const Cx<T> h = acc[2 * ch + k / NC][k % NC][i];
-                        v[k][i] = xpay ? Cx<T>{fma(coef, h.re, v[k][i].re), fma(coef, h.im, v[k][i].im)} : coef * h;
+                        v[k][i] = have ? Cx<T>{fma(coef, h.re, v[k][i].re), fma(coef, h.im, v[k][i].im)} : coef * h;
                     }
             }
 #pragma unroll
@@ -406,7 +487,7 @@ struct Clover {
 #pragma unroll
                     for (int i = 0; i < V; ++i) cfma(o[i], b, v[k][i]);
                 }
-                if (x) {
+                if (term) {
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
                         const Cx<T> h = acc[2 * ch + row / NC][row % NC][i];
@@ -417,6 +498,21 @@ struct Clover {
                 emit(ch * n + row, o, v[row]);
             }
         }
+    }
+
+    // x given: A x + coef acc (xpay not read); else A (coef acc + xpay); x, xpay RHS-innermost
+    template <int V, typename F>
+    __device__ __forceinline__ void rows(const Cx<T> (&acc)[4][NC][V], const typename Arith<S>::C *x,
+                                         const typename Arith<S>::C *xpay, T coef, const Place &p, int ns,
+                                         unsigned row_bytes, unsigned vec_bytes, F &&emit) const {
+        using RW = Raw<V * int(sizeof(typename Arith<S>::C))>;
+        const auto r_x = rsrc(x ? x : xpay, vec_bytes);
+        rows_of<V>(
+            acc, x != nullptr, xpay != nullptr, coef, min(p.local, ns - 1),
+            [&](int k) {
+                return __builtin_bit_cast(Vec<typename Arith<S>::C, V>, RW::load(r_x, p.vo, unsigned(k) * row_bytes));
+            },
+            emit);
     }
 };
 

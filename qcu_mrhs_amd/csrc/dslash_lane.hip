@@ -131,36 +131,8 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clov
                         });
 }
 
-// Small lattices: the two hops of each direction in a wavefront of their own, the four wavefronts' sums
-// combined through LDS (wavefront mu finishes spin mu).  A lane then waits for two dependent loads (its
-// walk row, then links and both spinors together) instead of ten, and a lattice that would leave most
-// SIMDs without a wavefront has four times as many.
-template <typename S, int NC, bool DAG, int MU>
-__device__ __forceinline__ void direction(Cx<typename Arith<S>::T> (&acc)[4][NC][1], const typename Arith<S>::C *in,
-                                          const typename Arith<S>::C *gauge, int Vh, unsigned rb, unsigned lo,
-                                          int parity, const int *row, unsigned vec_bytes) {
-    using A = Arith<S>;
-    using C = typename A::C;
-    constexpr int NN = NC * NC;
-    const int site = row[0], nf = row[1 + 2 * MU], nb = row[2 + 2 * MU];
-    const unsigned sb = 4u * NC * rb;
-    const auto r_in = rsrc(in, vec_bytes);
-    Vec<C, 1> wf[4][NC], wb[4][NC];
-    load_spinor<C, NC, 1>(wb, r_in, unsigned(nb) * sb + lo, rb);
-    load_spinor<C, NC, 1>(wf, r_in, unsigned(nf) * sb + lo, rb);
-    const C *gf = gauge + ((MU * 2 + parity) * long(Vh) + site) * NN, *gb = gauge + ((MU * 2 + 1 - parity) * long(Vh) + nb) * NN;
-    typename A::Link uf[NN], ub[NN];
-#pragma unroll
-    for (int a = 0; a < NC; ++a)
-#pragma unroll
-        for (int b = 0; b < NC; ++b) {
-            ub[a * NC + b] = A::link(gb[b * NC + a], false);
-            uf[a * NC + b] = A::link(gf[a * NC + b], true);
-        }
-    hop_arith<S, NC, 1, DAG, MU, false>(acc, wb, ub);
-    hop_arith<S, NC, 1, DAG, MU, true>(acc, wf, uf);
-}
-
+// Small lattices: a wavefront per direction (direction(), dslash_lane.h), summed through LDS; wavefront mu
+// finishes spin mu.
 template <typename S, int NC, bool DAG>
 __global__ __launch_bounds__(256) void k_dslash_lane_split(
     typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
@@ -178,18 +150,8 @@ __global__ __launch_bounds__(256) void k_dslash_lane_split(
     const int *row = walk + (long(parity) * Vh + pos0 + min(local, ns - 1)) * 9;
     const unsigned rb = unsigned(R) * unsigned(sizeof(C)), lo = unsigned(r) * unsigned(sizeof(C));
     Cx<T> acc[4][NC][1];
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[s][c][0] = {T(0), T(0)};
-    if (mu == 0) direction<S, NC, DAG, 0>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
-    else if (mu == 1) direction<S, NC, DAG, 1>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
-    else if (mu == 2) direction<S, NC, DAG, 2>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
-    else direction<S, NC, DAG, 3>(acc, in, gauge, Vh, rb, lo, parity, row, vec_bytes);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) part[((s * 4 + mu) * NC + c) * 64 + lane] = acc[s][c][0];
+    direction_of<S, NC, DAG>(mu, acc, MrhsRows<C, NC, 1>{rsrc(in, vec_bytes), rb, lo}, gauge, Vh, parity, row);
+    put_parts<T, NC>(part, mu, lane, acc);
     const bool active = local < ns;
     const unsigned vo = unsigned(row[0]) * 4u * NC * rb + unsigned(mu) * NC * rb + lo;
     C xw[NC];
@@ -203,8 +165,7 @@ __global__ __launch_bounds__(256) void k_dslash_lane_split(
     const auto r_out = rsrc(out, vec_bytes);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const Cx<T> *q = part + (mu * 4 * NC + c) * 64 + lane;
-        Cx<T> v = (q[0] + q[2 * NC * 64]) + (q[NC * 64] + q[3 * NC * 64]);  // the wave-per-site kernel's order
+        Cx<T> v = sum_parts<T, NC>(part, mu, lane, c);
         if (xpay) {
             Cx<T> x = load_cx<T>(&xw[c]);
             x.re = fma(coef, v.re, x.re);
@@ -527,15 +488,6 @@ hipError_t launch_clover_v(const DslashArgs &a, const DslashTune &t, hipStream_t
     return hipGetLastError();
 }
 
-// Four wavefronts per (site, RHS) pay while the lattice holds fewer lanes than four wavefronts per SIMD
-// (65536; 8^4, 4 RHS, FP64: 9.0 -> 5.6 us, 8^3 x 16, 16 RHS, FP16: 7.0 -> 5.5 us; at 98304 lanes 14.8 ->
-// 15.9 us), twice that for up to 4 RHS, whose links few lanes share (16^4, 4 RHS, FP32: 19.4 -> 15.6 us),
-// and with no more than a quarter of a wavefront's lanes idle.
-bool split_over_directions(const Geom &g, int R) {
-    if (R > 64 || (64 / R) * R < 48) return false;
-    return double(g.Vh) * R <= (R <= 4 ? 131072.0 : 65536.0);
-}
-
 template <typename S, int NC>
 hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
     using C = typename Arith<S>::C;
@@ -570,7 +522,7 @@ hipError_t launch_dag(const DslashArgs &a, const DslashTune &t, hipStream_t stre
 
 template <typename S, int NC>
 hipError_t launch_nc(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
-    if (!a.clover && split_over_directions(a.g, a.R)) return launch_split<S, NC>(a, t, stream);
+    if (!a.clover && split_over_directions(a.g.Vh, a.R)) return launch_split<S, NC>(a, t, stream);
     if constexpr (std::is_same<S, float>::value)
         if (a.keep_order)
             return a.dagger ? launch_v<S, NC, 1, true, true>(a, t, stream)
@@ -631,7 +583,7 @@ void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz) 
 
 bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t) {
     return t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec) && !a.keep_order &&
-           !split_over_directions(a.g, a.R);
+           !split_over_directions(a.g.Vh, a.R);
 }
 
 hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {

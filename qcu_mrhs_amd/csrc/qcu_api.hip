@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "clover.h"
+#include "dslash_direct.h"
 #include "groups.h"
 #include "layout.h"
 #include "lgnn.h"
@@ -324,6 +325,17 @@ void start_dslash(int parity, int daggerFlag) {
     if (parity != 0 && parity != 1) return set_error(kQcuErrorInvalidValue, "parity must be 0 or 1");
     const int P = c->iter_prec;
     const long n = c->half_n();
+    if (P == c->user_prec && c->gauge(P)) {
+        const OperatorArgs d{table(c->q_out, 0, P), table(c->q_in, 0, P), c->gauge(P), nullptr, 1.0, c->g, c->Nc, c->R,
+                             false, parity, daggerFlag ? 1 : 0, P};
+        if (operator_direct_supported(d)) {
+            if (hip_ok(launch_operator_direct(d, c->stream), "dslash"))
+                (void)hip_ok(hipStreamSynchronize(c->stream), "start_dslash");
+            c->q_in.clear();
+            c->q_out.clear();
+            return;
+        }
+    }
     bool ok = hip_ok(launch_gather(c->bufA, P, table(c->q_in, 0, c->user_prec), c->user_prec, n, c->R,
                                    c->stream), "gather");
     DslashArgs a{c->bufB, c->bufA, c->gauge(P), nullptr, 1.0, c->g, c->Nc, c->R, parity, daggerFlag ? 1 : 0, P};
@@ -344,6 +356,18 @@ void mat_Qcu(int daggerFlag) {
     const int P = c->iter_prec;
     const long n = c->half_n();
     const size_t eb = 2 * prec_bytes(P);
+    if (P == c->user_prec && c->gauge(P) && ensure_clover(c)) {
+        const OperatorArgs d{table(c->q_out, 0, P), table(c->q_in, 0, P), c->gauge(P),
+                             c->clover ? c->clover_set.term(P, 0) : nullptr, -c->kappa, c->g, c->Nc, c->R, true, 0,
+                             daggerFlag ? 1 : 0, P};
+        if (operator_direct_supported(d)) {
+            if (hip_ok(launch_operator_direct(d, c->stream), "mat_Qcu"))
+                (void)hip_ok(hipStreamSynchronize(c->stream), "mat_Qcu");
+            c->q_in.clear();
+            c->q_out.clear();
+            return;
+        }
+    }
     char *A = static_cast<char *>(c->bufA), *B = static_cast<char *>(c->bufB);
     bool ok = hip_ok(launch_gather(A, P, table(c->q_in, 0, c->user_prec), c->user_prec, 2 * n, c->R,
                                    c->stream), "gather");
