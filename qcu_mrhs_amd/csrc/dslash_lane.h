@@ -285,11 +285,12 @@ __device__ __forceinline__ Place hops_from(Cx<typename Arith<S>::T> (&acc)[4][NC
     if constexpr (SRC::kSiteFast) {
         p.rv = int(threadIdx.x) / spb;
         p.local = int(threadIdx.x) - p.rv * spb;
+        p.active = p.local < ns && p.rv < RV;
     } else {
         p.local = int(threadIdx.x) / RV;
         p.rv = int(threadIdx.x) - p.local * RV;
+        p.active = p.local < ns;
     }
-    p.active = p.local < ns && p.rv < RV;
     const int l = min(p.local, ns - 1);
     const int *row = sw + l * 9;
     const typename A::Link *U = sl + l * LR;
