@@ -55,8 +55,11 @@ template <> struct Raw<16> {
     __device__ __forceinline__ static type load(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
         return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, int(v), int(s), 0));
     }
+    // The row offset goes into the vector register: after a store of more than 8 bytes the compiler keeps two
+    // wait states before its data registers are written again, but not if the store has a scalar offset, and
+    // there rows have been stored with the next row's values in part (FP32, two per lane, 12 RHS at 24^4)
     __device__ __forceinline__ static void store(__amdgpu_buffer_rsrc_t r, type w, unsigned v, unsigned s) {
-        __builtin_amdgcn_raw_buffer_store_b128(w, r, int(v), int(s), kStorePolicy);
+        __builtin_amdgcn_raw_buffer_store_b128(w, r, int(v + s), 0, kStorePolicy);
     }
 };
 
