@@ -42,7 +42,7 @@ struct DslashArgs {
     // Sum the hops in the order of the wave-per-site kernel (16 bits: of the matrix-core kernel), bit for
     // bit: for callers that see the rounding of this storage type in vectors of a wider one
     bool keep_order = false;
-    // Clover blocks of the output parity (launch_dslash_clover, launch_dslash_omega and
+    // Clover blocks of the output parity (launch_dslash_clover, launch_dslash_dots and
     // launch_dslash_residual_lo), FP64 for FP64 storage, else FP32
     const void *clover = nullptr;
     const void *clover_in = nullptr;  // what they are applied to (null: the result of the hop)
@@ -81,8 +81,10 @@ bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t);
 int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec);
 hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
                                        const double *scale, double *partials, int &nblk, hipStream_t stream);
-hipError_t launch_dslash_lane_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
-                                    int &nblk);
+// inner products formed in a hop's epilogue: <r0, out>, or <out, x> and <out, out> with x = xpay (clover_in)
+enum DotsKind { kDotsAlpha, kDotsOmega };
+hipError_t launch_dslash_lane_dots(const DslashArgs &a, const DslashTune &t, DotsKind kind, const void *r0,
+                                   double *partials, hipStream_t stream, int &nblk);
 hipError_t launch_dslash_lane_groups(const DslashArgs &a, const SegTab &tab, int by, int bz, hipStream_t stream);
 hipError_t launch_dslash_lds(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_lds_supported(const Geom &g, int Nc, int prec);
@@ -117,13 +119,16 @@ hipError_t launch_dslash_residual_lo(const DslashArgs &a, const void *b, void *l
 // consecutive slices), fixed summation order
 hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, int slices, hipStream_t stream);
 
-// Second hop of the unpreconditioned FP16 / BF16 Schur operator, t = s + coef D in with
-// a.xpay = s, with omega's inner products <t, s>, <t, t> in its epilogue (lane or
-// matrix-core kernel, dagger 0): omega = <t, s> / <t, t> lands in st like launch_step_omega.
-// `partials` holds dslash_omega_partials(g, Nc, R) doubles.  Returns hipErrorNotSupported
-// (and launches nothing) when the tuned launch for these arguments is neither; the caller then runs the separate reduction.
-long dslash_omega_partials(const Geom &g, int Nc, int R);
-hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, Cx<double> *st, hipStream_t stream);
+// Second hop of a Schur operator, out = x + coef D in (x = a.xpay; with clover blocks A x + coef D in,
+// x = a.clover_in), dagger 0, with the inner products of a BiCGStab step in its epilogue, finished into st:
+// kDotsAlpha: out = v, alpha = rho / <r0, v> like launch_step_alpha; kDotsOmega: out = t, x = s,
+// omega = <t, s> / <t, t> like launch_step_omega (r0 not read).
+// `partials` holds dslash_dots_partials(g, Nc, R, prec) doubles.  Returns hipErrorNotSupported (and
+// launches nothing) when the launch chosen for these arguments has no such form (the lane kernel has both,
+// the 16-bit matrix-core kernel omega's without clover blocks); the caller then runs the separate reduction.
+long dslash_dots_partials(const Geom &g, int Nc, int R, int prec);
+hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0, double *partials, long cap,
+                              Cx<double> *st, hipStream_t stream);
 hipError_t launch_dslash_mfma_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
                                     int &nblk);
 

@@ -338,37 +338,34 @@ hipError_t launch_dslash_clover(const DslashArgs &a, hipStream_t stream) {
 constexpr int kMaxFinishRows = 4096;
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
-long dslash_omega_partials(const Geom &g, int Nc, int R) {
-    // one row of R x 4 per workgroup (matrix cores: at most one per 4 sites, or 64 per CU for the persistent grid)
-    const long lane = Nc <= 4 ? dslash_lane_blocks(g, Nc, R, kHalf) : 0;
-    const long nblk = std::max<long>({long(div_up(g.Vh, 4)), 64L * num_cus(), lane});
+long dslash_dots_partials(const Geom &g, int Nc, int R, int prec) {
+    // one row of R x 4 per workgroup: the lane kernel's, or a wavefront's worth of sites (a wavefront per
+    // direction); matrix cores: at most one per 4 sites, or 64 per CU for the persistent grid
+    long nblk = Nc <= 4 ? dslash_lane_blocks(g, Nc, R, prec) : 0;
+    if (R <= 64) nblk = std::max<long>(nblk, div_up(g.Vh, 64 / R));
+    if (prec == kHalf || prec == kBF16) nblk = std::max<long>({nblk, long(div_up(g.Vh, 4)), 64L * num_cus()});
     return (nblk + kDotSlices) * R * 4;
 }
 
-hipError_t launch_dslash_omega(const DslashArgs &a, double *partials, long cap, Cx<double> *st, hipStream_t stream) {
-    if (!dslash_supported(a.Nc, a.R) || a.g.Vh <= 0 || (a.prec != kHalf && a.prec != kBF16) || a.dagger ||
-        !(a.clover ? a.clover_in : a.xpay) || !partials || !st || a.R > kReduceThreads)
+hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0, double *partials, long cap,
+                              Cx<double> *st, hipStream_t stream) {
+    if (!dslash_supported(a.Nc, a.R) || a.g.Vh <= 0 || a.dagger || a.keep_order || !partials || !st ||
+        !(a.clover ? a.clover_in : a.xpay) || (kind == kDotsAlpha && !r0) || a.R > kReduceThreads)
         return hipErrorNotSupported;
-    DslashTune t = dslash_resolve(a);
-    if (a.clover && !dslash_lane_clover_fused(a, t)) return hipErrorNotSupported;
-    // below 32768 lanes the lane kernel's chain of eight hops is longer than the matrix-core kernel's
-    // one round of loads (8^3 x 16, 4 RHS: 8.1 against 6.7 us)
-    if (t.variant == kDslashLaneRhs && !a.clover && double(a.g.Vh) * a.R < 32768.0 && dslash_mfma_supported(a.Nc, a.prec)) {
-        t = DslashTune{};
-        t.variant = kDslashMfma;
-        t = dslash_fill_defaults(a, t);
-    }
+    const DslashTune t = dslash_resolve(a);
     const bool lane = t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
-    if (!lane && t.variant != kDslashMfma) return hipErrorNotSupported;
-    if (cap < dslash_omega_partials(a.g, a.Nc, a.R)) return hipErrorInvalidValue;
+    const bool mfma = t.variant == kDslashMfma && (a.prec == kHalf || a.prec == kBF16) && kind == kDotsOmega && !a.clover;
+    if ((!lane && !mfma) || (a.clover && !dslash_lane_clover_fused(a, t))) return hipErrorNotSupported;
+    if (cap < dslash_dots_partials(a.g, a.Nc, a.R, a.prec)) return hipErrorInvalidValue;
     int nblk = 0;
-    if (lane) QCU_HIP_TRY(launch_dslash_lane_omega(a, t, partials, stream, nblk));
+    if (lane) QCU_HIP_TRY(launch_dslash_lane_dots(a, t, kind, r0, partials, stream, nblk));
     else QCU_HIP_TRY(launch_dslash_mfma_omega(a, t, partials, stream, nblk));
-    if (nblk <= kMaxFinishRows) return launch_finish_omega(st, a.R, partials, nblk, stream);
+    const auto finish = kind == kDotsAlpha ? launch_finish_alpha : launch_finish_omega;
+    if (nblk <= kMaxFinishRows) return finish(st, a.R, partials, nblk, stream);
     // [nblk][R][4] -> [kDotSlices][R][4] (after them) -> the finisher sums the slices in order
     double *p2 = partials + long(nblk) * a.R * 4;
     QCU_HIP_TRY(launch_rows_sum(p2, partials, nblk, 4 * a.R, kDotSlices, stream));
-    return launch_finish_omega(st, a.R, p2, kDotSlices, stream);
+    return finish(st, a.R, p2, kDotSlices, stream);
 }
 
 }  // namespace qcu

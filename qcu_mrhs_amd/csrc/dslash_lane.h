@@ -9,6 +9,7 @@
 // neighbour spinors are buffer loads whose (spin, colour) row offset is scalar.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dslash_common.h"
@@ -519,6 +520,89 @@ struct Clover {
             emit);
     }
 };
+
+// Wavefronts per SIMD the register budget is set for: accumulators, a hop's spinor rows and its projected
+// entries fit without spilling (Nc = 3: 130 registers FP64, 67 FP32, 62 FP16).
+template <typename S, int NC, int V>
+constexpr int kMinWaves = NC * V * int(sizeof(typename Arith<S>::T)) >= 32 ? 2 : NC * V * int(sizeof(typename Arith<S>::T)) >= 24 ? 3 : 4;
+
+// 16 bits, Nc <= 3: the next hop's spinor is loaded ahead, at 12 registers and no loss of occupancy (24^3 x 48:
+// 104 -> 97 us at 4 RHS, 333 -> 328 at 24, equal at 32; Nc = 4: 84 -> 87 us at 16^3 x 32, 32 RHS).  Not in
+// FP32 and FP64, whose lines then come into the L2 a hop too early (16^3 x 32, 12 RHS, FP64: 107 -> 111 us;
+// 24^3 x 48, 16 RHS: 645 -> 683 us, FP32 325 -> 339 us).
+template <typename S, int NC>
+constexpr bool kAhead = sizeof(typename Arith<S>::C) == 4 && NC <= 3;
+
+// LDS of a workgroup with clover blocks: the hops', then the blocks.
+template <typename S, int NC>
+__host__ __device__ constexpr int clover_offset(int spb) {
+    return (spb * kSiteLds<S, NC> + 15) / 16 * 16;
+}
+template <typename S, int NC>
+__device__ __forceinline__ Clover<S, NC> clover_lds(const Cx<typename Arith<S>::T> *blocks, unsigned char *smem,
+                                                       int spb) {
+    return {blocks, reinterpret_cast<Cx<typename Arith<S>::T> *>(smem + clover_offset<S, NC>(spb))};
+}
+
+// Sums N values of V right-hand sides per lane over the workgroup's sites, per RHS, in site order; the sums
+// are those of the first RV lanes.  red: N V rows of blockDim.x doubles.
+template <int N, int V>
+__device__ __forceinline__ void sum_sites(double (&v)[N][V], double *red, const Place &p, int RV, int ns) {
+    __syncthreads();  // the hops' LDS is free
+    const int nt = blockDim.x;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int i = 0; i < V; ++i) red[(k * V + i) * nt + threadIdx.x] = p.active ? v[k][i] : 0.0;
+    __syncthreads();
+    if (int(threadIdx.x) < RV) {
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                double t = 0.0;
+                for (int l = 0; l < ns; ++l) t += red[(k * V + i) * nt + l * RV + threadIdx.x];
+                v[k][i] = t;
+            }
+    }
+}
+
+// Launch shape: V right-hand sides per lane, `spb` sites per workgroup of `threads` lanes.
+struct Shape {
+    int V, RV, spb, threads;
+    size_t lds;
+};
+
+template <typename S, int NC>
+Shape lane_shape(int Vh, int R, int v, bool clover = false) {
+    Shape s;
+    s.V = v;
+    s.RV = R / s.V;
+    const int blocks = clover ? kCloverRow<NC> * int(sizeof(Cx<typename Arith<S>::T>)) : 0;
+    const int per_site = kSiteLds<S, NC> + blocks;
+    // 256 lanes, fewer where the grid would leave compute units idle (a site's hops are one serial
+    // chain, so a small lattice runs at the speed of one workgroup: more, smaller ones)
+    s.threads = 256;
+    while (s.threads > 64 && s.threads / 2 >= s.RV && div_up(Vh, std::max(1, s.threads / s.RV)) < 2 * num_cus())
+        s.threads /= 2;
+    s.spb = std::max(1, s.threads / s.RV);
+    s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 || clover ? 65520 : 40960) / per_site));  // 64 KB of LDS at most
+    s.threads = (s.spb * s.RV + 63) / 64 * 64;
+    const size_t lds = clover ? clover_offset<S, NC>(s.spb) + size_t(s.spb) * blocks : size_t(s.spb) * per_site;
+    s.lds = std::max(lds, size_t(s.threads) * 3 * v * sizeof(double));  // hops, then sums over sites
+    return s;
+}
+
+// FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
+// the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
+// 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache
+// one per lane, at twice the wavefronts, is faster (16^3 x 32, 12 RHS: 57 against 61 us).
+template <typename S, int NC>
+bool two_per_lane(const DslashArgs &a) {
+    if (!std::is_same<S, float>::value || NC > 3) return false;
+    const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * 8.0;
+    return a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0;
+}
 
 }  // namespace lane
 }  // namespace qcu

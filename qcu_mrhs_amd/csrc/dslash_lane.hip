@@ -22,18 +22,6 @@ using namespace lane;
 
 extern __shared__ __align__(16) unsigned char lane_smem[];
 
-// Wavefronts per SIMD the register budget is set for: accumulators, a hop's spinor rows and its projected
-// entries fit without spilling (Nc = 3: 130 registers FP64, 67 FP32, 62 FP16).
-template <typename S, int NC, int V>
-constexpr int kMinWaves = NC * V * int(sizeof(typename Arith<S>::T)) >= 32 ? 2 : NC * V * int(sizeof(typename Arith<S>::T)) >= 24 ? 3 : 4;
-
-// 16 bits, Nc <= 3: the next hop's spinor is loaded ahead, at 12 registers and no loss of occupancy (24^3 x 48:
-// 104 -> 97 us at 4 RHS, 333 -> 328 at 24, equal at 32; Nc = 4: 84 -> 87 us at 16^3 x 32, 32 RHS).  Not in
-// FP32 and FP64, whose lines then come into the L2 a hop too early (16^3 x 32, 12 RHS, FP64: 107 -> 111 us;
-// 24^3 x 48, 16 RHS: 645 -> 683 us, FP32 325 -> 339 us).
-template <typename S, int NC>
-constexpr bool kAhead = sizeof(typename Arith<S>::C) == 4 && NC <= 3;
-
 // out = coef acc (+ xpay) at this lane's place
 template <typename S, int NC, int V>
 __device__ __forceinline__ void store_lane(const Cx<typename Arith<S>::T> (&acc)[4][NC][V], typename Arith<S>::C *out,
@@ -91,16 +79,6 @@ __global__ __launch_bounds__(256, ORD ? 2 : (kMinWaves<S, NC, V>)) void k_dslash
     if (p.active) store_lane<S, NC, V>(acc, out, xpay, coef, p, R, vec_bytes);
 }
 
-// LDS of a workgroup with clover blocks: the hops', then the blocks.
-template <typename S, int NC>
-__host__ __device__ constexpr int clover_offset(int spb) {
-    return (spb * kSiteLds<S, NC> + 15) / 16 * 16;
-}
-template <typename S, int NC>
-__device__ __forceinline__ Clover<S, NC> clover_lds(const Cx<typename Arith<S>::T> *blocks, int spb) {
-    return {blocks, reinterpret_cast<Cx<typename Arith<S>::T> *>(lane_smem + clover_offset<S, NC>(spb))};
-}
-
 // With the clover blocks of the output sites: out = A x + coef D in, or (x null) out = A (coef D in + xpay).
 // The hop's sums never leave the registers in between; a separate pass over the vector reads and writes it
 // once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 57 us, FP64 185 -> 143 us against hop and pass; FP32, 5 RHS, at
@@ -115,7 +93,7 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clov
     using C = typename Arith<S>::C;
     using RW = Raw<V * int(sizeof(C))>;
     const int pos0 = xcd_remap(blockIdx.x, gridDim.x) * spb;
-    const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
+    const Clover<S, NC> cl = clover_lds<S, NC>(blocks, lane_smem, spb);
     Cx<T> acc[4][NC][V];
     const Place p =
         hops<S, NC, V, DAG, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, RV, spb, pos0, parity, walk, vec_bytes, cl);
@@ -180,25 +158,6 @@ __global__ __launch_bounds__(256) void k_dslash_lane_split(
     }
 }
 
-// Sums `n` values per lane over the workgroup's sites, per RHS, in site order: row[rv] for the first RV lanes.
-// red: n rows of blockDim.x doubles.
-template <int N>
-__device__ __forceinline__ void sum_sites(double (&v)[N], double *red, const Place &p, int RV, int ns) {
-    __syncthreads();  // the hops' LDS is free
-    const int nt = blockDim.x;
-#pragma unroll
-    for (int k = 0; k < N; ++k) red[k * nt + threadIdx.x] = p.active ? v[k] : 0.0;
-    __syncthreads();
-    if (int(threadIdx.x) < RV) {
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            double t = 0.0;
-            for (int l = 0; l < ns; ++l) t += red[k * nt + l * RV + threadIdx.x];
-            v[k] = t;
-        }
-    }
-}
-
 // Reliable-update residual (FP64 hop): d = b - (xpay + coef D in) is not stored; lo = scale_r d in the inner
 // storage and part[block][r] = sum over the workgroup's sites of |d|^2.  CLOV: A xpay (clover blocks) in
 // place of xpay.
@@ -212,13 +171,13 @@ __global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane
     using W = Vec<Cx<double>, 1>;
     const int blk = xcd_remap(blockIdx.x, gridDim.x);
     Cx<double> acc[4][NC][1];
-    const Clover<double, NC> cl = clover_lds<double, NC>(blocks, spb);
+    const Clover<double, NC> cl = clover_lds<double, NC>(blocks, lane_smem, spb);
     Place p;
     if constexpr (CLOV)
         p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes, cl);
     else
         p = hops<double, NC, 1, false>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
-    double a2[1] = {0.0};
+    double a2[1][1] = {{0.0}};
     if (p.active) {
         const unsigned rb = unsigned(R) * 16u;
         const auto r_x = rsrc(xpay, vec_bytes), r_b = rsrc(b, vec_bytes);
@@ -226,7 +185,7 @@ __global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane
         const double sc = scale[p.rv];
         const auto finish = [&](int row, Cx<double> v, Cx<double> bv) {
             const Cx<double> d = bv - v;
-            a2[0] = fma(d.re, d.re, fma(d.im, d.im, a2[0]));
+            a2[0][0] = fma(d.re, d.re, fma(d.im, d.im, a2[0][0]));
             LO o;
             store_cx(&o, sc * d);
             RL::store(r_lo, __builtin_bit_cast(typename RL::type, o), p.vo / 16u * unsigned(sizeof(LO)),
@@ -256,68 +215,8 @@ __global__ __launch_bounds__(256, (kMinWaves<double, NC, 1>)) void k_dslash_lane
             }
         }
     }
-    sum_sites<1>(a2, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
-    if (int(threadIdx.x) < R) part[long(blockIdx.x) * R + threadIdx.x] = a2[0];
-}
-
-// Second hop of t = s + coef D in (16 bits) with omega's inner products over the stored values:
-// part[block][r][4] = Re, Im of <t, s>, <t, t>.  CLOV: t = A s + coef D in (clover blocks).
-template <typename S, int NC, bool CLOV>
-__global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_omega(
-    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
-    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
-    const Cx<float> *__restrict__ blocks, float coef, int Vh, int R, int spb, int parity,
-    const int *__restrict__ walk, unsigned vec_bytes, double *__restrict__ part) {
-    using C = typename Arith<S>::C;
-    using RW = Raw<int(sizeof(C))>;
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
-    Cx<float> acc[4][NC][1];
-    const Clover<S, NC> cl = clover_lds<S, NC>(blocks, spb);
-    Place p;
-    if constexpr (CLOV)
-        p = hops<S, NC, 1, false, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity,
-                                                        walk, vec_bytes, cl);
-    else
-        p = hops<S, NC, 1, false, false, kAhead<S, NC>>(acc, lane_smem, in, gauge, Vh, R, R, spb, blk * spb, parity, walk, vec_bytes);
-    float q[3] = {0.f, 0.f, 0.f};
-    if (p.active) {
-        const unsigned rb = unsigned(R) * unsigned(sizeof(C));
-        const auto r_out = rsrc(out, vec_bytes), r_x = rsrc(xpay, vec_bytes);
-        const auto finish = [&](int row, Cx<float> v, Cx<float> x) {
-            C o;
-            store_cx(&o, v);
-            RW::store(r_out, __builtin_bit_cast(typename RW::type, o), p.vo, unsigned(row) * rb);
-            const Cx<float> t = load_cx<float>(&o);  // as a separate reduction would read it
-            q[0] = fmaf(x.re, t.re, fmaf(x.im, t.im, q[0]));
-            q[1] = fmaf(t.re, x.im, fmaf(-t.im, x.re, q[1]));
-            q[2] = fmaf(t.re, t.re, fmaf(t.im, t.im, q[2]));
-        };
-        if constexpr (CLOV) {
-            cl.template rows<1>(acc, xpay, nullptr, coef, p, min(spb, Vh - blk * spb), rb, vec_bytes,
-                                [&](int row, const Cx<float>(&v)[1], const Cx<float>(&x)[1]) { finish(row, v[0], x[0]); });
-        } else {
-            C xw[4][NC];
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) xw[s][c] = __builtin_bit_cast(C, RW::load(r_x, p.vo, unsigned(s * NC + c) * rb));
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const Cx<float> x = load_cx<float>(&xw[s][c]);
-                    finish(s * NC + c, {fmaf(coef, acc[s][c][0].re, x.re), fmaf(coef, acc[s][c][0].im, x.im)}, x);
-                }
-        }
-    }
-    double w[3] = {double(q[0]), double(q[1]), double(q[2])};
-    sum_sites<3>(w, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
-    if (int(threadIdx.x) < R) {
-        double *row = part + (long(blockIdx.x) * R + threadIdx.x) * 4;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) row[k] = w[k];
-        row[3] = 0.0;
-    }
+    sum_sites<1, 1>(a2, reinterpret_cast<double *>(lane_smem), p, R, min(spb, Vh - blk * spb));
+    if (int(threadIdx.x) < R) part[long(blockIdx.x) * R + threadIdx.x] = a2[0][0];
 }
 
 // Every group of a batch in one launch (blockIdx.y = group, SegTab layout); spb[g] sites per workgroup.
@@ -342,32 +241,6 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_lane_grou
     const Place p = hops<S, NC, 1, DAG, false, kAhead<S, NC>>(acc, lane_smem, in + off, gauge, Vh, R, R, spb,
                                         xcd_remap(blockIdx.x, nblk) * spb, parity, walk, vec_bytes);
     if (p.active) store_lane<S, NC, 1>(acc, out + off, xpay ? xpay + off : nullptr, coef, p, R, vec_bytes);
-}
-
-// Launch shape: V right-hand sides per lane, `spb` sites per workgroup of `threads` lanes.
-struct Shape {
-    int V, RV, spb, threads;
-    size_t lds;
-};
-
-template <typename S, int NC>
-Shape lane_shape(int Vh, int R, int v, bool clover = false) {
-    Shape s;
-    s.V = v;
-    s.RV = R / s.V;
-    const int blocks = clover ? kCloverRow<NC> * int(sizeof(Cx<typename Arith<S>::T>)) : 0;
-    const int per_site = kSiteLds<S, NC> + blocks;
-    // 256 lanes, fewer where the grid would leave compute units idle (a site's hops are one serial
-    // chain, so a small lattice runs at the speed of one workgroup: more, smaller ones)
-    s.threads = 256;
-    while (s.threads > 64 && s.threads / 2 >= s.RV && div_up(Vh, std::max(1, s.threads / s.RV)) < 2 * num_cus())
-        s.threads /= 2;
-    s.spb = std::max(1, s.threads / s.RV);
-    s.spb = std::min(s.spb, std::max(1, (s.RV <= 2 || clover ? 65520 : 40960) / per_site));  // 64 KB of LDS at most
-    s.threads = (s.spb * s.RV + 63) / 64 * 64;
-    const size_t lds = clover ? clover_offset<S, NC>(s.spb) + size_t(s.spb) * blocks : size_t(s.spb) * per_site;
-    s.lds = std::max(lds, size_t(s.threads) * 3 * sizeof(double));  // hops, then sums over sites
-    return s;
 }
 
 // fewest sites per workgroup of the forms that leave a partial sum per workgroup
@@ -409,23 +282,6 @@ hipError_t launch_residual_lo(const DslashArgs &a, const DslashTune &t, const vo
         case kBF16: return launch_residual<NC, Bf162Store>(a, t, b, lo, scale, partials, nblk, stream);
         default: return hipErrorInvalidValue;
     }
-}
-
-template <typename S, int NC>
-hipError_t launch_omega(const DslashArgs &a, const DslashTune &t, double *partials, int &nblk, hipStream_t stream) {
-    using C = typename Arith<S>::C;
-    GeomTables tab;
-    QCU_HIP_TRY(geom_tables(a.g, t.by, t.bz, tab, stream));
-    const Shape sh = lane_shape<S, NC>(a.g.Vh, a.R, 1, a.clover != nullptr);
-    nblk = div_up(a.g.Vh, sh.spb);
-    const unsigned vec_bytes = unsigned(size_t(a.g.Vh) * 4 * NC * a.R * sizeof(C));
-    auto k = a.clover ? k_dslash_lane_omega<S, NC, true> : k_dslash_lane_omega<S, NC, false>;
-    hipLaunchKernelGGL(k, dim3(nblk), dim3(sh.threads), sh.lds, stream,
-                       static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
-                       static_cast<const C *>(a.clover ? a.clover_in : a.xpay),
-                       static_cast<const Cx<float> *>(a.clover), float(a.coef), a.g.Vh, a.R, sh.spb, a.parity, tab.walk,
-                       vec_bytes, partials);
-    return hipGetLastError();
 }
 
 template <typename S, int NC>
@@ -501,16 +357,6 @@ hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t st
                        static_cast<const C *>(a.xpay), typename Arith<S>::T(a.coef), a.g.Vh, a.R, spb, a.parity,
                        tab.walk, vec_bytes);
     return hipGetLastError();
-}
-
-// FP32: two right-hand sides per lane (16-byte loads, half the link reads) where the fields exceed
-// the 256 MiB memory-side cache and the rows are wide enough (24^3 x 48: 400 -> 323 us at 16 RHS,
-// 666 -> 574 at 24, 367 -> 357 at 12, but 243 -> 247 at 8 and 174 -> 203 at 4); inside the cache
-// one per lane, at twice the wavefronts, is faster (16^3 x 32, 12 RHS: 57 against 61 us).
-template <typename S, int NC>
-bool two_per_lane(const DslashArgs &a) {
-    const double bytes = double(a.g.Vh) * (8.0 * NC * NC + 8.0 * NC * a.R) * 8.0;
-    return a.R % 2 == 0 && a.R >= 12 && bytes > 268435456.0;
 }
 
 template <typename S, int NC, int V>
@@ -614,20 +460,6 @@ hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t,
         case 2: return launch_residual_lo<2>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
         case 3: return launch_residual_lo<3>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
         case 4: return launch_residual_lo<4>(a, t, b, lo, lo_prec, scale, partials, nblk, stream);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_dslash_lane_omega(const DslashArgs &a, const DslashTune &t, double *partials, hipStream_t stream,
-                                    int &nblk) {
-    if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 || a.g.L[1] % t.by || a.g.L[2] % t.bz)
-        return hipErrorInvalidValue;
-    const bool h = a.prec == kHalf;
-    if (!h && a.prec != kBF16) return hipErrorInvalidValue;
-    switch (a.Nc) {
-        case 2: return h ? launch_omega<__half, 2>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 2>(a, t, partials, nblk, stream);
-        case 3: return h ? launch_omega<__half, 3>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 3>(a, t, partials, nblk, stream);
-        case 4: return h ? launch_omega<__half, 4>(a, t, partials, nblk, stream) : launch_omega<__hip_bfloat16, 4>(a, t, partials, nblk, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -86,11 +86,9 @@ public:
 
 private:
     hipError_t ensure(int prec);
-    // t = A s whose second hop also forms omega's <t, s>, <t, t> and finishes omega into st_
-    // (FP16 / BF16, when the tuned dslash is the matrix-core kernel); fused = false: only t
-    // was computed and the caller runs the separate reduction
-    hipError_t schur_omega(void *out, const void *in, void *tmp, const void *gauge, int prec, double kappa,
-                           bool &fused, hipStream_t s);
+    // out = A in with the inner products of a step, and their alpha or omega in st_ (kDotsOmega: in = s)
+    hipError_t schur_dots(DotsKind kind, void *out, const void *in, void *tmp, const void *gauge, int prec,
+                          double kappa, hipStream_t s);
     // out = blocks clover_in + coef D in, or (clover_in null) blocks (coef D in + xpay)
     hipError_t dslash_clover(void *out, const void *in, const void *gauge, int prec, int parity, const void *blocks,
                              const void *clover_in, const void *xpay, double coef, int dagger, hipStream_t s);
@@ -122,7 +120,7 @@ private:
     double *h_ = nullptr;      // pinned host staging [8][R]
     double *part_ = nullptr;   // per-workgroup partial sums of the fused residual (mixed solves)
     long part_cap_ = 0;
-    double *dotp_ = nullptr;   // per-workgroup partials of the FP16/BF16 Schur hop's fused omega
+    double *dotp_ = nullptr;   // per-workgroup partials of the Schur hops' inner products
     long dotp_cap_ = 0;
     ReduceWork red_;
 };

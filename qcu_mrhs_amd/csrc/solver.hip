@@ -172,10 +172,14 @@ hipError_t BiCGStab::ensure(int prec) {
         if (err != hipSuccess) return err;
         alloc_prec_ = prec;
     }
-    if ((prec == kHalf || prec == kBF16) && !dotp_) {
-        dotp_cap_ = dslash_omega_partials(g_, Nc_, R_);
-        dotp_ = static_cast<double *>(dmalloc(sizeof(double) * size_t(dotp_cap_), err));
+    if (prec >= 0 && dotp_cap_ < dslash_dots_partials(g_, Nc_, R_, prec)) {
+        void *old = dotp_;
+        dfree(old);
+        const long cap = dslash_dots_partials(g_, Nc_, R_, prec);
+        dotp_cap_ = 0;
+        dotp_ = static_cast<double *>(dmalloc(sizeof(double) * size_t(cap), err));
         if (err != hipSuccess) return err;
+        dotp_cap_ = cap;
     }
     if (clover_ && !ax64_) {
         ax64_ = dmalloc(half64, err);
@@ -232,38 +236,21 @@ hipError_t BiCGStab::apply_schur(void *out, const void *in, void *tmp, const voi
     return hipSuccess;
 }
 
-hipError_t BiCGStab::schur_omega(void *out, const void *in, void *tmp, const void *gauge, int prec, double kappa,
-                                 bool &fused, hipStream_t s) {
-    fused = false;
-    if (!dotp_ || (prec != kHalf && prec != kBF16)) return apply_schur(out, in, tmp, gauge, prec, kappa, 0, s);
-    if (clover_)
-        QCU_HIP_TRY(dslash_clover(tmp, in, gauge, prec, 0, clover_->inverse(prec, 0), nullptr, nullptr, 1.0, 0, s));
-    else
-        QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, 0, s));
-    DslashArgs a;
-    a.out = out;
-    a.in = tmp;
-    a.gauge = gauge;
-    a.xpay = in;
+hipError_t BiCGStab::schur_dots(DotsKind kind, void *out, const void *in, void *tmp, const void *gauge, int prec,
+                                double kappa, hipStream_t s) {
+    DslashArgs a{out, tmp, gauge, in, -kappa * kappa, g_, Nc_, R_, 1, 0, prec};
     if (clover_) {
+        QCU_HIP_TRY(dslash_clover(tmp, in, gauge, prec, 0, clover_->inverse(prec, 0), nullptr, nullptr, 1.0, 0, s));
         a.clover = clover_->term(prec, 1);
         a.clover_in = in;
+    } else {
+        QCU_HIP_TRY(dslash(tmp, in, gauge, prec, 0, nullptr, 1.0, 0, s));
     }
-    a.coef = -kappa * kappa;
-    a.g = g_;
-    a.Nc = Nc_;
-    a.R = R_;
-    a.parity = 1;
-    a.dagger = 0;
-    a.prec = prec;
-    const hipError_t e = launch_dslash_omega(a, dotp_, dotp_cap_, st_, s);
-    if (e == hipSuccess) {
-        fused = true;
-        return hipSuccess;
-    }
+    const hipError_t e = launch_dslash_dots(a, kind, r0_, dotp_, dotp_cap_, st_, s);
     if (e != hipErrorNotSupported) return e;
-    if (clover_) return launch_dslash_clover(a, s);
-    return dslash(out, tmp, gauge, prec, 1, in, -kappa * kappa, 0, s);
+    QCU_HIP_TRY(clover_ ? launch_dslash_clover(a, s) : launch_dslash(a, s));
+    return kind == kDotsAlpha ? launch_step_alpha(st_, r0_, out, n_, R_, prec, red_, s)
+                              : launch_step_omega(st_, out, in, n_, R_, prec, red_, s);
 }
 
 hipError_t BiCGStab::residual_lo(const void *x_o, const void *g64, double kappa, int prec, hipStream_t s) {
@@ -409,8 +396,8 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
             QCU_HIP_TRY(prec->apply(ph_, p_, P, s));
             pin = ph_;
         }
-        QCU_HIP_TRY(apply_schur(v_, pin, tmp_, glo, P, kappa, 0, s));
-        QCU_HIP_TRY(launch_step_alpha(st_, r0_, v_, n_, R_, P, red_, s));
+        // v = A p and alpha = rho / <r0, v>, the inner product in the second hop's epilogue
+        QCU_HIP_TRY(schur_dots(kDotsAlpha, v_, pin, tmp_, glo, P, kappa, s));
         QCU_HIP_TRY(launch_step_s(s_, r_, v_, st_, n_, R_, P, s));
         const void *sin = s_;
         if (prec) {
@@ -418,11 +405,13 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
             sin = sh_;
         }
         // t = A s and omega = <t, s> / <t, t>: without a preconditioner the second hop's xpay vector
-        // is s, and the matrix-core kernel forms both inner products in its epilogue
-        bool fused = false;
-        if (!prec) QCU_HIP_TRY(schur_omega(t_, sin, tmp_, glo, P, kappa, fused, s));
-        else QCU_HIP_TRY(apply_schur(t_, sin, tmp_, glo, P, kappa, 0, s));
-        if (!fused) QCU_HIP_TRY(launch_step_omega(st_, t_, s_, n_, R_, P, red_, s));
+        // is s, and its epilogue forms both inner products
+        if (!prec) {
+            QCU_HIP_TRY(schur_dots(kDotsOmega, t_, sin, tmp_, glo, P, kappa, s));
+        } else {
+            QCU_HIP_TRY(apply_schur(t_, sin, tmp_, glo, P, kappa, 0, s));
+            QCU_HIP_TRY(launch_step_omega(st_, t_, s_, n_, R_, P, red_, s));
+        }
         QCU_HIP_TRY(launch_step_xr(x_it, r_, pin, sin, s_, t_, r0_, st_, n_, R_, P, red_, s));
         QCU_HIP_TRY(hipMemcpyAsync(h_, st_ + kRnorm2 * R_, sizeof(C64) * R_, hipMemcpyDeviceToHost, s));
         QCU_HIP_TRY(hipStreamSynchronize(s));
