@@ -104,9 +104,10 @@ hipError_t launch_step_omega(C64 *st, const void *t, const void *sv, long n, int
 // x += alpha p + omega shat ; r = s - omega t ; ||r||^2, <r0,r> ;
 // beta = ((alpha * rho_new) / omega) / rho ; rho <- rho_new.
 // Unpreconditioned: p = p, shat = s.  Right-preconditioned: p = N p, shat = N s.
+// host_r2, if given, is pinned host memory that also receives ||r||^2 (readable once the stream got there).
 hipError_t launch_step_xr(void *x, void *r, const void *p, const void *shat, const void *sv,
                           const void *t, const void *r0, C64 *st, long n, int R, int prec,
-                          ReduceWork &w, hipStream_t s);
+                          ReduceWork &w, hipStream_t s, double *host_r2 = nullptr);
 // p = r + beta * pscale * (p - omega v)
 hipError_t launch_step_p(void *p, const void *r, const void *v, const C64 *st, long n, int R,
                          int prec, hipStream_t s);

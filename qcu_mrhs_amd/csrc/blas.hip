@@ -337,6 +337,7 @@ struct XROp {  // x += a p + w shat ; r = s - w t ; ||r||^2 ; <r0, r> ; beta
     const CS *p, *shat, *s, *t, *r0;
     C64 *st;
     int R;
+    double *host_r2;  // optional host copy of ||r||^2 (pinned memory)
     struct L { Cx<T> al, om; };
     __device__ L local(int rhs) const { return {tc<T>(st[kAlpha * R + rhs]), tc<T>(st[kOmega * R + rhs])}; }
     // split form: every load of a trip is issued before the first store (the stores could
@@ -374,6 +375,7 @@ struct XROp {  // x += a p + w shat ; r = s - w t ; ||r||^2 ; <r0, r> ; beta
     __device__ void elem(long e, L l, double (&acc)[NA]) const { apply(e, load(e), l, acc); }
     __device__ void finish(int rr, const double (&tt)[NA]) const {
         st[kRnorm2 * R + rr] = {tt[0], 0.0};
+        if (host_r2) host_r2[rr] = tt[0];
         const C64 rho_new = {tt[1], tt[2]};
         st[kRhoNew * R + rr] = rho_new;
         // beta = ((alpha * rho_new) / omega) / rho (src/solver/bicgstab_solve.cu:350-374)
@@ -389,7 +391,7 @@ struct XROp {  // x += a p + w shat ; r = s - w t ; ||r||^2 ; <r0, r> ; beta
         st[kRho * R + rr] = rho_new;
     }
     __device__ XROp shifted(long off, int base) const {
-        return {x + off, r + off, p + off, shat + off, s + off, t + off, r0 + off, st + base, R};
+        return {x + off, r + off, p + off, shat + off, s + off, t + off, r0 + off, st + base, R, nullptr};
     }
 };
 
@@ -802,14 +804,14 @@ hipError_t launch_step_omega(C64 *st, const void *t, const void *sv, long n, int
 
 hipError_t launch_step_xr(void *x, void *r, const void *p, const void *shat, const void *sv,
                           const void *t, const void *r0, C64 *st, long n, int R, int prec,
-                          ReduceWork &w, hipStream_t s) {
+                          ReduceWork &w, hipStream_t s, double *host_r2) {
     QCU_PREC_DISPATCH(prec, {
         using CS = typename CxStore<typename PrecT<P>::S>::type;
         using T = typename PrecT<P>::T;
         XROp<CS, T> op{static_cast<CS *>(x), static_cast<CS *>(r), static_cast<const CS *>(p),
                        static_cast<const CS *>(shat), static_cast<const CS *>(sv),
                        static_cast<const CS *>(t),
-                       static_cast<const CS *>(r0), st, R};
+                       static_cast<const CS *>(r0), st, R, host_r2};
         return run_reduce(op, n, R, w, 2, s);
     })
 }
@@ -912,7 +914,7 @@ hipError_t seg_step_xr(void *x, void *r, const void *p, const void *sv, const vo
         using T = typename PrecT<P>::T;
         XROp<CS, T> op{static_cast<CS *>(x), static_cast<CS *>(r), static_cast<const CS *>(p),
                        static_cast<const CS *>(sv), static_cast<const CS *>(sv), static_cast<const CS *>(t),
-                       static_cast<const CS *>(r0), st, tab.Rtot};
+                       static_cast<const CS *>(r0), st, tab.Rtot, nullptr};
         QCU_HIP_TRY(run_seg_reduce(op, tab, w, s));
         hipLaunchKernelGGL(k_group_done, dim3(tab.G), dim3(64), 0, s, tab, st, done, iters);
         return hipGetLastError();

@@ -118,6 +118,8 @@ private:
     double *dn_ = nullptr;     // [4][R] norms
     double *dscale_ = nullptr; // [2][R] per-RHS scales (accumulation, new inner residual)
     double *h_ = nullptr;      // pinned host staging [8][R]
+    double *hr2_ = nullptr;    // [R] ||r||^2 of the iteration, written by its last kernel (pinned host memory)
+    hipEvent_t r2_ready_ = nullptr;
     double *part_ = nullptr;   // per-workgroup partial sums of the fused residual (mixed solves)
     long part_cap_ = 0;
     double *dotp_ = nullptr;   // per-workgroup partials of the Schur hops' inner products
