@@ -133,6 +133,9 @@ hipError_t seg_norm(double *res, const void *a, int prec, bool take_sqrt, const 
                     hipStream_t s);
 hipError_t seg_step_alpha(C64 *st, const void *r0, const void *v, int prec, const SegTab &tab, SegWork &w,
                           hipStream_t s);
+// alpha or omega of every running group from rows of partial sums (dslash_dots_rows)
+hipError_t seg_finish_alpha(C64 *st, const SegTab &tab, const SegRows &rows, const double *partials, hipStream_t s);
+hipError_t seg_finish_omega(C64 *st, const SegTab &tab, const SegRows &rows, const double *partials, hipStream_t s);
 hipError_t seg_step_s(void *sv, const void *r, const void *v, const C64 *st, int prec, const SegTab &tab,
                       hipStream_t s);
 hipError_t seg_step_omega(C64 *st, const void *t, const void *sv, int prec, const SegTab &tab, SegWork &w,

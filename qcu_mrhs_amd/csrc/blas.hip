@@ -473,6 +473,16 @@ __global__ __launch_bounds__(kFinishThreads) void k_reduce_seg_finish(Op op, Seg
     reduce_finish(op.shifted(off, base), nblk, R, blockIdx.x, partials + size_t(grp) * max_blocks * tab.Rmax * 4);
 }
 
+// The same from rows of partials left elsewhere
+template <class Op>
+__global__ __launch_bounds__(kFinishThreads) void k_finish_seg_rows(Op op, SegTab tab, SegRows rows,
+                                                                   const double *__restrict__ partials) {
+    int grp, R, base;
+    long off;
+    if (!seg_group(tab, grp, R, off, base) || int(blockIdx.x) >= R) return;
+    reduce_finish(op.shifted(off, base), rows.n[grp], R, blockIdx.x, partials + rows.off[grp]);
+}
+
 // Counts the iteration of every running group and raises its done flag once every RHS has
 // ||r||^2 <= st[kBnorm2] (the squared stopping threshold).
 __global__ __launch_bounds__(64) void k_group_done(SegTab tab, const C64 *__restrict__ st, int *done, int *iters) {
@@ -919,6 +929,26 @@ hipError_t seg_step_xr(void *x, void *r, const void *p, const void *sv, const vo
         hipLaunchKernelGGL(k_group_done, dim3(tab.G), dim3(64), 0, s, tab, st, done, iters);
         return hipGetLastError();
     })
+}
+
+namespace {
+template <class Op>
+hipError_t finish_seg_rows(const Op &op, const SegTab &tab, const SegRows &rows, const double *partials, hipStream_t s) {
+    if (!seg_ok(tab, nullptr)) return hipErrorInvalidValue;
+    int most = 1;
+    for (int k = 0; k < tab.G; ++k) most = std::max(most, rows.n[k]);
+    hipLaunchKernelGGL(k_finish_seg_rows<Op>, dim3(tab.Rmax, tab.G), dim3(finish_threads(most)), 0, s, op, tab, rows,
+                       partials);
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t seg_finish_alpha(C64 *st, const SegTab &tab, const SegRows &rows, const double *partials, hipStream_t s) {
+    return finish_seg_rows(AlphaOp<C64>{nullptr, nullptr, st, tab.Rtot}, tab, rows, partials, s);
+}
+
+hipError_t seg_finish_omega(C64 *st, const SegTab &tab, const SegRows &rows, const double *partials, hipStream_t s) {
+    return finish_seg_rows(OmegaOp<C64>{nullptr, nullptr, st, tab.Rtot}, tab, rows, partials, s);
 }
 
 hipError_t seg_step_s(void *sv, const void *r, const void *v, const C64 *st, int prec, const SegTab &tab,

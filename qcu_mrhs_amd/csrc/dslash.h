@@ -126,6 +126,14 @@ hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, i
 // `partials` holds dslash_dots_partials(g, Nc, R, prec) doubles.  Returns hipErrorNotSupported (and
 // launches nothing) when the launch chosen for these arguments has no such form (the lane kernel has both,
 // the 16-bit matrix-core kernel omega's without clover blocks); the caller then runs the separate reduction.
+// Rows that the finisher's one workgroup per RHS sums by itself: four per lane (20736 rows, 16 RHS: 72 us,
+// against 12 us through slices)
+constexpr int kMaxFinishRows = 4096;
+// The same on a batch (lane kernel, every running group in one launch), finished by seg_finish_alpha or
+// seg_finish_omega; false if a group's rows are more than one finishing pass takes
+bool dslash_dots_rows(const Geom &g, int Nc, int prec, const SegTab &tab, SegRows &rows);
+hipError_t launch_dslash_lane_dots_groups(const DslashArgs &a, DotsKind kind, const void *r0, const SegTab &tab,
+                                          const SegRows &rows, double *partials, int by, int bz, hipStream_t stream);
 long dslash_dots_partials(const Geom &g, int Nc, int R, int prec);
 hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0, double *partials, long cap,
                               Cx<double> *st, hipStream_t stream);

@@ -333,9 +333,6 @@ hipError_t launch_dslash_clover(const DslashArgs &a, hipStream_t stream) {
                                a.prec == kDouble ? kDouble : kSingle, stream);
 }
 
-// Rows that the finisher's one workgroup per RHS sums by itself: four per lane (20736 rows, 16 RHS: 72 us,
-// against 12 us through slices)
-constexpr int kMaxFinishRows = 4096;
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
 long dslash_dots_partials(const Geom &g, int Nc, int R, int prec) {

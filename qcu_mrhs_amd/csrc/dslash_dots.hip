@@ -48,21 +48,20 @@ __device__ __forceinline__ void put_row(double *part, int R, int r, const double
     for (int k = 0; k < kNumDots<KIND>; ++k) row[k] = q[k];
 }
 
-// out = xpay + coef D in, or with clover blocks A xpay + coef D in
+// out = xpay + coef D in, or with clover blocks A xpay + coef D in, from traversal position pos0 on
 template <typename S, int NC, int V, int KIND, bool CLOV>
-__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_dots(
-    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
-    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
-    const typename Arith<S>::C *__restrict__ r0, const Cx<typename Arith<S>::T> *__restrict__ blocks,
-    typename Arith<S>::T coef, int Vh, int R, int RV, int spb, int parity, const int *__restrict__ walk,
-    unsigned vec_bytes, double *__restrict__ part) {
+__device__ __forceinline__ void dots_body(typename Arith<S>::C *out, const typename Arith<S>::C *in,
+                                          const typename Arith<S>::C *gauge, const typename Arith<S>::C *xpay,
+                                          const typename Arith<S>::C *r0, const Cx<typename Arith<S>::T> *blocks,
+                                          typename Arith<S>::T coef, int Vh, int R, int RV, int spb, int pos0,
+                                          int parity, const int *walk, unsigned vec_bytes, double *part) {
     using T = typename Arith<S>::T;
     using C = typename Arith<S>::C;
     using RW = Raw<V * int(sizeof(C))>;
     using W = Vec<C, V>;
     using A = std::conditional_t<kSumFloat<S, KIND>, float, double>;
     constexpr int NA = kNumDots<KIND>, N = 4 * NC;
-    const int pos0 = xcd_remap(blockIdx.x, gridDim.x) * spb, ns = min(spb, Vh - pos0);
+    const int ns = min(spb, Vh - pos0);
     Cx<T> acc[4][NC][V];
     const Clover<S, NC> cl = clover_lds<S, NC>(blocks, dots_smem, spb);
     Place p;
@@ -129,6 +128,35 @@ __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_dots(
             put_row<KIND>(part, R, int(threadIdx.x) * V + i, row);
         }
     }
+}
+
+template <typename S, int NC, int V, int KIND, bool CLOV>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_dots(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
+    const typename Arith<S>::C *__restrict__ r0, const Cx<typename Arith<S>::T> *__restrict__ blocks,
+    typename Arith<S>::T coef, int Vh, int R, int RV, int spb, int parity, const int *__restrict__ walk,
+    unsigned vec_bytes, double *__restrict__ part) {
+    dots_body<S, NC, V, KIND, CLOV>(out, in, gauge, xpay, r0, blocks, coef, Vh, R, RV, spb,
+                                    xcd_remap(blockIdx.x, gridDim.x) * spb, parity, walk, vec_bytes, part);
+}
+
+// Every running group of a batch in one launch (blockIdx.y = group, SegTab layout)
+template <typename S, int NC, int KIND>
+__global__ __launch_bounds__(256, (kMinWaves<S, NC, 1>)) void k_dslash_dots_groups(
+    typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
+    const typename Arith<S>::C *__restrict__ gauge, const typename Arith<S>::C *__restrict__ xpay,
+    const typename Arith<S>::C *__restrict__ r0, typename Arith<S>::T coef, int Vh, int parity,
+    const int *__restrict__ walk, SegTab tab, SegRows rows, double *__restrict__ part) {
+    const int grp = blockIdx.y;
+    if (tab.done && tab.done[grp]) return;
+    const int nblk = rows.n[grp], R = tab.R[grp], spb = rows.sites[grp];
+    if (int(blockIdx.x) >= nblk) return;
+    const long off = tab.n * tab.base[grp];
+    const unsigned vec_bytes = unsigned(tab.n * R * long(sizeof(typename Arith<S>::C)));
+    dots_body<S, NC, 1, KIND, false>(out + off, in + off, gauge, xpay + off, r0 ? r0 + off : nullptr, nullptr, coef, Vh,
+                                     R, R, spb, xcd_remap(blockIdx.x, nblk) * spb, parity, walk, vec_bytes,
+                                     part + rows.off[grp]);
 }
 
 // Small lattices: a wavefront per direction, wavefront mu finishing spin mu (direction(), dslash_lane.h)
@@ -256,7 +284,77 @@ hipError_t launch_s(const DslashArgs &a, DotsKind kind, const void *r0, const Ge
     }
 }
 
+template <typename S, int NC>
+hipError_t launch_groups(const DslashArgs &a, DotsKind kind, const void *r0, const SegTab &seg, const SegRows &rows,
+                         const GeomTables &tab, double *part, hipStream_t stream) {
+    using C = typename Arith<S>::C;
+    constexpr int per_site = kSiteLds<S, NC>;
+    int nmax = 1, smax = 1;
+    for (int k = 0; k < seg.G; ++k) {
+        nmax = std::max(nmax, rows.n[k]);
+        smax = std::max(smax, rows.sites[k]);
+    }
+    auto k = kind == kDotsAlpha ? k_dslash_dots_groups<S, NC, kDotsAlpha> : k_dslash_dots_groups<S, NC, kDotsOmega>;
+    hipLaunchKernelGGL(k, dim3(nmax, seg.G), dim3(256), std::max(size_t(smax) * per_site, size_t(256) * 3 * 8), stream,
+                       static_cast<C *>(a.out), static_cast<const C *>(a.in), static_cast<const C *>(a.gauge),
+                       static_cast<const C *>(a.xpay), static_cast<const C *>(r0), typename Arith<S>::T(a.coef), a.g.Vh,
+                       a.parity, tab.walk, seg, rows, part);
+    return hipGetLastError();
+}
+
+template <typename S>
+hipError_t launch_groups_s(const DslashArgs &a, DotsKind kind, const void *r0, const SegTab &seg, const SegRows &rows,
+                           const GeomTables &tab, double *part, hipStream_t stream) {
+    switch (a.Nc) {
+        case 2: return launch_groups<S, 2>(a, kind, r0, seg, rows, tab, part, stream);
+        case 3: return launch_groups<S, 3>(a, kind, r0, seg, rows, tab, part, stream);
+        case 4: return launch_groups<S, 4>(a, kind, r0, seg, rows, tab, part, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+int site_lds(int Nc, int prec) {
+    const auto of = [&](auto nc) {
+        constexpr int NC = decltype(nc)::value;
+        return prec == kDouble ? kSiteLds<double, NC> : prec == kSingle ? kSiteLds<float, NC> : kSiteLds<__half, NC>;
+    };
+    return Nc == 2   ? of(std::integral_constant<int, 2>{})
+           : Nc == 3 ? of(std::integral_constant<int, 3>{})
+                     : of(std::integral_constant<int, 4>{});
+}
+
 }  // namespace
+
+bool dslash_dots_rows(const Geom &g, int Nc, int prec, const SegTab &tab, SegRows &rows) {
+    if (tab.G < 1 || tab.G > kMaxGroups || Nc > 4) return false;
+    rows = SegRows{};
+    for (int k = 0; k < tab.G; ++k) {
+        if (tab.R[k] < 1 || tab.R[k] > 256 || !dslash_lane_supported(g, Nc, tab.R[k], prec)) return false;
+        rows.sites[k] = std::min(std::max(1, 256 / tab.R[k]), std::max(1, 40960 / site_lds(Nc, prec)));
+        rows.n[k] = div_up(g.Vh, rows.sites[k]);
+        if (rows.n[k] > kMaxFinishRows) return false;
+        rows.off[k] = rows.total;
+        rows.total += long(rows.n[k]) * tab.R[k] * 4;
+    }
+    return true;
+}
+
+hipError_t launch_dslash_lane_dots_groups(const DslashArgs &a, DotsKind kind, const void *r0, const SegTab &tab,
+                                          const SegRows &rows, double *partials, int by, int bz, hipStream_t stream) {
+    SegRows check;
+    if (!dslash_dots_rows(a.g, a.Nc, a.prec, tab, check) || check.total != rows.total || !partials || a.dagger ||
+        !a.xpay || by <= 0 || bz <= 0 || a.g.L[1] % by || a.g.L[2] % bz)
+        return hipErrorInvalidValue;
+    GeomTables g;
+    QCU_HIP_TRY(geom_tables(a.g, by, bz, g, stream));
+    switch (a.prec) {
+        case kDouble: return launch_groups_s<double>(a, kind, r0, tab, rows, g, partials, stream);
+        case kSingle: return launch_groups_s<float>(a, kind, r0, tab, rows, g, partials, stream);
+        case kHalf: return launch_groups_s<__half>(a, kind, r0, tab, rows, g, partials, stream);
+        case kBF16: return launch_groups_s<__hip_bfloat16>(a, kind, r0, tab, rows, g, partials, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
 
 hipError_t launch_dslash_lane_dots(const DslashArgs &a, const DslashTune &t, DotsKind kind, const void *r0,
                                    double *partials, hipStream_t stream, int &nblk) {

@@ -102,6 +102,8 @@ private:
     double *dn_ = nullptr, *scale_ = nullptr;
     int *done_ = nullptr, *odone_ = nullptr, *iters_ = nullptr;
     double *h_ = nullptr;  // pinned staging
+    double *dotp_ = nullptr;  // rows of partial sums of the fused inner products (null: separate reductions)
+    SegRows rows_;
     SegWork work_;
 };
 

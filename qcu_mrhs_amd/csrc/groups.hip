@@ -41,7 +41,8 @@ GroupSolver::GroupSolver(const Geom &g, int Nc, const std::vector<int> &Rs)
 GroupSolver::~GroupSolver() {
     for (void *p : {b_, x_, bp_, r64_, t64_, u64_, r_, r0_, p_, v_, s_, t_, tmp_, xl_, static_cast<void *>(st_),
                     static_cast<void *>(ones_), static_cast<void *>(dn_), static_cast<void *>(scale_),
-                    static_cast<void *>(done_), static_cast<void *>(odone_), static_cast<void *>(iters_)})
+                    static_cast<void *>(done_), static_cast<void *>(odone_), static_cast<void *>(iters_),
+                    static_cast<void *>(dotp_)})
         if (p) (void)hipFree(p);
     if (h_) (void)hipHostFree(h_);
     seg_work_free(work_);
@@ -82,6 +83,12 @@ hipError_t GroupSolver::ensure(int prec) {
             *p = gmalloc(nR * 2 * prec_bytes(prec), err);
         }
         if (err != hipSuccess) return err;
+        if (dotp_) (void)hipFree(dotp_);
+        dotp_ = nullptr;
+        if (dslash_dots_rows(g_, Nc_, prec, tab_, rows_)) {
+            dotp_ = static_cast<double *>(gmalloc(sizeof(double) * size_t(rows_.total), err));
+            if (err != hipSuccess) return err;
+        }
         lo_prec_ = prec;
         // default traversal tile for the wave kernel at this site size
         DslashArgs a{nullptr, nullptr, nullptr, nullptr, 1.0, g_, Nc_, 16, 1, 0, prec};
@@ -302,12 +309,27 @@ hipError_t GroupSolver::iteration(const void *glo, int P, double kappa, hipStrea
     const SegTab t = tab_with(done_);
     const double k2 = -kappa * kappa;
     QCU_HIP_TRY(dslash(tmp_, p_, glo, P, 0, nullptr, 1.0, t, s));
-    QCU_HIP_TRY(dslash(v_, tmp_, glo, P, 1, p_, k2, t, s));
-    QCU_HIP_TRY(seg_step_alpha(st_, r0_, v_, P, t, work_, s));
+    // the lane kernel forms the inner products of a step in its second hop
+    const bool dots = variant_ == kDslashLaneRhs && dotp_;
+    const auto hop_dots = [&](DotsKind kind, void *out, const void *x) -> hipError_t {
+        DslashArgs a{out, tmp_, glo, x, k2, g_, Nc_, 0, 1, 0, P};
+        QCU_HIP_TRY(launch_dslash_lane_dots_groups(a, kind, r0_, t, rows_, dotp_, lane_by_[0], lane_bz_[0], s));
+        return kind == kDotsAlpha ? seg_finish_alpha(st_, t, rows_, dotp_, s) : seg_finish_omega(st_, t, rows_, dotp_, s);
+    };
+    if (dots) {
+        QCU_HIP_TRY(hop_dots(kDotsAlpha, v_, p_));
+    } else {
+        QCU_HIP_TRY(dslash(v_, tmp_, glo, P, 1, p_, k2, t, s));
+        QCU_HIP_TRY(seg_step_alpha(st_, r0_, v_, P, t, work_, s));
+    }
     QCU_HIP_TRY(seg_step_s(s_, r_, v_, st_, P, t, s));
     QCU_HIP_TRY(dslash(tmp_, s_, glo, P, 0, nullptr, 1.0, t, s));
-    QCU_HIP_TRY(dslash(t_, tmp_, glo, P, 1, s_, k2, t, s));
-    QCU_HIP_TRY(seg_step_omega(st_, t_, s_, P, t, work_, s));
+    if (dots) {
+        QCU_HIP_TRY(hop_dots(kDotsOmega, t_, s_));
+    } else {
+        QCU_HIP_TRY(dslash(t_, tmp_, glo, P, 1, s_, k2, t, s));
+        QCU_HIP_TRY(seg_step_omega(st_, t_, s_, P, t, work_, s));
+    }
     QCU_HIP_TRY(seg_step_xr(xl_, r_, p_, s_, t_, r0_, st_, done_, iters_, P, t, work_, s));
     QCU_HIP_TRY(seg_step_p(p_, r_, v_, st_, P, t, s));
     return hipSuccess;

@@ -66,6 +66,14 @@ struct SegTab {
     const int *done = nullptr;     // device flags [G]; null = every group active
 };
 
+// Rows of partial sums that a batch's kernel leaves per group: n[g] rows of R[g] x 4 doubles from off[g] on
+struct SegRows {
+    int n[kMaxGroups] = {};
+    int sites[kMaxGroups] = {};    // lattice sites per row
+    long off[kMaxGroups] = {};
+    long total = 0;                // doubles over all groups
+};
+
 inline Geom make_geom(const int L[4]) {
     Geom g;
     for (int i = 0; i < 4; ++i) g.L[i] = L[i];
