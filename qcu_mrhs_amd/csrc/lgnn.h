@@ -110,7 +110,7 @@ private:
                        const Cx<float> *stencil = nullptr);
     // gradient of a loss whose derivative with respect to the network output N w is dphi (FP32 odd fields)
     hipError_t accumulate_grad(const void *w, const void *dphi, hipStream_t s);
-    hipError_t tables(GeomTables &tab, hipStream_t s) const;  // walk table in the FP32 hop's traversal order
+    hipError_t tables(GeomTables &tab, int prec, hipStream_t s) const;  // walk table in the traversal order of that storage's hop
     // FP32 odd Schur operator with the FP32 gauge copy: out = A in (dagger: A^+)
     hipError_t schur32(void *out, const void *in, double kappa, int dagger, hipStream_t s);
     hipError_t ensure_power(int K, hipStream_t s);
