@@ -81,8 +81,8 @@ __global__ __launch_bounds__(256, ORD ? 2 : (kMinWaves<S, NC, V>)) void k_dslash
 
 // With the clover blocks of the output sites: out = A x + coef D in, or (x null) out = A (coef D in + xpay).
 // The hop's sums never leave the registers in between; a separate pass over the vector reads and writes it
-// once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 57 us, FP64 185 -> 143 us against hop and pass; FP32, 5 RHS, at
-// 20 x 14 x 10 x 18 34 -> 29 us).  Half of what is left over the bare hop is the blocks' 72 LDS reads per lane.
+// once more (16^3 x 32, SU(3), 12 RHS: FP16 64 -> 47.5 us, FP64 185 -> 134 us against hop and pass).  The
+// blocks' LDS reads and products are most of what is left over the bare hop (35 us in FP16).
 template <typename S, int NC, int V, bool DAG>
 __global__ __launch_bounds__(256, (kMinWaves<S, NC, V>)) void k_dslash_lane_clover(
     typename Arith<S>::C *__restrict__ out, const typename Arith<S>::C *__restrict__ in,
