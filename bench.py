@@ -562,8 +562,8 @@ def main():
     dom = {2: "double", 1: "single", 0: "half", 4: "bf16"}[head_prec]
     if dom not in dslash:
         dom = next(iter(dslash))
-    kname = {"double": "k_dslash_wave<double>", "single": "k_dslash_wave<float>",
-             "half": "k_dslash_mfma<__half>", "bf16": "k_dslash_mfma<__hip_bfloat16>"}[dom]
+    kname = {"double": "k_dslash_lane<double>", "single": "k_dslash_lane<float>",
+             "half": "k_dslash_lane<__half>", "bf16": "k_dslash_lane<__hip_bfloat16>"}[dom]
     roof = {"bound": "hbm", "achieved": dslash[dom]["GBps"], "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": dslash[dom]["frac_of_8TBps"],
             "traffic": measured_traffic(args.workload, dom, args.dslash_variant),

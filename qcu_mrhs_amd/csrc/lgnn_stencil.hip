@@ -21,7 +21,7 @@
 //
 // Measured at 16^3 x 32, 16 RHS (SU(3)): k_lgnn_mix32 342 us (transport to 8 fields and a
 // VALU product before: 666 us), k_lgnn_gram 583 us (transport and a VALU FP64 sum
-// through LDS before: 2960 us); a gradient pass of power 2 15.1 -> 5.97 ms.
+// through LDS before: 2960 us); a gradient pass of power 3 15.1 -> 5.97 ms.
 #include <algorithm>
 
 #include "dslash_common.h"
