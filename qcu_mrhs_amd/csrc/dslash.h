@@ -76,6 +76,8 @@ hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStrea
 bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
 void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
 // workgroups of a launch with one RHS per lane (rows of partial sums of the fused forms below); Nc <= 4
+// the lane kernel gives each direction a wavefront on this lattice
+bool dslash_lane_split(const Geom &g, int R);
 // the clover forms of the lane kernel replace the separate clover pass for these arguments and shape
 bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t);
 int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec);

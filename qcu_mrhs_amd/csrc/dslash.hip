@@ -252,6 +252,15 @@ int automatic_variant(const DslashArgs &a) {
     const bool fits16 = double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 &&
                         double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;  // what the matrix-core kernel addresses
     if (lane && fits16 && (a.R % 4 == 0 || a.R > 16)) return kDslashLaneRhs;
+    // Up to 3 right-hand sides leave 13 of the matrix cores' 16 columns empty.  From 8192 sites (8^3 x 16 with
+    // 4096: even) a lane per site is faster where the lattice takes a wavefront per direction (FP16 16^3 x 32,
+    // SU(3): 13 against 45 us at 1, 21 / 46 at 2; beyond it 24^4, SU(3): 118 / 89 at 1; SU(4) 16^4: 13 / 25 at 1,
+    // but 21 / 25 at 3, which a solve does not see) and beyond it where the rows of a site still share lines
+    // (SU(2): 24^3 x 48 80 / 127 at 1, 84 / 128 at 3; SU(3) at 3: 24^4 82 / 88, 24^3 x 48 145 / 205)
+    const bool split = dslash_lane_split(a.g, a.R);
+    if (lane && fits16 && a.R <= 3 && a.g.Vh >= 8192 &&
+        (a.Nc == 2 || (a.Nc == 3 && (split || a.R == 3)) || (a.Nc == 4 && split && a.R == 1)))
+        return kDslashLaneRhs;
     return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
 }
 }  // namespace

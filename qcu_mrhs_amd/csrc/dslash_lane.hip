@@ -427,6 +427,8 @@ void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz) 
     }
 }
 
+bool dslash_lane_split(const Geom &g, int R) { return split_over_directions(g.Vh, R); }
+
 bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t) {
     return t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec) && !a.keep_order &&
            !split_over_directions(a.g.Vh, a.R);
