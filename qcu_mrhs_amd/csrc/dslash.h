@@ -15,8 +15,10 @@ enum DslashVariant : int {
     kDslashLaneRhs = 1,   // one lane per (site, rhs), all 8 hops per lane; tiled traversal for Nc <= 4
     kDslashWaveSite = 2,  // one wavefront per site: lanes = 16 rhs x 4 dimensions (VALU)
     kDslashMfma = 3,      // one wavefront per site on MFMA (FP16 / BF16 storage)
-    kDslashLds = 4        // MFMA with the input rows staged in LDS: one workgroup per 4-site segment of an
+    kDslashLds = 4,       // MFMA with the input rows staged in LDS: one workgroup per 4-site segment of an
                           // x-row sweeping `spw` consecutive t (FP16 / BF16, Nc <= 4); chosen explicitly
+    kDslashLane16 = 5     // kDslashLaneRhs in FP16 / BF16, Nc <= 4, with the projected spinors rounded to the
+                          // storage type and 16-bit dot products, as kDslashMfma (kDslashLaneRhs: all in FP32)
 };
 
 // Launch shape of the wave-per-site kernels.
@@ -75,11 +77,16 @@ bool dslash_mfma_supported(int Nc, int prec);
 hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream);
 bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
 void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
-// workgroups of a launch with one RHS per lane (rows of partial sums of the fused forms below); Nc <= 4
 // the lane kernel gives each direction a wavefront on this lattice
 bool dslash_lane_split(const Geom &g, int R);
+// the lane kernel that t names has the forms with clover blocks and inner products (in 16 bits: kDslashLane16)
+inline bool dslash_lane_forms(const DslashArgs &a, const DslashTune &t) {
+    const bool bits16 = a.prec == kHalf || a.prec == kBF16;
+    return t.variant == (bits16 ? kDslashLane16 : kDslashLaneRhs) && dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
+}
 // the clover forms of the lane kernel replace the separate clover pass for these arguments and shape
 bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t);
+// workgroups of a launch with one RHS per lane (rows of partial sums of the fused forms below); Nc <= 4
 int dslash_lane_blocks(const Geom &g, int Nc, int R, int prec);
 hipError_t launch_dslash_lane_residual(const DslashArgs &a, const DslashTune &t, const void *b, void *lo, int lo_prec,
                                        const double *scale, double *partials, int &nblk, hipStream_t stream);

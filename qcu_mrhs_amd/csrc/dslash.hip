@@ -233,6 +233,11 @@ std::vector<std::pair<std::array<int, 7>, DslashTune>> dslash_tuned_entries() {
 }
 
 namespace {
+// what the 16-bit matrix-core kernel addresses
+bool fits_mfma16(const DslashArgs &a) {
+    return double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 && double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;
+}
+
 // Kernel chosen for a hop that names none.
 int automatic_variant(const DslashArgs &a) {
     const bool lane = dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
@@ -249,9 +254,8 @@ int automatic_variant(const DslashArgs &a) {
     // pieces (24^3 x 48, SU(3) FP16: 103 against 179 us matrix cores at 8 RHS, 188 / 207 at 12,
     // 213 / 245 at 16, 374 / 759 at 32) or needs a second 16-wide matrix-core chunk (370 / 536 at 17);
     // otherwise its loads straddle those pieces (190 / 175 at 6, 220 / 191 at 10)
-    const bool fits16 = double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 &&
-                        double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;  // what the matrix-core kernel addresses
-    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16)) return kDslashLaneRhs;
+    const bool fits16 = fits_mfma16(a);
+    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16)) return kDslashLane16;
     // Up to 3 right-hand sides leave 13 of the matrix cores' 16 columns empty.  From 8192 sites (8^3 x 16 with
     // 4096: even) a lane per site is faster where the lattice takes a wavefront per direction (FP16 16^3 x 32,
     // SU(3): 13 against 45 us at 1, 21 / 46 at 2; beyond it 24^4, SU(3): 118 / 89 at 1; SU(4) 16^4: 13 / 25 at 1,
@@ -260,14 +264,20 @@ int automatic_variant(const DslashArgs &a) {
     const bool split = dslash_lane_split(a.g, a.R);
     if (lane && fits16 && a.R <= 3 && a.g.Vh >= 8192 &&
         (a.Nc == 2 || (a.Nc == 3 && (split || a.R == 3)) || (a.Nc == 4 && split && a.R == 1)))
-        return kDslashLaneRhs;
+        return kDslashLane16;
     return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
 }
 }  // namespace
 
 DslashTune dslash_fill_defaults(const DslashArgs &a, DslashTune t) {
     if (t.variant == kDslashAuto) t.variant = automatic_variant(a);
-    if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)) {
+    if (t.variant == kDslashLane16) {
+        if (a.prec == kSingle || a.prec == kDouble) t.variant = kDslashLaneRhs;
+        else if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec))
+            t.variant = dslash_mfma_supported(a.Nc, a.prec) && fits_mfma16(a) ? kDslashMfma : kDslashWaveSite;
+    }
+    if ((t.variant == kDslashLaneRhs || t.variant == kDslashLane16) &&
+        dslash_lane_supported(a.g, a.Nc, a.R, a.prec)) {
         dslash_lane_tile(a.g, a.Nc, a.R, a.prec, t.by, t.bz);
         return t;
     }
@@ -311,7 +321,8 @@ hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
     const DslashTune t = dslash_resolve(a);
     if (t.variant == kDslashWaveSite) return launch_dslash_wave(a, t, stream);
     if (t.variant == kDslashLds) return launch_dslash_lds(a, t, stream);
-    if (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec))
+    if (t.variant == kDslashLane16 ||
+        (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)))
         return launch_dslash_lane(a, t, stream);
     if (t.variant == kDslashMfma)
         return (a.prec == kSingle || a.prec == kDouble) ? launch_dslash_mfma32(a, t, stream)
@@ -359,7 +370,7 @@ hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0
         !(a.clover ? a.clover_in : a.xpay) || (kind == kDotsAlpha && !r0) || a.R > kReduceThreads)
         return hipErrorNotSupported;
     const DslashTune t = dslash_resolve(a);
-    const bool lane = t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
+    const bool lane = dslash_lane_forms(a, t);
     const bool mfma = t.variant == kDslashMfma && (a.prec == kHalf || a.prec == kBF16) && kind == kDotsOmega && !a.clover;
     if ((!lane && !mfma) || (a.clover && !dslash_lane_clover_fused(a, t))) return hipErrorNotSupported;
     if (cap < dslash_dots_partials(a.g, a.Nc, a.R, a.prec)) return hipErrorInvalidValue;

@@ -1,5 +1,6 @@
-// dslash_lane.hip -- lane-per-(site, RHS) Wilson hopping term (variant
-// kDslashLaneRhs, dslash_lane.h), every storage precision, Nc <= 4.
+// dslash_lane.hip -- lane-per-(site, RHS) Wilson hopping term (variants
+// kDslashLaneRhs and, in 16 bits, kDslashLane16; dslash_lane.h), every storage
+// precision, Nc <= 4.
 //
 // What bounds it: the bytes that miss the XCD's L2 (FP64, FP32: 4.9 and 2.2 GB
 // per hop at 24^3 x 48, 16 RHS, at 6-7 TB/s, against 2.4 and 1.2 GB that the
@@ -361,7 +362,9 @@ hipError_t launch_split(const DslashArgs &a, const DslashTune &t, hipStream_t st
 
 template <typename S, int NC, int V>
 hipError_t launch_dag(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
-    if (a.clover)
+    if constexpr (kWide<S>) {
+        if (a.clover) return hipErrorInvalidValue;
+    } else if (a.clover)
         return a.dagger ? launch_clover_v<S, NC, V, true>(a, t, stream) : launch_clover_v<S, NC, V, false>(a, t, stream);
     return a.dagger ? launch_v<S, NC, V, true>(a, t, stream) : launch_v<S, NC, V, false>(a, t, stream);
 }
@@ -430,19 +433,19 @@ void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz) 
 bool dslash_lane_split(const Geom &g, int R) { return split_over_directions(g.Vh, R); }
 
 bool dslash_lane_clover_fused(const DslashArgs &a, const DslashTune &t) {
-    return t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec) && !a.keep_order &&
-           !split_over_directions(a.g.Vh, a.R);
+    return dslash_lane_forms(a, t) && !a.keep_order && !split_over_directions(a.g.Vh, a.R);
 }
 
 hipError_t launch_dslash_lane(const DslashArgs &a, const DslashTune &t, hipStream_t stream) {
     if (!dslash_lane_supported(a.g, a.Nc, a.R, a.prec) || t.by <= 0 || t.bz <= 0 || a.g.L[1] % t.by ||
         a.g.L[2] % t.bz)
         return hipErrorInvalidValue;
+    const bool wide = t.variant == kDslashLaneRhs;
     switch (a.prec) {
         case kDouble: return launch_s<double>(a, t, stream);
         case kSingle: return launch_s<float>(a, t, stream);
-        case kHalf: return launch_s<__half>(a, t, stream);
-        case kBF16: return launch_s<__hip_bfloat16>(a, t, stream);
+        case kHalf: return wide ? launch_s<WideHalf>(a, t, stream) : launch_s<__half>(a, t, stream);
+        case kBF16: return wide ? launch_s<WideBf16>(a, t, stream) : launch_s<__hip_bfloat16>(a, t, stream);
         default: return hipErrorInvalidValue;
     }
 }

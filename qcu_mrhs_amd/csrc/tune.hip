@@ -116,11 +116,12 @@ hipError_t dslash_autotune(const int L[4], int Nc, int R, int prec, int reps, Ds
         }
     }
     add(kDslashLaneRhs, 0, 0, 0);
+    add(kDslashLane16, 0, 0, 0);
     if (dslash_lane_supported(g, Nc, R, prec))  // its traversal tiles of 256 to 1536 sites per slice
         for (int by : bys)
             for (int bz : bzs)
                 if (by * bz * g.Lxh >= 256 && by * bz * g.Lxh <= 1536 && by <= 2 * bz && bz <= 2 * by)
-                    add(kDslashLaneRhs, by, bz, 0);
+                    add(kDslashLane16, by, bz, 0);
     // (the LDS-staged kernel, kDslashLds, is not a candidate: on the synthetic fill timed here it
     // runs up to 14 % faster than on physical fields, enough to win a pick it then loses)
     auto time_shape = [&](const DslashTune &t, double &us) -> hipError_t {
@@ -205,7 +206,7 @@ hipError_t dslash_tune_load(const char *path, int &n_loaded) {
         int v[11];
         if (sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6],
                    &v[7], &v[8], &v[9], &v[10]) != 11 ||
-            v[7] < kDslashLaneRhs || v[7] > kDslashLds || v[8] < 0 || v[9] < 0 || v[10] < -64 ||
+            v[7] < kDslashLaneRhs || v[7] > kDslashLane16 || v[8] < 0 || v[9] < 0 || v[10] < -64 ||
             (v[10] < 0 && v[7] != kDslashMfma) ||
             !dslash_supported(v[4], v[5])) {
             err = hipErrorInvalidValue;
