@@ -79,6 +79,8 @@ bool dslash_lane_supported(const Geom &g, int Nc, int R, int prec);
 void dslash_lane_tile(const Geom &g, int Nc, int R, int prec, int &by, int &bz);
 // the lane kernel gives each direction a wavefront on this lattice
 bool dslash_lane_split(const Geom &g, int R);
+// kDslashLaneRhs runs the general kernel (dslash.hip), which has no tile, for this shape
+bool dslash_general_faster(const DslashArgs &a);
 // the lane kernel that t names has the forms with clover blocks and inner products (in 16 bits: kDslashLane16)
 inline bool dslash_lane_forms(const DslashArgs &a, const DslashTune &t) {
     const bool bits16 = a.prec == kHalf || a.prec == kBF16;

@@ -10,9 +10,10 @@
 // This file holds the dispatcher and the general lane-per-(site, rhs) VALU
 // kernel: R lanes of one site read R consecutive complex numbers for every
 // (spin, colour); the link is a broadcast load shared by those lanes.  It
-// serves variant kDslashLaneRhs for Nc = 8 and for vectors of 4 GiB and more;
-// the one for Nc <= 4 is in dslash_lane.hip.  The wave-per-site kernels live in
-// dslash_wave.hip (VALU) and dslash_mfma.hip (matrix cores).  Every variant has an optional epilogue
+// serves variant kDslashLaneRhs for Nc = 8, for vectors of 4 GiB and more and
+// for few right-hand sides on large lattices (dslash_general_faster); the one for the
+// other shapes of Nc <= 4 is in dslash_lane.hip.  The wave-per-site kernels live
+// in dslash_wave.hip (VALU) and dslash_mfma.hip (matrix cores).  Every variant has an optional epilogue
 // out = x + coef * D psi (Schur operator, full-lattice M, source preparation).
 #include <algorithm>
 #include <array>
@@ -315,6 +316,28 @@ DslashTune dslash_fill_defaults(const DslashArgs &a, DslashTune t) {
     return t;
 }
 
+// kDslashLaneRhs, Nc <= 4: the general kernel of this file instead of the one of dslash_lane.hip.  There a
+// workgroup holds the links of all its sites in LDS, so with few right-hand sides LDS, not registers, limits
+// the wavefronts on a compute unit.  24^3 x 48, general against lane kernel: SU(3) 1 RHS FP16 54 / 207,
+// FP32 76 / 235, FP64 270 / 534 us; 2 RHS 82 / 153, 112 / 189, 307 / 354 (but 158 / 152 at 24^4, SU(2) 137 /
+// 127); FP32 147 / 177 at 3 but 174 / 172 at 4, FP64 397 / 282 at 3; SU(4) FP16 195 / 261 at 3, 309 / 362 at 6, 262 / 249 at 8, BF16 258 / 259 at 3, 287 /
+// 209 at 4 (the general kernel spills there).  In the cache FP32 gains up to 5 (16^3 x 32, SU(3) 38 / 48 at 5).
+// A wavefront per direction (dslash_lane_split) is better until the lattice fills the GPU without it (8^4, 1
+// RHS, FP32 7.9 / 4.9, FP64 13.1 / 6.0 us; 16^3 x 32 14.1 / 20.3, 24.2 / 39.6; FP16 16^3 x 24 9.9 / 9.3,
+// 16^3 x 32 10.5 / 11.2).
+bool dslash_general_faster(const DslashArgs &a) {
+    if (a.keep_order || a.Nc > 4) return false;
+    const bool split = dslash_lane_split(a.g, a.R);
+    const long sites = a.g.Vh, lanes = sites * a.R;
+    if (a.prec == kDouble) {
+        if (split || a.R != 2) return a.R == 1 && (!split || lanes >= 49152);
+        return a.Nc == 4 || (a.Nc == 3 && sites > 131072);
+    }
+    if (a.prec == kSingle) return split ? a.R <= 2 && lanes >= 49152 : a.R <= 3 || (a.R <= 5 && sites <= 65536);
+    const bool spills = a.prec == kBF16 && a.Nc == 4;
+    return split ? a.R <= 2 && sites >= 65536 && !spills : a.R <= (spills ? 3 : 7);
+}
+
 hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
     if (!dslash_supported(a.Nc, a.R)) return hipErrorInvalidValue;
     if (a.g.Vh <= 0) return hipSuccess;
@@ -322,7 +345,7 @@ hipError_t launch_dslash(const DslashArgs &a, hipStream_t stream) {
     if (t.variant == kDslashWaveSite) return launch_dslash_wave(a, t, stream);
     if (t.variant == kDslashLds) return launch_dslash_lds(a, t, stream);
     if (t.variant == kDslashLane16 ||
-        (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec)))
+        (t.variant == kDslashLaneRhs && dslash_lane_supported(a.g, a.Nc, a.R, a.prec) && !dslash_general_faster(a)))
         return launch_dslash_lane(a, t, stream);
     if (t.variant == kDslashMfma)
         return (a.prec == kSingle || a.prec == kDouble) ? launch_dslash_mfma32(a, t, stream)

@@ -117,7 +117,8 @@ hipError_t dslash_autotune(const int L[4], int Nc, int R, int prec, int reps, Ds
     }
     add(kDslashLaneRhs, 0, 0, 0);
     add(kDslashLane16, 0, 0, 0);
-    if (dslash_lane_supported(g, Nc, R, prec))  // its traversal tiles of 256 to 1536 sites per slice
+    const bool bits16 = prec == kHalf || prec == kBF16;
+    if (dslash_lane_supported(g, Nc, R, prec) && (bits16 || !dslash_general_faster(base)))  // its traversal tiles of 256 to 1536 sites per slice
         for (int by : bys)
             for (int bz : bzs)
                 if (by * bz * g.Lxh >= 256 && by * bz * g.Lxh <= 1536 && by <= 2 * bz && bz <= 2 * by)
