@@ -331,7 +331,7 @@ bool dslash_general_faster(const DslashArgs &a) {
     const long sites = a.g.Vh, lanes = sites * a.R;
     if (a.prec == kDouble) {
         if (split || a.R != 2) return a.R == 1 && (!split || lanes >= 49152);
-        return a.Nc == 4 || (a.Nc == 3 && sites > 131072);
+        return a.Nc == 4 || (a.Nc == 3 && sites > 200000);
     }
     if (a.prec == kSingle) return split ? a.R <= 2 && lanes >= 49152 : a.R <= 3 || (a.R <= 5 && sites <= 65536);
     const bool spills = a.prec == kBF16 && a.Nc == 4;
