@@ -4,7 +4,7 @@
 //
 // A separate reduction reads the stored vector and the other one again (two vectors of traffic and a
 // launch); here the result is in registers, and s is the hop's own xpay vector.  The sums are of the
-// stored (rounded) values, in FP64 (omega in 16 bits: FP32 over a lane's 4 NC entries), over a
+// stored (rounded) values, in FP64 for every storage type as in the separate reductions, over a
 // workgroup's sites in order, then over workgroups by the reductions' finisher.
 // Hop and reduction before -> now: alpha FP16 24^3 x 48, 16 RHS 319 -> 263 us, FP32 16^3 x 32, 12 RHS 102 ->
 // 93 us; omega FP32 94 -> 74 us (16 bits had it); FP64 8^4, 4 RHS 9.6 -> 7.1 and 10.1 -> 7.9 us.
@@ -21,15 +21,13 @@ using namespace lane;
 
 extern __shared__ __align__(16) unsigned char dots_smem[];
 
-template <typename S, int KIND>
-constexpr bool kSumFloat = KIND == kDotsOmega && !std::is_same<S, float>::value && !std::is_same<S, double>::value;
 template <int KIND>
 constexpr int kNumDots = KIND == kDotsOmega ? 3 : 2;
 
 // KIND's products of one stored entry o with u (alpha: of r0, omega: of s)
-template <int KIND, typename A, typename C>
-__device__ __forceinline__ void add_products(A (&q)[kNumDots<KIND>], const C &o, const C &u) {
-    const Cx<A> t = load_cx<A>(&o), w = load_cx<A>(&u);
+template <int KIND, typename C>
+__device__ __forceinline__ void add_products(double (&q)[kNumDots<KIND>], const C &o, const C &u) {
+    const Cx<double> t = load_cx<double>(&o), w = load_cx<double>(&u);
     if constexpr (KIND == kDotsAlpha) {  // <r0, v>
         q[0] = fma(w.re, t.re, fma(w.im, t.im, q[0]));
         q[1] = fma(w.re, t.im, fma(-w.im, t.re, q[1]));
@@ -59,7 +57,6 @@ __device__ __forceinline__ void dots_body(typename Arith<S>::C *out, const typen
     using C = typename Arith<S>::C;
     using RW = Raw<V * int(sizeof(C))>;
     using W = Vec<C, V>;
-    using A = std::conditional_t<kSumFloat<S, KIND>, float, double>;
     constexpr int NA = kNumDots<KIND>, N = 4 * NC;
     const int ns = min(spb, Vh - pos0);
     Cx<T> acc[4][NC][V];
@@ -71,11 +68,11 @@ __device__ __forceinline__ void dots_body(typename Arith<S>::C *out, const typen
     else
         p = hops<S, NC, V, false, false, kAhead<S, NC>>(acc, dots_smem, in, gauge, Vh, R, RV, spb, pos0, parity, walk,
                                                         vec_bytes);
-    A q[V][NA];
+    double q[V][NA];
 #pragma unroll
     for (int i = 0; i < V; ++i)
 #pragma unroll
-        for (int k = 0; k < NA; ++k) q[i][k] = A(0);
+        for (int k = 0; k < NA; ++k) q[i][k] = 0.0;
     if (p.active) {
         const unsigned rb = unsigned(R) * unsigned(sizeof(C));
         const auto r_out = rsrc(out, vec_bytes), r_x = rsrc(xpay, vec_bytes), r_r = rsrc(r0, vec_bytes);
@@ -117,7 +114,7 @@ __device__ __forceinline__ void dots_body(typename Arith<S>::C *out, const typen
 #pragma unroll
     for (int i = 0; i < V; ++i)
 #pragma unroll
-        for (int k = 0; k < NA; ++k) w[k][i] = double(q[i][k]);
+        for (int k = 0; k < NA; ++k) w[k][i] = q[i][k];
     sum_sites<NA, V>(w, reinterpret_cast<double *>(dots_smem), p, RV, ns);
     if (int(threadIdx.x) < RV) {
 #pragma unroll
@@ -169,7 +166,6 @@ __global__ __launch_bounds__(256) void k_dslash_dots_split(
     using T = typename Arith<S>::T;
     using C = typename Arith<S>::C;
     using RW = Raw<int(sizeof(C))>;
-    using A = std::conditional_t<kSumFloat<S, KIND>, float, double>;
     constexpr int NA = kNumDots<KIND>;
     auto *sums = reinterpret_cast<Cx<T> *>(dots_smem);
     const int lane = threadIdx.x & 63;
@@ -191,9 +187,9 @@ __global__ __launch_bounds__(256) void k_dslash_dots_split(
         if constexpr (KIND == kDotsAlpha) u[c] = __builtin_bit_cast(C, RW::load(r_r, vo, unsigned(c) * rb));
     }
     __syncthreads();
-    A q[NA];
+    double q[NA];
 #pragma unroll
-    for (int k = 0; k < NA; ++k) q[k] = A(0);
+    for (int k = 0; k < NA; ++k) q[k] = 0.0;
     Place p;
     p.active = local < ns;
     if (p.active) {
@@ -211,7 +207,7 @@ __global__ __launch_bounds__(256) void k_dslash_dots_split(
     auto *red = reinterpret_cast<double *>(dots_smem);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NA; ++k) red[k * 256 + threadIdx.x] = p.active ? double(q[k]) : 0.0;
+    for (int k = 0; k < NA; ++k) red[k * 256 + threadIdx.x] = p.active ? q[k] : 0.0;
     __syncthreads();
     if (int(threadIdx.x) < R) {
         double t[NA];
