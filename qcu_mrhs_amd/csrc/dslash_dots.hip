@@ -346,8 +346,8 @@ hipError_t launch_dslash_lane_dots_groups(const DslashArgs &a, DotsKind kind, co
     switch (a.prec) {
         case kDouble: return launch_groups_s<double>(a, kind, r0, tab, rows, g, partials, stream);
         case kSingle: return launch_groups_s<float>(a, kind, r0, tab, rows, g, partials, stream);
-        case kHalf: return launch_groups_s<__half>(a, kind, r0, tab, rows, g, partials, stream);
-        case kBF16: return launch_groups_s<__hip_bfloat16>(a, kind, r0, tab, rows, g, partials, stream);
+        case kHalf: return launch_groups_s<WideHalf>(a, kind, r0, tab, rows, g, partials, stream);
+        case kBF16: return launch_groups_s<WideBf16>(a, kind, r0, tab, rows, g, partials, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -135,8 +135,9 @@ struct Arith<__hip_bfloat16> {
     }
 };
 
-// FP16 / BF16 storage with everything from the loads on in FP32 (kDslashLaneRhs), at twice the instructions
-// of a product: 31.7 -> 36.9 us at 16^3 x 32, SU(3), 16 RHS in FP16, BF16 even.
+// FP16 / BF16 storage with everything from the loads on in FP32 (kDslashLaneRhs and the batches, whose other
+// kernel does so too), at twice the instructions of a product: 31.7 -> 36.9 us at 16^3 x 32, SU(3), 16 RHS in
+// FP16, BF16 even.
 struct WideHalf {};
 struct WideBf16 {};
 template <typename CS>

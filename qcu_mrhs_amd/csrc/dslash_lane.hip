@@ -478,8 +478,8 @@ hipError_t launch_dslash_lane_groups(const DslashArgs &a, const SegTab &tab, int
     switch (a.prec) {
         case kDouble: return launch_groups_s<double>(a, tab, by, bz, stream);
         case kSingle: return launch_groups_s<float>(a, tab, by, bz, stream);
-        case kHalf: return launch_groups_s<__half>(a, tab, by, bz, stream);
-        case kBF16: return launch_groups_s<__hip_bfloat16>(a, tab, by, bz, stream);
+        case kHalf: return launch_groups_s<WideHalf>(a, tab, by, bz, stream);
+        case kBF16: return launch_groups_s<WideBf16>(a, tab, by, bz, stream);
         default: return hipErrorInvalidValue;
     }
 }
