@@ -324,8 +324,8 @@ def bench_groups(args):
             runs.append((time.perf_counter() - t0, info))
         wall = float(np.mean([r[0] for r in runs]))
         info = runs[-1][1]
-        variant = {2: "VALU wave per site", 3: "FP32 matrix cores", 5: "FP32 matrix cores, packed RHS"}.get(api.lib().qcuGroupsDslashVariant(), "?")
-        variant64 = {2: "VALU wave per site", 3: "FP64 matrix cores", 5: "FP64 matrix cores, packed RHS"}.get(api.lib().qcuGroupsDslashVariant64(), "?")
+        variant = {2: "VALU wave per site", 3: "FP32 matrix cores", 5: "FP32 matrix cores, packed RHS", 6: "lane per (site, RHS)"}.get(api.lib().qcuGroupsDslashVariant(), "?")
+        variant64 = {2: "VALU wave per site", 3: "FP64 matrix cores", 5: "FP64 matrix cores, packed RHS", 6: "lane per (site, RHS)"}.get(api.lib().qcuGroupsDslashVariant64(), "?")
         res = {"batch_s": wall, "rhs_per_s": sum(sizes) / wall, "dslash_kernel": variant,
                "dslash_kernel_fp64": variant64,
                "groups": [{"m_rhs": R, "converged": bool(i["converged"]), "iterations": i["iterations"],

@@ -34,9 +34,11 @@ struct GroupResult {
 
 // groups dslash variant: matrix cores over the groups' RHS packed into shared 16-RHS chunks
 constexpr int kGroupsPacked = 5;
+// and that of the lane-per-(site, RHS) kernel over the batch (Nc <= 4)
+constexpr int kGroupsLane = 6;
 
 // Process-wide override of the groups' dslash kernels (inner hops, FP64 hops): 0 = the timed choice,
-// else 2 (VALU), 3 (matrix cores per group) or 5 (packed); applied after the timing of each batch shape.
+// else 2 (VALU), 3 (matrix cores per group), 5 (packed) or 6 (lane); applied after the timing of each batch shape.
 void groups_force_variants(int inner, int fp64);
 
 class GroupSolver {
@@ -57,10 +59,10 @@ public:
     // Allocates the batch buffers and picks each group's dslash shape (sites
     // per wavefront) by timing it on the inner precision; cached per precision.
     hipError_t autotune(const void *glo, int prec, hipStream_t s);
-    // dslash kernel the autotuner chose for the batch (1 = lane per (site, RHS), 2 = VALU wave-per-site,
-    // 3 = FP32 matrix cores per group, 5 = FP32 matrix cores over the groups' RHS packed into shared chunks)
+    // dslash kernel the autotuner chose for the batch (2 = VALU wave-per-site, 3 = FP32 matrix cores per
+    // group, 5 = FP32 matrix cores over the groups' RHS packed into shared chunks, 6 = lane per (site, RHS))
     int dslash_variant() const { return variant_; }
-    // and for the FP64 hops of the defect correction (1 = lane, 2 = wave, 3 / 5 = FP64 matrix cores; timed in solve)
+    // and for the FP64 hops of the defect correction (2 = wave, 3 / 5 = FP64 matrix cores, 6 = lane; timed in solve)
     int dslash_variant64() const { return variant64_; }
 
     // Solve M x = b for the batch held in b_full(); result in x_full().
@@ -83,8 +85,8 @@ private:
     SegTab tab_;
     int by_ = 0, bz_ = 0;
     int lane_by_[2] = {0, 0}, lane_bz_[2] = {0, 0};  // traversal tiles of the lane kernel: inner precision, FP64
-    // group dslash kernel (autotuned): 1 = lane per (site, RHS), 2 = wave-per-site VALU, 3 = matrix cores per group, 5 = matrix cores
-    // with the groups' RHS packed into shared 16-RHS chunks (sites per wavefront spw_packed_)
+    // group dslash kernel (autotuned): 2 = wave-per-site VALU, 3 = matrix cores per group, 5 = matrix cores
+    // with the groups' RHS packed into shared 16-RHS chunks (sites per wavefront spw_packed_), 6 = lane per (site, RHS)
     int variant_ = 2;
     int spw_packed_ = 1;
     int variant64_ = 2;  // the same for the FP64 hops

@@ -117,7 +117,7 @@ hipError_t GroupSolver::dslash(void *out, const void *in, const void *gauge, int
     DslashArgs a{out, in, gauge, xpay, coef, g_, Nc_, 0, parity, 0, prec};
     const int v = prec == kDouble ? variant64_ : variant_;
     const int hi = prec == kDouble ? 1 : 0;
-    if (v == kDslashLaneRhs) return launch_dslash_lane_groups(a, tab, lane_by_[hi], lane_bz_[hi], s);
+    if (v == kGroupsLane) return launch_dslash_lane_groups(a, tab, lane_by_[hi], lane_bz_[hi], s);
     if (v == kGroupsPacked && dslash_groups_matrix_supported(Nc_, prec))
         return launch_dslash_mfma32_packed(a, tab, by_, bz_, prec == kDouble ? spw_packed64_ : spw_packed_, s);
     if (v == kDslashMfma && dslash_groups_matrix_supported(Nc_, prec))
@@ -148,7 +148,7 @@ hipError_t GroupSolver::tune64(const void *g64, hipStream_t s) {
     int best_spw = 1;
     std::vector<std::pair<int, int>> cands{{kDslashWaveSite, 0}, {kDslashMfma, 0}, {kGroupsPacked, 1},
                                            {kGroupsPacked, 2}, {kGroupsPacked, 4}};
-    if (lane_supported(kDouble)) cands.push_back({kDslashLaneRhs, 0});
+    if (lane_supported(kDouble)) cands.push_back({kGroupsLane, 0});
     for (const auto &c : cands) {
         variant64_ = c.first;
         if (c.second > 0) spw_packed64_ = c.second;
@@ -168,7 +168,8 @@ hipError_t GroupSolver::tune64(const void *g64, hipStream_t s) {
     }
     variant64_ = best_v;
     if (best_spw > 0) spw_packed64_ = best_spw;
-    if (g_force_fp64 == kDslashWaveSite || g_force_fp64 == kDslashMfma || g_force_fp64 == kGroupsPacked)
+    if (g_force_fp64 == kDslashWaveSite || g_force_fp64 == kDslashMfma || g_force_fp64 == kGroupsPacked ||
+        (g_force_fp64 == kGroupsLane && lane_supported(kDouble)))
         variant64_ = g_force_fp64;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -275,7 +276,7 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
         for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = 0;
         err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
         const SegTab t = tab_with(done_);
-        variant_ = kDslashLaneRhs;
+        variant_ = kGroupsLane;
         if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);  // warm-up
         if (err == hipSuccess) err = hipEventRecord(e0, s);
         for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
@@ -286,12 +287,12 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
         if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
         if (err == hipSuccess && ms < best_total) {
             best_total = ms;
-            best_variant = kDslashLaneRhs;
+            best_variant = kGroupsLane;
         }
     }
     variant_ = best_variant;
     spw_packed_ = best_packed;
-    if (g_force_inner == kDslashWaveSite || ((g_force_inner == kDslashMfma || g_force_inner == kGroupsPacked) &&
+    if (g_force_inner == kDslashWaveSite || (g_force_inner == kGroupsLane && lane_supported(prec)) || ((g_force_inner == kDslashMfma || g_force_inner == kGroupsPacked) &&
                                              dslash_groups_matrix_supported(Nc_, prec)))
         variant_ = g_force_inner;
     for (int k = 0; k < tab_.G; ++k) tab_.spw[k] = best_spw_of[k];
@@ -310,7 +311,7 @@ hipError_t GroupSolver::iteration(const void *glo, int P, double kappa, hipStrea
     const double k2 = -kappa * kappa;
     QCU_HIP_TRY(dslash(tmp_, p_, glo, P, 0, nullptr, 1.0, t, s));
     // the lane kernel forms the inner products of a step in its second hop
-    const bool dots = variant_ == kDslashLaneRhs && dotp_;
+    const bool dots = variant_ == kGroupsLane && dotp_;
     const auto hop_dots = [&](DotsKind kind, void *out, const void *x) -> hipError_t {
         DslashArgs a{out, tmp_, glo, x, k2, g_, Nc_, 0, 1, 0, P};
         QCU_HIP_TRY(launch_dslash_lane_dots_groups(a, kind, r0_, t, rows_, dotp_, lane_by_[0], lane_bz_[0], s));

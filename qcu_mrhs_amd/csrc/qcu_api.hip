@@ -884,9 +884,9 @@ int qcuGroupsDslashVariant(void) {
 }
 
 int qcuGroupsDslashTune(int variant, int variant64) {
-    auto ok = [](int v) { return v == 0 || v == kDslashWaveSite || v == kDslashMfma || v == kGroupsPacked; };
+    auto ok = [](int v) { return v == 0 || v == kDslashWaveSite || v == kDslashMfma || v == kGroupsPacked || v == kGroupsLane; };
     if (!ok(variant) || !ok(variant64)) {
-        set_error(kQcuErrorInvalidValue, "qcuGroupsDslashTune: variants are 0, 2, 3 or 5");
+        set_error(kQcuErrorInvalidValue, "qcuGroupsDslashTune: variants are 0, 2, 3, 5 or 6");
         return g_err;
     }
     groups_force_variants(variant, variant64);
