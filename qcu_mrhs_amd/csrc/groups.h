@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "blas.h"
+#include "dslash.h"
 
 namespace qcu {
 
@@ -56,8 +57,8 @@ public:
     void *b_full() const { return b_; }
     void *x_full() const { return x_; }
 
-    // Allocates the batch buffers and picks each group's dslash shape (sites
-    // per wavefront) by timing it on the inner precision; cached per precision.
+    // Allocates the batch buffers and picks each group's dslash shape (sites per wavefront) and the batch's
+    // kernel by timing them on the inner precision; cached per precision.
     hipError_t autotune(const void *glo, int prec, hipStream_t s);
     // dslash kernel the autotuner chose for the batch (2 = VALU wave-per-site, 3 = FP32 matrix cores per
     // group, 5 = FP32 matrix cores over the groups' RHS packed into shared chunks, 6 = lane per (site, RHS))
@@ -74,6 +75,8 @@ private:
     hipError_t dslash(void *out, const void *in, const void *gauge, int prec, int parity, const void *xpay,
                       double coef, const SegTab &tab, hipStream_t s);
     hipError_t iteration(const void *glo, int P, double kappa, hipStream_t s);
+    hipError_t schur_dots(DotsKind kind, void *out, const void *in, const void *glo, int P, double k2, const SegTab &t,
+                          hipStream_t s);
     hipError_t tune64(const void *g64, hipStream_t s);
     SegTab tab_with(const int *done) const;
     bool lane_supported(int prec) const;

@@ -185,85 +185,74 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
     QCU_HIP_TRY(hipEventCreate(&e1));
     // bounded (zero) contents for the timing launches
     QCU_HIP_TRY(launch_scalar_fill(st_, C64{0.0, 0.0}, kNumSlots * tab_.Rtot, s));
-    QCU_HIP_TRY(hipMemsetAsync(p_, 0, size_t(n_) * tab_.Rtot * 2 * prec_bytes(prec), s));
+    for (void *p : {p_, s_, r0_}) QCU_HIP_TRY(hipMemsetAsync(p, 0, size_t(n_) * tab_.Rtot * 2 * prec_bytes(prec), s));
     hipError_t err = hipSuccess;
-    // Kernel variants: the wave-per-site VALU kernel and, for FP32 storage, the FP32 matrix-core
-    // kernel.  Per variant every group is timed alone (the others flagged done) over sites per
-    // wavefront, then the whole batch with those shapes; the variant whose batch launch is
-    // faster serves all groups (one launch covers the batch).
-    std::vector<int> variants{kDslashWaveSite};
-    if (dslash_groups_matrix_supported(Nc_, prec)) variants.push_back(kDslashMfma);
-    double best_total = 1e30;
+    // milliseconds of five launches
+    const auto time = [&](const auto &launch) -> float {
+        if (err == hipSuccess) err = launch();  // warm-up
+        if (err == hipSuccess) err = hipEventRecord(e0, s);
+        for (int rep = 0; rep < 5 && err == hipSuccess; ++rep) err = launch();
+        if (err == hipSuccess) err = hipEventRecord(e1, s);
+        if (err == hipSuccess) err = hipEventSynchronize(e1);
+        float ms = 1e30f;
+        if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
+        return ms;
+    };
+    // the groups of `mask` active, the others flagged done
+    const auto activate = [&](unsigned mask) {
+        for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = (mask >> j & 1) ? 0 : 1;
+        if (err == hipSuccess) err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
+        if (err == hipSuccess) err = hipStreamSynchronize(s);
+    };
+    // Kernel variants: the wave-per-site VALU kernel, for FP32 and FP64 storage the matrix-core kernels, for
+    // Nc <= 4 the lane kernel.  Each is timed by what an iteration runs of it -- the whole batch's Schur
+    // operators with their inner products, which the lane kernel forms in its hops (SU(4), 6 x 10 x 14 x 18,
+    // groups of 3, 8, 17: its bare hops are slower than the packed matrix-core ones, its solve takes 3.9
+    // against 4.2 ms).
+    float best_total = 1e30f;
     int best_variant = kDslashWaveSite, best_packed = 1;
     int best_spw_of[kMaxGroups] = {};
+    const auto time_step = [&]() -> float {
+        const SegTab t = tab_with(done_);
+        return time([&]() -> hipError_t {
+            QCU_HIP_TRY(schur_dots(kDotsAlpha, v_, p_, glo, prec, 0.0, t, s));
+            return schur_dots(kDotsOmega, t_, s_, glo, prec, 0.0, t, s);
+        });
+    };
+    std::vector<int> variants{kDslashWaveSite};
+    if (dslash_groups_matrix_supported(Nc_, prec)) variants.push_back(kDslashMfma);
     for (int v : variants) {
         variant_ = v;
-        double total = 0.0;
-        int spw_of[kMaxGroups] = {};
-        for (int k = 0; k < tab_.G && err == hipSuccess; ++k) {
-            // only group k active
-            for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = (j == k) ? 0 : 1;
-            err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
-            if (err == hipSuccess) err = hipStreamSynchronize(s);
-            double best = 1e30;
+        // every group alone over sites per wavefront, then the batch with those shapes
+        for (int k = 0; k < tab_.G; ++k) {
+            activate(1u << k);
+            float best = 1e30f;
             int best_spw = 1;
             for (int spw : {1, 2, 4, 8, 16}) {
                 SegTab t = tab_with(done_);
                 t.spw[k] = spw;
-                if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);  // warm-up
-                if (err == hipSuccess) err = hipEventRecord(e0, s);
-                for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
-                    err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
-                if (err == hipSuccess) err = hipEventRecord(e1, s);
-                if (err == hipSuccess) err = hipEventSynchronize(e1);
-                float ms = 0.f;
-                if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
+                const float ms = time([&] { return dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s); });
                 if (err == hipSuccess && ms < best) {
                     best = ms;
                     best_spw = spw;
                 }
             }
-            spw_of[k] = best_spw;
-            total += best;
+            tab_.spw[k] = best_spw;
         }
-        // the batch as it runs: every group active, each with its own best shape
-        if (err == hipSuccess && variants.size() > 1) {
-            for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = 0;
-            err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
-            SegTab t = tab_with(done_);
-            for (int k = 0; k < tab_.G; ++k) t.spw[k] = spw_of[k];
-            if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
-            if (err == hipSuccess) err = hipEventRecord(e0, s);
-            for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
-                err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
-            if (err == hipSuccess) err = hipEventRecord(e1, s);
-            if (err == hipSuccess) err = hipEventSynchronize(e1);
-            float ms = 0.f;
-            if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
-            total = ms;
-        }
-        if (err == hipSuccess && total < best_total) {
-            best_total = total;
+        activate(~0u);
+        const float ms = time_step();
+        if (err == hipSuccess && ms < best_total) {
+            best_total = ms;
             best_variant = v;
-            for (int k = 0; k < tab_.G; ++k) best_spw_of[k] = spw_of[k];
+            for (int k = 0; k < tab_.G; ++k) best_spw_of[k] = tab_.spw[k];
         }
     }
-    // the groups' RHS packed into shared 16-RHS chunks: the whole batch over sites per wavefront
-    if (err == hipSuccess && dslash_groups_matrix_supported(Nc_, prec)) {
-        for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = 0;
-        err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
-        const SegTab t = tab_with(done_);
+    // the groups' RHS packed into shared 16-RHS chunks, over sites per wavefront
+    if (dslash_groups_matrix_supported(Nc_, prec)) {
         variant_ = kGroupsPacked;
         for (int spw : {1, 2, 4, 8}) {
             spw_packed_ = spw;
-            if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);  // warm-up
-            if (err == hipSuccess) err = hipEventRecord(e0, s);
-            for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
-                err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
-            if (err == hipSuccess) err = hipEventRecord(e1, s);
-            if (err == hipSuccess) err = hipEventSynchronize(e1);
-            float ms = 0.f;
-            if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
+            const float ms = time_step();
             if (err == hipSuccess && ms < best_total) {
                 best_total = ms;
                 best_variant = kGroupsPacked;
@@ -272,19 +261,9 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
         }
     }
     // a lane per (site, RHS): its launch shape follows from the group sizes
-    if (err == hipSuccess && lane_supported(prec)) {
-        for (int j = 0; j < kMaxGroups; ++j) reinterpret_cast<int *>(h_)[j] = 0;
-        err = hipMemcpyAsync(done_, h_, sizeof(int) * kMaxGroups, hipMemcpyHostToDevice, s);
-        const SegTab t = tab_with(done_);
+    if (lane_supported(prec)) {
         variant_ = kGroupsLane;
-        if (err == hipSuccess) err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);  // warm-up
-        if (err == hipSuccess) err = hipEventRecord(e0, s);
-        for (int rep = 0; rep < 5 && err == hipSuccess; ++rep)
-            err = dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s);
-        if (err == hipSuccess) err = hipEventRecord(e1, s);
-        if (err == hipSuccess) err = hipEventSynchronize(e1);
-        float ms = 0.f;
-        if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
+        const float ms = time_step();
         if (err == hipSuccess && ms < best_total) {
             best_total = ms;
             best_variant = kGroupsLane;
@@ -292,8 +271,8 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
     }
     variant_ = best_variant;
     spw_packed_ = best_packed;
-    if (g_force_inner == kDslashWaveSite || (g_force_inner == kGroupsLane && lane_supported(prec)) || ((g_force_inner == kDslashMfma || g_force_inner == kGroupsPacked) &&
-                                             dslash_groups_matrix_supported(Nc_, prec)))
+    if (g_force_inner == kDslashWaveSite || (g_force_inner == kGroupsLane && lane_supported(prec)) ||
+        ((g_force_inner == kDslashMfma || g_force_inner == kGroupsPacked) && dslash_groups_matrix_supported(Nc_, prec)))
         variant_ = g_force_inner;
     for (int k = 0; k < tab_.G; ++k) tab_.spw[k] = best_spw_of[k];
     (void)hipEventDestroy(e0);
@@ -305,32 +284,27 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
     return err;
 }
 
+// out = A in and alpha or omega (in = s) in st_; the lane kernel forms the inner products in its second hop
+hipError_t GroupSolver::schur_dots(DotsKind kind, void *out, const void *in, const void *glo, int P, double k2,
+                                   const SegTab &t, hipStream_t s) {
+    QCU_HIP_TRY(dslash(tmp_, in, glo, P, 0, nullptr, 1.0, t, s));
+    if (variant_ == kGroupsLane && dotp_) {
+        DslashArgs a{out, tmp_, glo, in, k2, g_, Nc_, 0, 1, 0, P};
+        QCU_HIP_TRY(launch_dslash_lane_dots_groups(a, kind, r0_, t, rows_, dotp_, lane_by_[0], lane_bz_[0], s));
+        return kind == kDotsAlpha ? seg_finish_alpha(st_, t, rows_, dotp_, s) : seg_finish_omega(st_, t, rows_, dotp_, s);
+    }
+    QCU_HIP_TRY(dslash(out, tmp_, glo, P, 1, in, k2, t, s));
+    return kind == kDotsAlpha ? seg_step_alpha(st_, r0_, out, P, t, work_, s)
+                              : seg_step_omega(st_, out, in, P, t, work_, s);
+}
+
 // one BiCGStab iteration of every active group (graph-captured)
 hipError_t GroupSolver::iteration(const void *glo, int P, double kappa, hipStream_t s) {
     const SegTab t = tab_with(done_);
     const double k2 = -kappa * kappa;
-    QCU_HIP_TRY(dslash(tmp_, p_, glo, P, 0, nullptr, 1.0, t, s));
-    // the lane kernel forms the inner products of a step in its second hop
-    const bool dots = variant_ == kGroupsLane && dotp_;
-    const auto hop_dots = [&](DotsKind kind, void *out, const void *x) -> hipError_t {
-        DslashArgs a{out, tmp_, glo, x, k2, g_, Nc_, 0, 1, 0, P};
-        QCU_HIP_TRY(launch_dslash_lane_dots_groups(a, kind, r0_, t, rows_, dotp_, lane_by_[0], lane_bz_[0], s));
-        return kind == kDotsAlpha ? seg_finish_alpha(st_, t, rows_, dotp_, s) : seg_finish_omega(st_, t, rows_, dotp_, s);
-    };
-    if (dots) {
-        QCU_HIP_TRY(hop_dots(kDotsAlpha, v_, p_));
-    } else {
-        QCU_HIP_TRY(dslash(v_, tmp_, glo, P, 1, p_, k2, t, s));
-        QCU_HIP_TRY(seg_step_alpha(st_, r0_, v_, P, t, work_, s));
-    }
+    QCU_HIP_TRY(schur_dots(kDotsAlpha, v_, p_, glo, P, k2, t, s));
     QCU_HIP_TRY(seg_step_s(s_, r_, v_, st_, P, t, s));
-    QCU_HIP_TRY(dslash(tmp_, s_, glo, P, 0, nullptr, 1.0, t, s));
-    if (dots) {
-        QCU_HIP_TRY(hop_dots(kDotsOmega, t_, s_));
-    } else {
-        QCU_HIP_TRY(dslash(t_, tmp_, glo, P, 1, s_, k2, t, s));
-        QCU_HIP_TRY(seg_step_omega(st_, t_, s_, P, t, work_, s));
-    }
+    QCU_HIP_TRY(schur_dots(kDotsOmega, t_, s_, glo, P, k2, t, s));
     QCU_HIP_TRY(seg_step_xr(xl_, r_, p_, s_, t_, r0_, st_, done_, iters_, P, t, work_, s));
     QCU_HIP_TRY(seg_step_p(p_, r_, v_, st_, P, t, s));
     return hipSuccess;

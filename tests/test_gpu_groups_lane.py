@@ -64,3 +64,10 @@ def test_other_shapes_keep_the_timed_choice():
     api.check(api.lib().qcuGroupsDslashTune(LANE, LANE))
     inner, fp64 = _solve((4, 4, 4, 4), 8, (3, 5), 1, 1960)
     assert inner in (2, 3, 5) and fp64 in (2, 3, 5)
+
+
+def test_choice_is_by_what_an_iteration_runs():
+    """The lane kernel's bare hop is slower here than the packed matrix-core
+    one, its iteration, which needs no separate inner products, faster by a
+    tenth: the batch takes it."""
+    assert _solve((6, 10, 14, 18), 4, (3, 8, 17), 1, 1970)[0] == LANE
