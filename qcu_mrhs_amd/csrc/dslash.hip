@@ -239,6 +239,42 @@ bool fits_mfma16(const DslashArgs &a) {
     return double(a.g.Vh) * 16.0 * a.Nc * a.R < 2147483647.0 && double(a.g.Vh) * 32.0 * a.Nc * a.Nc < 2147483647.0;
 }
 
+// 16 bits: a lane per (site, RHS) instead of the matrix cores (lane / matrix cores below, us, FP16).
+// A row of right-hand sides has to be a whole number of 16-byte pieces, or to need a second chunk of the
+// matrix cores' 16 columns; otherwise the lanes' loads straddle those pieces (24^3 x 48, SU(3) 190 / 175 at 6,
+// 220 / 191 at 10).
+bool row_fits_lanes(int R) { return R % 4 == 0 || R > 16; }
+
+bool lane16_faster(const DslashArgs &a) {
+    if (!fits_mfma16(a)) return false;
+    const long sites = a.g.Vh, lanes = sites * a.R;
+    const bool split = dslash_lane_split(a.g, a.R);
+    // Up to 3 right-hand sides leave 13 of the matrix cores' 16 columns empty.  From 8192 sites (8^3 x 16 with
+    // 4096: even) a lane per site is faster where the lattice takes a wavefront per direction (16^3 x 32,
+    // SU(3): 13 / 45 at 1, 21 / 46 at 2; beyond it 24^4, SU(3): 118 / 89 at 1; SU(4) 16^4: 13 / 25 at 1, but
+    // 21 / 25 at 3, where solves on SU(4) lose 5 %) and beyond it where the rows of a site still share lines
+    // (SU(2): 24^3 x 48 80 / 127 at 1, 84 / 128 at 3; SU(3) at 3: 24^4 82 / 88, 24^3 x 48 145 / 205)
+    if (a.R <= 3)
+        return sites >= 8192 && (a.Nc == 2 || (a.Nc == 3 && (split || a.R == 3)) || (a.Nc == 4 && split && a.R == 1));
+    if (!row_fits_lanes(a.R)) return false;
+    // clover blocks are applied in the lane kernel's epilogue only
+    if (a.clover) return true;
+    // A site's arithmetic takes the matrix cores fewer cycles, the lane kernel moves fewer bytes (24^3 x 48, SU(3):
+    // 100 / 181 at 8, 209 / 242 at 16, 361 / 761 at 32).  SU(2): lanes but in the smallest ragged launches
+    // (at 17: 8^3 x 16 5.8 / 5.4, 12^4 9.1 / 10.5)
+    if (a.Nc == 2) return a.R % 4 == 0 || lanes > 98304;
+    // SU(3) beyond 8 and two chunks: more than three wavefronts per SIMD (SU(3) 12^4 8.8 / 8.1 at 16, 10.5 / 13.3
+    // at 20, 16^4 18.1 / 19.0 at 16, 8^4 6.3 / 5.5 at 48; SU(4) 8^3 x 16 13.4 / 12.4 at 48, 13.6 / 15.8 at 64,
+    // 12^4 18.7 / 16.4 at 17)
+    if (a.R > 16 || (a.Nc == 3 && a.R > 8)) return lanes > 196608;
+    if (a.Nc == 3) return true;
+    // SU(4), one chunk: up to 8 a wavefront per direction (12^4 6.4 / 9.4 at 4) or four wavefronts per SIMD
+    // (at 8: 12^4 11.6 / 9.6, 16^4 20.6 / 22.6); 12 and 16 once the fields exceed the 256 MiB memory-side cache
+    // (at 16: 12^4 13.8 / 9.5, 16^3 x 32 48 / 43, 24^4 120 / 165)
+    if (a.R <= 8) return split || lanes >= 262144;
+    return double(sites) * (8.0 * a.Nc * a.Nc + 8.0 * a.Nc * a.R) * 4.0 > 268435456.0;
+}
+
 // Kernel chosen for a hop that names none.
 int automatic_variant(const DslashArgs &a) {
     const bool lane = dslash_lane_supported(a.g, a.Nc, a.R, a.prec);
@@ -251,21 +287,7 @@ int automatic_variant(const DslashArgs &a) {
         if (a.Nc == 8) return kDslashMfma;
         return lane ? kDslashLaneRhs : kDslashWaveSite;
     }
-    // 16 bits: a lane per (site, RHS) where a row of right-hand sides is a whole number of 16-byte
-    // pieces (24^3 x 48, SU(3) FP16: 103 against 179 us matrix cores at 8 RHS, 188 / 207 at 12,
-    // 213 / 245 at 16, 374 / 759 at 32) or needs a second 16-wide matrix-core chunk (370 / 536 at 17);
-    // otherwise its loads straddle those pieces (190 / 175 at 6, 220 / 191 at 10)
-    const bool fits16 = fits_mfma16(a);
-    if (lane && fits16 && (a.R % 4 == 0 || a.R > 16)) return kDslashLane16;
-    // Up to 3 right-hand sides leave 13 of the matrix cores' 16 columns empty.  From 8192 sites (8^3 x 16 with
-    // 4096: even) a lane per site is faster where the lattice takes a wavefront per direction (FP16 16^3 x 32,
-    // SU(3): 13 against 45 us at 1, 21 / 46 at 2; beyond it 24^4, SU(3): 118 / 89 at 1; SU(4) 16^4: 13 / 25 at 1,
-    // but 21 / 25 at 3, which a solve does not see) and beyond it where the rows of a site still share lines
-    // (SU(2): 24^3 x 48 80 / 127 at 1, 84 / 128 at 3; SU(3) at 3: 24^4 82 / 88, 24^3 x 48 145 / 205)
-    const bool split = dslash_lane_split(a.g, a.R);
-    if (lane && fits16 && a.R <= 3 && a.g.Vh >= 8192 &&
-        (a.Nc == 2 || (a.Nc == 3 && (split || a.R == 3)) || (a.Nc == 4 && split && a.R == 1)))
-        return kDslashLane16;
+    if (lane && lane16_faster(a)) return kDslashLane16;
     return dslash_mfma_supported(a.Nc, a.prec) ? kDslashMfma : kDslashWaveSite;
 }
 }  // namespace
@@ -376,6 +398,16 @@ hipError_t launch_dslash_clover(const DslashArgs &a, hipStream_t stream) {
                                a.prec == kDouble ? kDouble : kSingle, stream);
 }
 
+namespace {
+// no kernel is named for these arguments: by themselves, for the process or in the tuning table
+bool automatic(const DslashArgs &a) {
+    if (a.tune.variant != kDslashAuto) return false;
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    return g_override.variant == kDslashAuto &&
+           !g_tuned.count(std::make_tuple(a.g.L[0], a.g.L[1], a.g.L[2], a.g.L[3], a.Nc, a.R, a.prec));
+}
+}  // namespace
+
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
 long dslash_dots_partials(const Geom &g, int Nc, int R, int prec) {
@@ -392,7 +424,14 @@ hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0
     if (!dslash_supported(a.Nc, a.R) || a.g.Vh <= 0 || a.dagger || a.keep_order || !partials || !st ||
         !(a.clover ? a.clover_in : a.xpay) || (kind == kDotsAlpha && !r0) || a.R > kReduceThreads)
         return hipErrorNotSupported;
-    const DslashTune t = dslash_resolve(a);
+    DslashTune t = dslash_resolve(a);
+    // alpha's products in the lane kernel's epilogue save a pass over two vectors, more than its hop is behind
+    // that of the matrix cores where lane16_faster prefers those (SU(3) 12^4, 12 RHS: 0.7 us, the pass 6 us)
+    if (kind == kDotsAlpha && t.variant == kDslashMfma && row_fits_lanes(a.R) && automatic(a)) {
+        t = DslashTune{};
+        t.variant = kDslashLane16;
+        t = dslash_fill_defaults(a, t);
+    }
     const bool lane = dslash_lane_forms(a, t);
     const bool mfma = t.variant == kDslashMfma && (a.prec == kHalf || a.prec == kBF16) && kind == kDotsOmega && !a.clover;
     if ((!lane && !mfma) || (a.clover && !dslash_lane_clover_fused(a, t))) return hipErrorNotSupported;
