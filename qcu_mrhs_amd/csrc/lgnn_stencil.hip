@@ -307,8 +307,11 @@ template <typename CS, int NC>
 hipError_t mix_nc(void *q, const void *in, const void *gauge, const C32 *mcol, const int *walk, const Geom &g, int R,
                   hipStream_t s) {
     const int rc = chunk_rhs(NC, R), nt = div_up(NC * rc, 16);
-    // several sites per workgroup share the fragments of M; at least two workgroups per compute unit and chunk
-    const int sites = std::max(1, std::min(16, g.Vh / (8 * num_cus())));
+    // Several sites per workgroup share the fragments of M and overlap a site's loads with the last one's
+    // products: up to 16 where eight workgroups per compute unit and chunk are left, up to 4 where two are (8^4,
+    // SU(3), whole application with 1 site 87 us at 32 RHS and 61 at 16, with 4 sites 65 and 50; 8^3 x 16, 32 RHS
+    // with 2 sites 109, with 4 97 us; 4^4, 64 RHS, which gets 1, 38.5 against 41 us with 4)
+    const int sites = std::max({1, std::min(4, g.Vh / (2 * num_cus())), std::min(16, g.Vh / (8 * num_cus()))});
     const dim3 grid(div_up(g.Vh, sites), div_up(R, rc));
     // items per thread: one for 8 right-hand sides per chunk
     auto k = nt == 1 ? mix_kernel<CS, NC, 1>(rc) : nt == 2 ? mix_kernel<CS, NC, 2>(rc)
