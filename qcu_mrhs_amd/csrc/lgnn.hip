@@ -439,11 +439,17 @@ hipError_t LgnnPreconditioner::collapse(hipStream_t s) {
     return hipGetLastError();
 }
 
-// the lane hopping kernel's tile (16 bits, 24^3 x 48, 16 RHS: mix 484 -> 471 us, gather 343 -> 334 us against
-// the untiled order)
+// The lane hopping kernel's tile where a field is larger than half of the eight XCDs' 4 MB L2s (16 bits,
+// 24^3 x 48, 16 RHS: mix 484 -> 471 us, gather 343 -> 334 us against the untiled order; whole application SU(3)
+// 16^4 97.8 -> 93.1 us with fields of 18 MiB); smaller ones are read again from there in either order, and the
+// untiled one keeps more of the lattice's planes in one piece (SU(2) 16^4, 16 MiB 72.9 against 76.2 us, SU(3)
+// 12^4, 15 MiB 86.2 against 88.5 us).
 hipError_t LgnnPreconditioner::tables(GeomTables &tab, int prec, hipStream_t s) const {
-    int by = 0, bz = 0;
-    dslash_lane_tile(g_, Nc_, R_, prec, by, bz);
+    int by = g_.L[1], bz = g_.L[2];
+    if (double(n_) * R_ * 2 * double(prec_bytes(prec)) > 16777216.0) {
+        by = bz = 0;
+        dslash_lane_tile(g_, Nc_, R_, prec, by, bz);
+    }
     return geom_tables(g_, by, bz, tab, s);
 }
 
