@@ -134,9 +134,10 @@ hipError_t launch_rows_sum(double *out, const double *in, int nrows, int cols, i
 // x = a.clover_in), dagger 0, with the inner products of a BiCGStab step in its epilogue, finished into st:
 // kDotsAlpha: out = v, alpha = rho / <r0, v> like launch_step_alpha; kDotsOmega: out = t, x = s,
 // omega = <t, s> / <t, t> like launch_step_omega (r0 not read).
-// `partials` holds dslash_dots_partials(g, Nc, R, prec) doubles.  Returns hipErrorNotSupported (and
-// launches nothing) when the launch chosen for these arguments has no such form (the lane kernel has both,
-// the 16-bit matrix-core kernel omega's without clover blocks); the caller then runs the separate reduction.
+// `partials` holds dslash_dots_partials(g, Nc, R, prec) doubles (0, and null, where no kernel has the form).
+// Returns hipErrorNotSupported (and launches nothing) when the launch chosen for these arguments has no such
+// form (the lane kernel has both, the 16-bit matrix-core kernel omega's without clover blocks); the caller then
+// runs the separate reduction.
 // Rows that the finisher's one workgroup per RHS sums by itself: four per lane (20736 rows, 16 RHS: 72 us,
 // against 12 us through slices)
 constexpr int kMaxFinishRows = 4096;

@@ -411,12 +411,16 @@ bool automatic(const DslashArgs &a) {
 constexpr int kDotSlices = 512;  // first-level slices of the per-workgroup partials
 
 long dslash_dots_partials(const Geom &g, int Nc, int R, int prec) {
-    // one row of R x 4 per workgroup: the lane kernel's, or a wavefront's worth of sites (a wavefront per
-    // direction); matrix cores: at most one per 4 sites, or 64 per CU for the persistent grid
-    long nblk = Nc <= 4 ? dslash_lane_blocks(g, Nc, R, prec) : 0;
-    if (R <= 64) nblk = std::max<long>(nblk, div_up(g.Vh, 64 / R));
-    if (prec == kHalf || prec == kBF16) nblk = std::max<long>({nblk, long(div_up(g.Vh, 4)), 64L * num_cus()});
-    return (nblk + kDotSlices) * R * 4;
+    // one row of R x 4 per workgroup of the forms that exist for these arguments: the lane kernel's, or a
+    // wavefront's worth of sites (a wavefront per direction); matrix cores: at most one per 4 sites, or 64 per
+    // CU for the persistent grid
+    long nblk = 0;
+    if (dslash_lane_supported(g, Nc, R, prec)) {
+        nblk = dslash_lane_blocks(g, Nc, R, prec);
+        if (dslash_lane_split(g, R)) nblk = std::max<long>(nblk, div_up(g.Vh, 64 / R));
+    }
+    if (dslash_mfma_supported(Nc, prec)) nblk = std::max<long>({nblk, long(div_up(g.Vh, 4)), 64L * num_cus()});
+    return nblk ? (nblk + kDotSlices) * R * 4 : 0;
 }
 
 hipError_t launch_dslash_dots(const DslashArgs &a, DotsKind kind, const void *r0, double *partials, long cap,
