@@ -59,6 +59,7 @@ _SYMBOLS = {
                          [_G, _i, _i, _T, _W]),
     "launch_dslash_dots": ("_ZN3qcu18launch_dslash_dotsERKNS_10DslashArgsENS_8DotsKindEPKvPdlPNS_2CxIdEEP12ihipStream_t",
                            _i, [_A, _i, _vp, _vp, _l, _vp, _vp]),
+    "launch_dslash_clover": ("_ZN3qcu20launch_dslash_cloverERKNS_10DslashArgsEP12ihipStream_t", _i, [_A, _vp]),
     "launch_dslash_lane_dots_groups": ("_ZN3qcu30launch_dslash_lane_dots_groupsERKNS_10DslashArgsENS_8DotsKindEPKvRKNS_6SegTab"
                                        "ERKNS_7SegRowsEPdiiP12ihipStream_t", _i, [_A, _i, _vp, _T, _W, _vp, _i, _i, _vp]),
     "launch_dslash_lane_groups": ("_ZN3qcu25launch_dslash_lane_groupsERKNS_10DslashArgsERKNS_6SegTabEiiP12ihipStream_t", _i,
