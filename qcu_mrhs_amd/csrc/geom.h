@@ -1,6 +1,6 @@
 // geom.h -- device index tables of a lattice: traversal order and the eight
-// neighbour indices of every checkerboard site.  Built once per lattice (and
-// per traversal tile) on the device and cached for the life of the process.
+// neighbour indices of every checkerboard site.  Built once per GPU, lattice (and
+// traversal tile) on the current device and cached for the life of the process.
 // They cost 4 + 32 bytes per site per dslash (about 2% of the compulsory
 // spinor + link traffic of a 16-RHS FP16 dslash) and remove every integer
 // division and wrap test from the hopping kernels.

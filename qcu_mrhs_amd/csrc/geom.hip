@@ -41,39 +41,42 @@ __global__ void k_build_walk(int *walk, const int *order, const int *nbr, int Vh
     for (int k = 0; k < 8; ++k) row[1 + k] = nbr[(long(parity) * Vh + site) * 8 + k];
 }
 
-using Key4 = std::tuple<int, int, int, int>;
-using Key6 = std::tuple<int, int, int, int, int, int>;
+// the tables lie in one GPU's memory: device, lattice (, tile)
+using KeyNbr = std::tuple<int, int, int, int, int>;
+using KeyOrder = std::tuple<int, int, int, int, int, int, int>;
 std::mutex g_mu;
-std::map<Key4, int *> g_nbr;
-std::map<Key6, int *> g_order;
-std::map<Key6, int *> g_walk;
+std::map<KeyNbr, int *> g_nbr;
+std::map<KeyOrder, int *> g_order;
+std::map<KeyOrder, int *> g_walk;
 
 }  // namespace
 
 hipError_t geom_tables(const Geom &g, int by, int bz, GeomTables &out, hipStream_t stream) {
+    int dev = 0;
+    QCU_HIP_TRY(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_mu);
     bool built = false;
-    const Key4 k4{g.L[0], g.L[1], g.L[2], g.L[3]};
-    auto it = g_nbr.find(k4);
+    const KeyNbr kn{dev, g.L[0], g.L[1], g.L[2], g.L[3]};
+    auto it = g_nbr.find(kn);
     if (it == g_nbr.end()) {
         built = true;
         int *p = nullptr;
         QCU_HIP_TRY(hipMalloc(&p, sizeof(int) * 16 * size_t(g.Vh)));
         hipLaunchKernelGGL(k_build_nbr, dim3(div_up(2L * g.Vh, 256)), dim3(256), 0, stream, p, g);
         QCU_HIP_TRY(hipGetLastError());
-        it = g_nbr.emplace(k4, p).first;
+        it = g_nbr.emplace(kn, p).first;
     }
-    const Key6 k6{g.L[0], g.L[1], g.L[2], g.L[3], by, bz};
-    auto jt = g_order.find(k6);
+    const KeyOrder ko{dev, g.L[0], g.L[1], g.L[2], g.L[3], by, bz};
+    auto jt = g_order.find(ko);
     if (jt == g_order.end()) {
         built = true;
         int *p = nullptr;
         QCU_HIP_TRY(hipMalloc(&p, sizeof(int) * size_t(g.Vh)));
         hipLaunchKernelGGL(k_build_order, dim3(div_up(g.Vh, 256)), dim3(256), 0, stream, p, g, by, bz);
         QCU_HIP_TRY(hipGetLastError());
-        jt = g_order.emplace(k6, p).first;
+        jt = g_order.emplace(ko, p).first;
     }
-    auto wt = g_walk.find(k6);
+    auto wt = g_walk.find(ko);
     if (wt == g_walk.end()) {
         built = true;
         int *p = nullptr;
@@ -81,7 +84,7 @@ hipError_t geom_tables(const Geom &g, int by, int bz, GeomTables &out, hipStream
         hipLaunchKernelGGL(k_build_walk, dim3(div_up(2L * g.Vh, 256)), dim3(256), 0, stream, p, jt->second,
                            it->second, g.Vh);
         QCU_HIP_TRY(hipGetLastError());
-        wt = g_walk.emplace(k6, p).first;
+        wt = g_walk.emplace(ko, p).first;
     }
     out.nbr = it->second;
     out.order = jt->second;
