@@ -187,11 +187,11 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
     QCU_HIP_TRY(launch_scalar_fill(st_, C64{0.0, 0.0}, kNumSlots * tab_.Rtot, s));
     for (void *p : {p_, s_, r0_}) QCU_HIP_TRY(hipMemsetAsync(p, 0, size_t(n_) * tab_.Rtot * 2 * prec_bytes(prec), s));
     hipError_t err = hipSuccess;
-    // milliseconds of five launches
-    const auto time = [&](const auto &launch) -> float {
+    // milliseconds of `reps` launches
+    const auto time = [&](int reps, const auto &launch) -> float {
         if (err == hipSuccess) err = launch();  // warm-up
         if (err == hipSuccess) err = hipEventRecord(e0, s);
-        for (int rep = 0; rep < 5 && err == hipSuccess; ++rep) err = launch();
+        for (int rep = 0; rep < reps && err == hipSuccess; ++rep) err = launch();
         if (err == hipSuccess) err = hipEventRecord(e1, s);
         if (err == hipSuccess) err = hipEventSynchronize(e1);
         float ms = 1e30f;
@@ -214,7 +214,7 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
     int best_spw_of[kMaxGroups] = {};
     const auto time_step = [&]() -> float {
         const SegTab t = tab_with(done_);
-        return time([&]() -> hipError_t {
+        return time(2, [&]() -> hipError_t {
             QCU_HIP_TRY(schur_dots(kDotsAlpha, v_, p_, glo, prec, 0.0, t, s));
             return schur_dots(kDotsOmega, t_, s_, glo, prec, 0.0, t, s);
         });
@@ -231,7 +231,7 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
             for (int spw : {1, 2, 4, 8, 16}) {
                 SegTab t = tab_with(done_);
                 t.spw[k] = spw;
-                const float ms = time([&] { return dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s); });
+                const float ms = time(5, [&] { return dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s); });
                 if (err == hipSuccess && ms < best) {
                     best = ms;
                     best_spw = spw;
@@ -247,17 +247,24 @@ hipError_t GroupSolver::autotune(const void *glo, int prec, hipStream_t s) {
             for (int k = 0; k < tab_.G; ++k) best_spw_of[k] = tab_.spw[k];
         }
     }
-    // the groups' RHS packed into shared 16-RHS chunks, over sites per wavefront
+    // the groups' RHS packed into shared 16-RHS chunks: the batch's hop over sites per wavefront
     if (dslash_groups_matrix_supported(Nc_, prec)) {
         variant_ = kGroupsPacked;
+        float best = 1e30f;
         for (int spw : {1, 2, 4, 8}) {
             spw_packed_ = spw;
-            const float ms = time_step();
-            if (err == hipSuccess && ms < best_total) {
-                best_total = ms;
-                best_variant = kGroupsPacked;
+            const SegTab t = tab_with(done_);
+            const float ms = time(5, [&] { return dslash(tmp_, p_, glo, prec, 0, nullptr, 1.0, t, s); });
+            if (err == hipSuccess && ms < best) {
+                best = ms;
                 best_packed = spw;
             }
+        }
+        spw_packed_ = best_packed;
+        const float ms = time_step();
+        if (err == hipSuccess && ms < best_total) {
+            best_total = ms;
+            best_variant = kGroupsPacked;
         }
     }
     // a lane per (site, RHS): its launch shape follows from the group sizes
