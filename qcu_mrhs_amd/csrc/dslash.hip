@@ -241,8 +241,8 @@ bool fits_mfma16(const DslashArgs &a) {
 
 // 16 bits: a lane per (site, RHS) instead of the matrix cores (lane / matrix cores below, us, FP16).
 // A row of right-hand sides has to be a whole number of 16-byte pieces, or to need a second chunk of the
-// matrix cores' 16 columns; otherwise the lanes' loads straddle those pieces (24^3 x 48, SU(3) 190 / 175 at 6,
-// 220 / 191 at 10).
+// matrix cores' 16 columns; otherwise the lanes' loads straddle those pieces (at 5 to 15 on lattices from 12^4 to
+// 24^3 x 48 SU(3) 1.05 to 1.6 times, SU(4) 1.1 to 2.1 times the matrix cores' time, SU(2) 0.8 to 1.5 times).
 bool row_fits_lanes(int R) { return R % 4 == 0 || R > 16; }
 
 bool lane16_faster(const DslashArgs &a) {
